@@ -28,6 +28,10 @@ int pow2_io(const FftParams &P, int map, unsigned grid, unsigned block, size_t l
 long long pow2_rowpair_grid(long long signals, long long L2, int TB);
 hipError_t launch_fft_pow2(const FftParams &P, int map, unsigned grid, unsigned block, size_t lds, hipStream_t s);
 
+// fft_mix.hip
+int mix_wpe(unsigned grid, unsigned block);   // waves per SIMD of the instance a launch takes
+hipError_t launch_fft_mix(const FftParams &P, unsigned grid, unsigned block, size_t lds, hipStream_t s);
+
 // status codes (mirror impulse_fft_status)
 enum Status { OK = 0, E_INVALID = 1, E_NOMEM = 2, E_HIP = 3, E_UNSUPPORTED = 4, E_NODEVICE = 5 };
 
@@ -73,7 +77,7 @@ struct HostStage {
 enum BufRef : int { REF_IN = 0, REF_OUT = 1, REF_S0 = 2, REF_S1 = 3, REF_TMP = 4, REF_NONE = 5 };
 
 struct Pass {
-    enum Kind { FFT_LDS, FFT_POW2, REAL_POST } kind;
+    enum Kind { FFT_LDS, FFT_POW2, FFT_MIX, REAL_POST } kind;
     int map = 0;                          // FFT_POW2 lane mapping (0 row, 1 col, 2 row load / col store)
     FftParams fp{};
     RealPostParams rp{};
@@ -88,6 +92,8 @@ struct Pass {
     // source pointer is 16-byte aligned at execute time)
     bool has_alt = false;
     FftParams fp_alt{};
+    // FFT_MIX: the half-length real side moves as complex words when its pointer is aligned to them
+    bool in_words = false, out_words = false;
 };
 
 struct R2r;   // DCT / DST plan data (dct.hip)
@@ -182,6 +188,10 @@ int mfma_create(Mfma **out, size_t length, size_t batch, int precision, Error &e
 int mfma_execute(Mfma &m, const void *in, void *out, int forward, double fct, hipStream_t s, Error &err);
 size_t mfma_workspace_bytes(const Mfma &m);
 void mfma_destroy(Mfma *m);
+
+// mixed-radix shapes (twiddle.hip)
+bool mix_factor(int N, int max_threads, std::vector<int> &radices, int &threads);
+void mix_table(std::vector<double2> &out, const std::vector<int> &radices, int sign);
 
 // host FP64 twiddles (twiddle.hip)
 void twiddle_table(std::vector<double2> &out, uint64_t n, uint64_t count, uint64_t step);

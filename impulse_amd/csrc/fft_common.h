@@ -177,6 +177,17 @@ __device__ __forceinline__ void bstore2(__amdgpu_buffer_rsrc_t r, int off, doubl
                                            r, off, 0, 0);
 }
 
+__device__ __forceinline__ void bstore1(__amdgpu_buffer_rsrc_t r, int off, double v)
+{
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned int, v), r,
+                                          off, 0, 0);
+}
+
+__device__ __forceinline__ void bstoref1(__amdgpu_buffer_rsrc_t r, int off, double v)
+{
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, (float)v), r, off, 0, 0);
+}
+
 // v rounded to complex float
 __device__ __forceinline__ void bstoref2(__amdgpu_buffer_rsrc_t r, int off, double2 v)
 {

@@ -28,6 +28,8 @@ constexpr int kMaxBatchDims = 8;
 constexpr int kMaxTB = 64;          // transforms per workgroup
 constexpr int kMaxLdsLen = 8192;    // longest single-pass FP64 transform (128 KiB of LDS)
 constexpr int kMaxThreads = 512;       // workgroup size cap (256 VGPRs per lane available)
+constexpr int kMixMinLen = 17;         // shortest length of the mixed-radix kernel
+constexpr int kMixMaxThreads = 512;    // workgroup size cap of the mixed-radix kernel
 
 enum LoadMode : int {
     LD_C2C = 0,       // z = x[pos]                                  (complex input)
@@ -73,6 +75,7 @@ struct FftParams {
     int N;                     // transform length in LDS (points)
     int nst;                   // number of Stockham stages
     int radix[kMaxStages];
+    unsigned codes;            // mixed-radix kernel: radix - 1 of stage k in bits 4k .. 4k + 3
     int NT;                    // threads per transform
     int TB;                    // transforms per workgroup
     int LD;                    // LDS words (double2) per transform
@@ -90,6 +93,8 @@ struct FftParams {
     int M;                     // half length (real-half modes) or odd length (pair modes)
     int src32, dst32;          // the source / destination array holds float (complex: float2)
                                // rather than double; arithmetic stays FP64 (workspaces are FP64)
+    int in_words, out_words;   // mixed-radix kernel, half-length real sides: x[2p], x[2p+1] move as one
+                               // complex word (unit stride, even batch strides, aligned pointer)
     int nload;                 // local points loaded per transform (the rest of the row is zero)
     int nstore;                // points stored per transform
     double fct;

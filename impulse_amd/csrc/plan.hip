@@ -17,6 +17,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 
 #include "butterflies.h"
 #include "engine.h"
@@ -219,6 +220,7 @@ struct Job {
 struct Builder {
     Plan &plan;
     Error &err;
+    std::map<std::pair<int, int>, const double2 *> mix_tw;   // stage tables by length and sign
 
     std::shared_ptr<DevBuf> upload(const std::vector<double2> &v)
     {
@@ -385,9 +387,7 @@ struct Builder {
     static void make_alt(Pass &ps)
     {
         const FftParams &P = ps.fp;
-        if (P.load_mode != LD_REAL_HALF || P.in.sax != 1 || P.in.kind != SIDE_DIMS || P.in.isig % 2) return;
-        for (int d = 0; d < P.in.nbd; ++d)
-            if (P.in.str[d] % 2) return;
+        if (P.load_mode != LD_REAL_HALF || !even_side(P.in)) return;
         ps.fp_alt = P;
         ps.fp_alt.load_mode = LD_C2C;
         for (int d = 0; d < P.in.nbd; ++d) ps.fp_alt.in.str[d] /= 2;
@@ -395,12 +395,122 @@ struct Builder {
         ps.has_alt = true;
     }
 
+    // bytes of the array behind `r` that a pass may address (the workspace of a linear side: its
+    // own extent, whatever the final allocation)
+    long long ref_bytes(BufRef r, const Side &S, const FftParams &P) const
+    {
+        if (r == REF_IN) return (long long)(plan.in_hi - plan.in_lo);
+        if (r == REF_OUT) return (long long)(plan.out_hi - plan.out_lo);
+        if (r == REF_TMP) return (long long)plan.tmp_bytes;
+        return S.kind == SIDE_LINEAR ? (P.ntf / std::max<long long>(1, P.ni)) * S.lin * 16 : LLONG_MAX;
+    }
+
+    // The mixed-radix kernel: plain c2c, four-step twiddled stores and single-pass real transforms
+    // of lengths that split into radices 2..16, all offsets within 31 bits.  1: added, 0: not for
+    // this kernel, -1: error.
+    int try_mix(FftParams P, BufRef src, BufRef dst, bool uses_fct, bool colL, bool colS)
+    {
+        const bool modes = (P.load_mode == LD_C2C && (P.store_mode == ST_C2C || P.store_mode == ST_TWIDDLE)) ||
+                           (P.load_mode == LD_REAL_HALF && P.store_mode == ST_R2C_HALF) ||
+                           (P.load_mode == LD_R2C_PAIR && P.store_mode == ST_R2C_PAIR) ||
+                           (P.load_mode == LD_C2R_HALF && P.store_mode == ST_C2R_HALF) ||
+                           (P.load_mode == LD_C2R_PAIR && P.store_mode == ST_C2R_PAIR);
+        const bool half = P.load_mode == LD_REAL_HALF || P.load_mode == LD_C2R_HALF;
+        const bool real = P.load_mode != LD_C2C;
+        if (!modes || P.N < kMixMinLen || P.conv || P.chirp_in || P.chirp_out || P.conj_in || P.conj_out) return 0;
+        if (P.nload != P.N || (half && !P.rtw) || (real && P.ni != 1)) return 0;
+        if (P.store_mode == ST_TWIDDLE && (P.tw_mul != 1 || P.dst32)) return 0;
+        if ((P.ni - 1) * P.in.ipos + (long long)(P.N - 1) * P.in.pst >= P.ilim ||
+            (P.ni - 1) * P.out.ipos + (long long)(P.N - 1) * P.out.pst >= P.olim)
+            return 0;
+        const long long win = 0x7fffffffLL;
+        if (ref_bytes(src, P.in, P) > win || ref_bytes(dst, P.out, P) > win) return 0;
+        std::vector<int> rad;
+        int nt = 0;
+        if (!mix_factor(P.N, kMixMaxThreads, rad, nt)) return 0;
+        const auto key = std::make_pair(P.N, P.sign);
+        auto it = mix_tw.find(key);
+        if (it == mix_tw.end()) {
+            std::vector<double2> v;
+            mix_table(v, rad, P.sign);
+            auto b = upload(v);
+            if (!b) return -1;
+            it = mix_tw.emplace(key, (const double2 *)b->p).first;
+        }
+        P.tw = it->second;
+        P.nst = (int)rad.size();
+        P.codes = 0;
+        for (size_t k = 0; k < rad.size(); ++k) P.codes |= (unsigned)(rad[k] - 1) << (4 * k);
+        P.NT = nt;
+        // Transforms per workgroup.  Along rows one where it fills a wavefront, else two wavefronts'
+        // worth: small workgroups overlap one's loads with another's stages (float r2c rows of 1920
+        // 0.104 ms with 256 threads, 0.098 ms so; c2c rows of 1920 0.033 -> 0.031 ms).  Across
+        // transforms runs of 64 bytes, which 32-byte runs lose to (1080-point columns 0.171 ->
+        // 0.210 ms).  At most 80 KiB of LDS, so that two workgroups share a CU, and small grids
+        // are spread over the chip first.
+        const bool col = colL || colS;
+        const long long per = (long long)P.N * (long long)sizeof(double2);
+        const long long eb = (P.src32 || P.dst32) ? 8 : 16;
+        long long tb = col ? std::max<long long>(64 / eb, 256 / nt) : (nt >= 64 ? 1 : 128 / nt);
+        const long long cap = max_lds_bytes() - (long long)sizeof(long long) * 8 * kMaxTB - 1024;
+        const long long budget = std::min<long long>(80 * 1024, cap);
+        tb = std::min<long long>(std::min<long long>(tb, kMaxTB), std::min<long long>(budget / per, kMixMaxThreads / nt));
+        const long long want = std::max<long long>(col ? 2 : 1, P.ntf / 512);
+        tb = std::max<long long>(1, std::min(tb, want));
+        if (col)
+            while (tb & (tb - 1)) tb &= tb - 1;   // a power of two: lanes split with a mask
+        P.TB = (int)tb;
+        // lanes that walk across transforms meet distinct bank groups: row stride 8 / TB mod 8
+        P.LD = P.N;
+        if (col && tb > 1) {
+            const int off = tb >= 8 ? 1 : 8 / (int)tb;
+            while (P.LD % 8 != off) ++P.LD;
+        }
+        if ((long long)P.LD * tb * (long long)sizeof(double2) > cap) return 0;
+        P.col_load = tb > 1 && colL;
+        P.col_store = tb > 1 && colS;
+        Pass ps;
+        ps.kind = Pass::FFT_MIX;
+        ps.fp = P;
+        ps.block = (unsigned)(tb * nt);
+        const long long grid = (P.ntf + tb - 1) / tb;
+        if (grid > INT_MAX) return 0;
+        ps.grid = (unsigned)std::max<long long>(1, grid);
+        ps.lds = (size_t)P.LD * (size_t)tb * sizeof(double2);
+        ps.src = src;
+        ps.dst = dst;
+        ps.uses_fct = uses_fct;
+        ps.name = "k_fft_mix";
+        ps.bytes_in = side_bytes(P, true);
+        ps.bytes_out = side_bytes(P, false);
+        ps.in_words = P.load_mode == LD_REAL_HALF && even_side(P.in);
+        ps.out_words = P.store_mode == ST_C2R_HALF && even_side(P.out);
+        plan.passes.push_back(ps);
+        return 1;
+    }
+
+    // a real side whose elements 2p and 2p + 1 form one complex word at an even offset
+    static bool even_side(const Side &S)
+    {
+        if (S.sax != 1 || S.kind != SIDE_DIMS || S.isig % 2) return false;
+        for (int d = 0; d < S.nbd; ++d)
+            if (S.str[d] % 2) return false;
+        return true;
+    }
+
     // colL / colS: whether consecutive transforms are closer in memory than
     // consecutive points on the load / store side
     bool add_fft(FftParams P, BufRef src, BufRef dst, bool uses_fct, bool colL, bool colS)
     {
         io_flags(P, src, dst);
+        if (P.N > 1 && pow2_supported(P.N) && !P.tw && !(P.tw = table_direct(P.N))) return false;
         if (try_pow2(P, src, dst, uses_fct, colL, colS)) return true;
+        switch (try_mix(P, src, dst, uses_fct, colL, colS)) {
+            case 1: return true;
+            case -1: return false;
+            default: break;
+        }
+        if (P.N > 1 && !P.tw && !(P.tw = table_direct(P.N))) return false;
         const long long per = (long long)P.LD * (long long)sizeof(double2) * P.TB;
         const long long cap = max_lds_bytes() - (long long)sizeof(long long) * 8 * kMaxTB - 1024;
         if (per > cap) {
@@ -465,9 +575,7 @@ struct Builder {
         const bool real = J.kind != J_C2C;
         const bool pair = real && odd;
         const long long M = real ? (odd ? L : L / 2) : L;    // complex points in LDS
-        FftParams P = base(M);
-        P.tw = M > 1 ? table_direct(M) : nullptr;
-        if (M > 1 && !P.tw) return false;
+        FftParams P = base(M);   // the twiddle table follows from the kernel (add_fft)
         P.fwd_flag = J.forward;
         P.adj_w = J.adj;
         P.M = (int)M;
@@ -1329,7 +1437,7 @@ static int plan_execute_ws(Plan &P, const void *in, void *out, double fct, hipSt
         auto &ps = P.passes[pi];
         hipError_t e;
         if (prof) (void)hipEventRecord(ev[2 * pi], stream);
-        if (ps.kind == Pass::FFT_LDS || ps.kind == Pass::FFT_POW2) {
+        if (ps.kind == Pass::FFT_LDS || ps.kind == Pass::FFT_POW2 || ps.kind == Pass::FFT_MIX) {
             const void *srcp = resolve(ps.src);
             FftParams fp = (ps.has_alt && ((uintptr_t)srcp % (ps.fp_alt.src32 ? 8 : 16)) == 0) ? ps.fp_alt : ps.fp;
             fp.src = srcp;
@@ -1337,7 +1445,13 @@ static int plan_execute_ws(Plan &P, const void *in, void *out, double fct, hipSt
             window(ps.src, fp.src_lo, fp.src_span);
             window(ps.dst, fp.dst_lo, fp.dst_span);
             fp.fct = ps.uses_fct ? fct : 1.0;
-            if (ps.kind == Pass::FFT_POW2) {
+            if (ps.kind == Pass::FFT_MIX) {
+                fp.in_words = ps.in_words && (uintptr_t)srcp % (fp.src32 ? 8 : 16) == 0;
+                fp.out_words = ps.out_words && (uintptr_t)fp.dst % (fp.dst32 ? 8 : 16) == 0;
+                e = launch_fft_mix(fp, ps.grid, ps.block, ps.lds, stream);
+                ps.kname = "k_fft_mix<" + std::to_string(fp.load_mode) + ", " + std::to_string(fp.store_mode) + ", " +
+                           std::to_string(mix_wpe(ps.grid, ps.block)) + ">";
+            } else if (ps.kind == Pass::FFT_POW2) {
                 e = launch_fft_pow2(fp, ps.map, ps.grid, ps.block, ps.lds, stream);
                 ps.kname = "k_fft_pow2<" + std::to_string(fp.N) + ", " + std::to_string(ps.map) + ", " +
                            std::to_string(pow2_io(fp, ps.map, ps.grid, ps.block, ps.lds)) + ">";

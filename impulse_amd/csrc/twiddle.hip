@@ -6,6 +6,7 @@
 // which the reference's exact known-answer tests rely on
 // (tests/test_fft2.nim:7-15); PocketFFT obtains the same property by its own
 // octant reduction (impulse/fft/cpp_pocketfft/pocketfft_hdronly.h:277-349).
+#include <algorithm>
 #include <cmath>
 
 #include "engine.h"
@@ -52,6 +53,78 @@ void twiddle_table(std::vector<double2> &out, uint64_t n, uint64_t count, uint64
     out.resize(count);
     for (uint64_t j = 0; j < count; ++j)
         out[j] = twiddle_at((uint64_t)(((unsigned __int128)j * step) % n), n);
+}
+
+// ---------------------------------------------------------------------------
+// mixed-radix shapes (mix_fft.h)
+// ---------------------------------------------------------------------------
+
+// VALU operations of one radix-R butterfly, counted from the code
+static int dft_ops(int R)
+{
+    static const int ops[17] = {0, 0, 4, 16, 16, 40, 44, 72, 60, 120, 100, 160, 112, 216, 172, 200, 170};
+    return ops[R];
+}
+
+// Factors N into 2 .. 4 radices of 2 .. 16 and the threads per transform they take, or returns
+// false.  The cheapest order by operation count wins: butterflies, twiddle products, the LDS
+// accesses of each stage with the bank conflicts of the first stage's writes (their stride is the
+// radix: 16-byte words fall on 8 bank groups, so an odd first radix has none), and the
+// per-stage overhead of every thread.
+bool mix_factor(int N, int max_threads, std::vector<int> &radices, int &threads)
+{
+    if (N < 4) return false;
+    double best = -1.0;
+    std::vector<int> cur;
+    auto nb_of = [](int R) { return R > 8 ? 1 : 16 / R; };   // mix_nb
+    auto rec = [&](auto &&self, int n) -> void {
+        if (n == 1 && cur.size() >= 2) {
+            int nt = 1;
+            for (int R : cur) nt = std::max(nt, (N / R + nb_of(R) - 1) / nb_of(R));
+            if (nt > max_threads) return;
+            double cost = 0.0;
+            for (size_t k = 0; k < cur.size(); ++k) {
+                const int R = cur[k];
+                cost += (double)(N / R) * (dft_ops(R) + (k ? 4 * (R - 1) : 0) + 10 * R) + 60.0 * nt;
+            }
+            int g = cur[0];
+            g = (g & 1) ? 1 : (g & 2) ? 2 : (g & 4) ? 4 : 8;   // gcd with the 8 bank groups
+            cost += 4.0 * N * (g - 1);
+            if (best < 0.0 || cost < best) {
+                best = cost;
+                radices = cur;
+                threads = nt;
+            }
+            return;
+        }
+        if (cur.size() >= 4) return;
+        for (int R = 2; R <= 16; ++R)
+            if (n % R == 0) {
+                cur.push_back(R);
+                self(self, n / R);
+                cur.pop_back();
+            }
+    };
+    rec(rec, N);
+    return best >= 0.0;
+}
+
+// the twiddles of stages 1, 2, ... in stage order: W_{pR}^{qk} at (q - 1) p + k, q = 1 .. R - 1,
+// k < p, p the product of the earlier radices; conjugated for sign > 0
+void mix_table(std::vector<double2> &out, const std::vector<int> &radices, int sign)
+{
+    out.clear();
+    int p = radices[0];
+    for (size_t s = 1; s < radices.size(); ++s) {
+        const int R = radices[s];
+        for (int q = 1; q < R; ++q)
+            for (int k = 0; k < p; ++k) {
+                double2 w = twiddle_at((uint64_t)q * (uint64_t)k, (uint64_t)p * (uint64_t)R);
+                if (sign > 0) w.y = -w.y;
+                out.push_back(w);
+            }
+        p *= R;
+    }
 }
 
 }  // namespace ifft
