@@ -12,28 +12,40 @@
 // stored by the forward pass.  Inputs and outputs are float32 or float64; all
 // arithmetic is FP64.
 //
-// Fused path (7-smooth grids with Q/2 <= 2560 and P <= 2560): three kinds of LDS kernels
-// over half spectra kept in row layout S[img][r][j] (j < Qh = Q/2 + 1), and only
-// for the rows an image occupies:
+// Fused path (grids with P <= 2560 and Q/2 <= 2560): three kinds of mixed-radix kernels (mix_fft.h)
+// over half spectra, and only for the rows an image occupies:
 //   rows   : real rows read straight from the caller's array (the padding is
 //            generated, never stored), r2c of length Q by the half-length
 //            complex transform, half spectrum out;
-//   columns: each column group loads its image rows at their grid offset (the
-//            other P - H rows are zeros in LDS), transforms, multiplies by K^
-//            (conj K^ for the adjoint) and transforms back, keeping only the
+//   columns: each workgroup loads its columns' image rows at their grid offset (the
+//            other P - H rows are zeros), transforms, multiplies by K^ (conj K^ for
+//            the adjoint) and transforms back in one kernel, keeping only the
 //            rows the crop needs -- or, for the kernel gradient, sums
 //            conj(X^_b) G^_b over the images of a chunk;
 //   rows^-1: c2r of the kept rows, the cropped columns scaled and stored in the
 //            caller's dtype.
 // Three passes over half spectra instead of pad / r2c / multiply / c2r / crop
 // over the whole padded grid.  Larger grids take the plan-based path.
+//
+// The half spectra are kept in column blocks, S[img][block][row][cb] with cb neighbouring columns
+// (the columns of one workgroup): a column workgroup reads and writes one contiguous run of
+// memory, and a row workgroup of several rows writes rows cb 16 bytes at a time.
+//
+// Measured on one MI355X, 16 x 2048^2 images and a 63 x 63 kernel in float32 (grid 2160 x 2100),
+// against LDS kernels that staged every point at both ends: rows 0.41 -> 0.25 ms (0.82 GB moved),
+// columns of the convolution 1.04 -> 0.31 ms (1.10 GB), of the kernel gradient 1.21 -> 0.57 ms (1.10
+// GB), rows^-1 0.35 -> 0.26 ms; forward and backward together 5.2 -> 2.6 ms.  Bounds now: the
+// convolution's columns move their bytes at 3.5 TB/s with VALU issue at 40 %; the rows are held by
+// LDS (67 KB, two workgroups a CU); the kernel gradient's image loop serialises its loads with its
+// barriers, at 12 wavefronts a CU.
 #include <algorithm>
 #include <cstring>
+#include <initializer_list>
 #include <vector>
 
 #include "engine.h"
 #include "fft_common.h"
-#include "lds_fft.h"
+#include "mix_fft.h"
 
 namespace ifft {
 
@@ -96,243 +108,416 @@ __global__ void k_spec_corr_reduce(const double2 *__restrict__ a, const double2 
 // fused path
 // ---------------------------------------------------------------------------
 
-// The LDS transforms are inlined (no call frames in scratch memory) and use
-// radices 2-8 only, so the fused path runs on 7-smooth grids: kConvPPT points a
-// thread at most, 512-thread row kernels (two workgroups a CU) and 1,024-thread
-// column kernels, all within 128 registers.
-constexpr int kConvPPT = 5;
-constexpr int kConvOrder = 2;          // powers of two as radix-8 stages
-constexpr int kConvRowThreads = 512;
-constexpr int kConvColThreads = 1024;
-constexpr int kConvColPoints = kConvPPT * kConvColThreads;   // points of one column LDS batch
+constexpr int kConvThreads = 512;      // workgroup size cap of the fused kernels
+constexpr int kConvMaxLen = 2560;      // longest rows (complex points) and columns of the fused path
+constexpr int kConvMaxTb = 64;         // rows per workgroup of the row kernels at most
+constexpr int kConvAcc = 8;            // kernel-gradient sums a thread holds (P / 2 points over NT threads)
 
-// real rows -> half spectra: row q of src (W values, placed at grid columns
-// [rx, rx + W) of a Q-point row, zeros elsewhere) -> S[q][0 .. Q/2]
-struct ConvRows {
-    const void *src;
-    double2 *S;
-    const double2 *tq;   // W_Q^j = exp(-2 pi i j / Q), j < Q
-    long long rows;
-    int W, Q, rx, f32, count, lc;
+// half spectra in column blocks: element (img, row, j) of `rows` rows per image
+struct ConvSpec {
+    double2 *p;
+    int rows, nblk, lcb;   // rows per image, blocks per row, log2 of the columns per block
+    __device__ __forceinline__ long long block(long long img, int blk) const
+    {
+        return ((img * nblk + blk) * rows) << lcb;
+    }
 };
 
-// half spectra -> real rows: S[q][0 .. Q/2] -> dst[q][c] = scale * x[ox + c], c < Wout,
-// x the unnormalised c2r of length Q
-struct ConvRowsInv {
-    const double2 *S;
+// real rows -> half spectra: row q of src (W values, placed at grid columns
+// [rx, rx + W) of a 2 M-point row, zeros elsewhere) -> S(q, 0 .. M)
+struct ConvRowSet {
+    const void *src;
+    ConvSpec S;
+    long long rows;       // rows of all images
+    long long span;       // bytes a workgroup's rows may reach from their first image on
+    int W, rx;
+    unsigned groups;      // workgroups of this set
+};
+// Up to three sets of rows share one launch: the few rows of the convolution kernel would take a
+// launch of their own 44 us (one workgroup's latency) beside the 250 us of the images' rows.
+struct ConvRows {
+    ConvRowSet set[3];
+    MixShape F;
+    const double2 *rtw;   // W_{2M}^k, k <= M / 2
+    int nset, f32, ltb;   // ltb: log2 of the rows per workgroup
+};
+
+// half spectra -> real rows: S(q, 0 .. M) -> dst[q][c] = scale * x[ox + c], c < Wout,
+// x the unnormalised c2r of length 2 M
+struct ConvRowInvSet {
+    ConvSpec S;
     void *dst;
-    const double2 *tq;
-    long long rows;
-    int Wout, Q, ox, f32, count, lc;
+    long long rows, span;
+    int Wout, ox;
+    unsigned groups;
+};
+struct ConvRowsInv {
+    ConvRowInvSet set[2];
+    MixShape F;
+    const double2 *rtw;
+    int nset, f32, ltb;
     double scale;
 };
 
-// column groups of `count` spectrum columns (grid rows 0 .. P-1)
+// column passes over blocks of cb columns (grid rows 0 .. P-1, image rows at [r0, r0 + S.rows))
 struct ConvCols {
-    const double2 *Sa;   // image rows [img][Ha][Qh], placed at grid rows [ra, ra + Ha)
-    const double2 *Sg;   // kernel gradient: gradient rows [img][Ha][Qh] at grid rows [rg, rg + Ha)
-    double2 *Sout;       // kept rows [oy, oy + Ho) as [img][Ho][Qh]; spectrum mode: [Qh][P]
-    const double2 *KT;   // kernel spectrum [Qh][P]
-    double2 *acc;        // kernel-gradient partial sums [nchunk][Qh][P]
-    const double2 *tp;   // W_P^j, j < P
-    int P, Qh, Ha, ra, rg, oy, Ho, nimg, chunk, nchunk, count, lc, conjk;
+    ConvSpec Sa, Sg;       // image rows; gradient rows (kernel gradient)
+    ConvSpec So;           // kept rows: grid rows [oy, oy + So.rows)
+    double2 *KT;           // kernel spectrum [block][P][cb]
+    double2 *acc;          // kernel-gradient partial sums [chunk][block][P][cb]
+    MixShape F, I;         // forward, and the inverse with reversed radices
+    int ra, rg, oy, nimg, chunk, nchunk, conjk, sub;
 };
 
 enum ConvColMode { CC_SPECTRUM = 0, CC_CONV = 1, CC_GK = 2, CC_GK_FINAL = 3 };
 
-template <int THREADS>
-__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) k_conv_rows(const ConvRows P)
-{
-    extern __shared__ double2 zl[];
-    const int M = P.Q >> 1, Qh = M + 1;
-    const int NT = THREADS >> P.lc;
-    const int t = (int)threadIdx.x / NT, i = (int)threadIdx.x - t * NT;
-    for (long long r0 = (long long)blockIdx.x * P.count; r0 < P.rows; r0 += (long long)gridDim.x * P.count) {
-        const long long row = r0 + t;
-        const bool valid = row < P.rows;
-        if (valid) {
-            const long long base = row * P.W;
-            for (int m = i; m < M; m += NT) {
-                const int c0 = 2 * m - P.rx, c1 = c0 + 1;
-                const double a = (c0 >= 0 && c0 < P.W) ? gld_r(P.src, P.f32, base + c0) : 0.0;
-                const double b = (c1 >= 0 && c1 < P.W) ? gld_r(P.src, P.f32, base + c1) : 0.0;
-                zl[lpad(t * M + m)] = make_double2(a, b);
-            }
-        }
-        __syncthreads();
-        lds_fft_inline<kConvPPT, true>(zl, M, P.count, -1.0, kConvOrder, TwTable{P.tq, P.Q});   // ends with a barrier
-        if (valid) {
-            // X[k] = E + W_Q^k O, E = (Z[k] + conj Z[M-k]) / 2, O = (Z[k] - conj Z[M-k]) / 2i, k <= M
-            double2 *out = P.S + row * Qh;
-            for (int k = i; k <= M; k += NT) {
-                const double2 zk = zl[lpad(t * M + (k == M ? 0 : k))];
-                const double2 zm = zl[lpad(t * M + (k == 0 ? 0 : M - k))];
-                const double2 e = cscale(cadd(zk, cconj(zm)), 0.5), d = csub(zk, cconj(zm));
-                const double2 o = make_double2(0.5 * d.y, -0.5 * d.x);
-                out[k] = cadd(e, cmul(o, P.tq[k]));
-            }
-        }
-        __syncthreads();
-    }
-}
+// 32-bit offset that a buffer access never finds in range: loads give zero, stores are dropped
+constexpr int kNowhere = 0x7ffffff0;
 
-template <int THREADS>
-__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) k_conv_rows_inv(const ConvRowsInv P)
-{
-    extern __shared__ double2 zl[];
-    const int M = P.Q >> 1, Qh = M + 1;
-    const int NT = THREADS >> P.lc;
-    const int t = (int)threadIdx.x / NT, i = (int)threadIdx.x - t * NT;
-    for (long long r0 = (long long)blockIdx.x * P.count; r0 < P.rows; r0 += (long long)gridDim.x * P.count) {
-        const long long row = r0 + t;
-        const bool valid = row < P.rows;
-        if (valid) {
-            // Z[k] = E + i O, E = (X[k] + conj X[M-k]) / 2, O = (X[k] - conj X[M-k]) conj(W_Q^k) / 2;
-            // the imaginary parts of X[0] and X[M] are ignored, as c2r does
-            const double2 *X = P.S + row * Qh;
-            for (int k = i; k < M; k += NT) {
-                double2 a = X[k], b = X[M - k];
-                if (k == 0) {
-                    a.y = 0.0;
-                    b.y = 0.0;
-                }
-                const double2 e = cscale(cadd(a, cconj(b)), 0.5);
-                const double2 o = cmul(cscale(csub(a, cconj(b)), 0.5), cconj(P.tq[k]));
-                zl[lpad(t * M + k)] = make_double2(e.x - o.y, e.y + o.x);
-            }
-        }
-        __syncthreads();
-        lds_fft_inline<kConvPPT, true>(zl, M, P.count, 1.0, kConvOrder, TwTable{P.tq, P.Q});   // ends with a barrier
-        if (valid) {
-            // x[2m] = 2 Re z[m], x[2m+1] = 2 Im z[m] for the unnormalised length-Q transform
-            const double f = 2.0 * P.scale;
-            for (int c = i; c < P.Wout; c += NT) {
-                const int q = c + P.ox;
-                const double2 z = zl[lpad(t * M + (q >> 1))];
-                gst_r(P.dst, P.f32, row * P.Wout + c, f * ((q & 1) ? z.y : z.x));
-            }
-        }
-        __syncthreads();
-    }
-}
-
-// One workgroup per column group (and, for the convolution and the backward
-// pass, per chunk of images).  Column positions run with the column index
-// fastest (e = m * count + t), so a wave reads and writes runs of `count`
-// neighbouring bins of a spectrum row.
-template <int MODE>
-__global__ void __launch_bounds__(kConvColThreads) 
-k_conv_cols(const ConvCols C)
-{
-    extern __shared__ double2 zl[];
-    constexpr int T = kConvColThreads;
-    const int P = C.P, Qh = C.Qh, cnt = C.count, lc = C.lc, n = cnt * P;
-    const int ngroups = (Qh + cnt - 1) >> lc;
-    const int logical = (int)xcd_block(blockIdx.x, gridDim.x);
-    const int group = logical % ngroups, chunk = logical / ngroups;
-    const int tid = (int)threadIdx.x;
-    const TwTable tw{C.tp, P};
-
-    // image rows of column group `group` at grid rows [r0, r0 + Ha), zeros elsewhere
-    constexpr int NQ = kConvColPoints / T + 1;   // column-group positions a thread owns: e = tid + q T
-    auto load = [&](double2 *buf, const double2 *S, long long img, int r0) {
-        for (int e = tid; e < n; e += T) {
-            const int t = e & (cnt - 1), m = e >> lc, j = group * cnt + t, r = m - r0;
-            double2 v = make_double2(0.0, 0.0);
-            if (j < Qh && r >= 0 && r < C.Ha) v = S[(img * C.Ha + r) * Qh + j];
-            buf[lpad(t * P + m)] = v;
-        }
-        __syncthreads();
-    };
-    auto store = [&](const double2 *buf, long long img) {
-        for (int e = tid; e < cnt * C.Ho; e += T) {
-            const int t = e & (cnt - 1), r = e >> lc, j = group * cnt + t;
-            if (j < Qh) C.Sout[(img * C.Ho + r) * Qh + j] = buf[lpad(t * P + C.oy + r)];
-        }
-        __syncthreads();
-    };
-    // the kernel spectrum at the thread's positions, read once for all images of the chunk
-    auto kernel_values = [&](double2 (&kr)[NQ], bool conj) {
+struct ConvRowIn {
+    __amdgpu_buffer_rsrc_t r;
+    int base, W, rx, f32;   // element offset of the row in the window (kNowhere / 16: no row)
+    bool pairs;             // both words of a point sit in one aligned complex word, or are both outside
+    template <int R> __device__ __forceinline__ void load(double2 *v, int b, int nb) const
+    {
+        if (pairs && f32) {
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const int e = tid + q * T, t = e & (cnt - 1), m = e >> lc, j = group * cnt + t;
-            double2 k = make_double2(0.0, 0.0);
-            if (e < n && j < Qh) k = C.KT[(long long)j * P + m];
-            kr[q] = conj ? cconj(k) : k;
+            for (int q = 0; q < R; ++q) {
+                const int c = 2 * (b + q * nb) - rx;
+                const float2 f = bloadf2(r, (unsigned)c < (unsigned)W ? (base + c) * 4 : kNowhere);
+                v[q] = make_double2((double)f.x, (double)f.y);
+            }
+        } else if (pairs) {
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                const int c = 2 * (b + q * nb) - rx;
+                v[q] = bload2(r, (unsigned)c < (unsigned)W ? (base + c) * 8 : kNowhere);
+            }
+        } else if (f32) {
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                const int c = 2 * (b + q * nb) - rx;
+                v[q] = make_double2((double)bloadf1(r, (unsigned)c < (unsigned)W ? (base + c) * 4 : kNowhere),
+                                    (double)bloadf1(r, (unsigned)(c + 1) < (unsigned)W ? (base + c + 1) * 4 : kNowhere));
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                const int c = 2 * (b + q * nb) - rx;
+                v[q] = make_double2(bload1(r, (unsigned)c < (unsigned)W ? (base + c) * 8 : kNowhere),
+                                    bload1(r, (unsigned)(c + 1) < (unsigned)W ? (base + c + 1) * 8 : kNowhere));
+            }
         }
-    };
+    }
+};
+
+// byte offset of row `row`'s first bin from the start of image img0
+__device__ __forceinline__ int conv_row_off(const ConvSpec &S, long long row, long long img0)
+{
+    const long long img = row / S.rows;
+    const int r = (int)(row - img * S.rows);
+    return (int)((S.block(img, 0) - S.block(img0, 0) + ((long long)r << S.lcb)) * 16);
+}
+// byte offset of bin k from its row's first bin
+__device__ __forceinline__ int conv_bin_off(const ConvSpec &S, int k)
+{
+    return (((k >> S.lcb) * S.rows << S.lcb) + (k & ((1 << S.lcb) - 1))) * 16;
+}
+
+template <int WPE>
+__global__ void __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(WPE))) k_conv_rows(const ConvRows P)
+{
+    extern __shared__ double2 zl[];
+    __shared__ int roff[kConvMaxTb];
+    const int tid = (int)threadIdx.x, M = P.F.N, NT = P.F.NT, tb = 1 << P.ltb;
+    unsigned blk = xcd_block(blockIdx.x, gridDim.x);
+    int which = 0;
+    while (which + 1 < P.nset && blk >= P.set[which].groups) blk -= P.set[which++].groups;
+    const ConvRowSet &A = P.set[which];
+    const ConvSpec S = A.S;
+    const long long q0 = (long long)blk * tb;
+    const int t = tid / NT, i = tid - t * NT;
+    const int es = P.f32 ? 4 : 8;
+    const int nrow = (int)(A.rows - q0 < tb ? A.rows - q0 : tb);
+    const long long img0 = q0 / S.rows;
+    if (tid < nrow) roff[tid] = conv_row_off(S, q0 + tid, img0);
+    ConvRowIn in;
+    in.r = make_rsrc((const char *)A.src + q0 * A.W * es, (long long)nrow * A.W * es);
+    in.base = t * A.W;
+    in.W = t < nrow ? A.W : 0;
+    in.rx = A.rx;
+    in.f32 = P.f32;
+    in.pairs = !(A.rx & 1) && !(A.W & 1) && (uintptr_t)A.src % (2 * es) == 0;
+    double2 *row = zl + t * M;
+    mix_fft<false, true, -1>(P.F, row, i, true, row, i, true, -1.0, in, MixLds{row});   // ends with a barrier
+    // X[k] = E + W_{2M}^k O and X[M-k] = conj(E) - conj(W^k O), E = (Z[k] + conj Z[M-k]) / 2,
+    // O = (Z[k] - conj Z[M-k]) / 2i.  Lanes walk a block's columns, then the rows; four bin pairs
+    // in flight per thread.
+    const int nthr = tb * NT, lc = S.lcb + P.ltb;
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(P.rtw, ((long long)(M / 2) + 1) * 16);
+    const __amdgpu_buffer_rsrc_t ro = make_rsrc(S.p + S.block(img0, 0), A.span);
+    const int top = M / 2;
+    const int total = ((top >> S.lcb) + 1) << lc;   // whole blocks of bins
+    for (int e0 = tid; e0 < total; e0 += 4 * nthr) {
+        double2 w[4], z[4], m[4];
+        int kk[4], tt[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int e = e0 + c * nthr;
+            tt[c] = (e >> S.lcb) & (tb - 1);
+            kk[c] = (e >> lc << S.lcb) + (e & ((1 << S.lcb) - 1));
+            const int k = min(kk[c], top);
+            w[c] = bload2(rw, k * 16);
+            const double2 *zr = zl + tt[c] * M;
+            z[c] = zr[k];
+            m[c] = zr[k ? M - k : 0];
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int k = kk[c], km = M - k;
+            if (k > top || tt[c] >= nrow) continue;
+            const double2 zm = cconj(m[c]);
+            const double2 ev = cscale(cadd(z[c], zm), 0.5), d = csub(z[c], zm);
+            const double2 o = cmul(make_double2(0.5 * d.y, -0.5 * d.x), w[c]);
+            const int off = roff[tt[c]];
+            bstore2(ro, off + conv_bin_off(S, k), cadd(ev, o));
+            bstore2(ro, off + conv_bin_off(S, km), make_double2(ev.x - o.x, o.y - ev.y));
+        }
+    }
+}
+
+struct ConvRowOut {
+    __amdgpu_buffer_rsrc_t r;
+    int base, Wout, ox, f32;
+    double f;
+    template <int R, class G> __device__ __forceinline__ void store(const double2 *v, int n, int dn, G) const
+    {
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const int c = 2 * (n + q * dn) - ox;
+            const bool a = (unsigned)c < (unsigned)Wout, b = (unsigned)(c + 1) < (unsigned)Wout;
+            if (f32) {
+                bstoref1(r, a ? (base + c) * 4 : kNowhere, f * v[q].x);
+                bstoref1(r, b ? (base + c + 1) * 4 : kNowhere, f * v[q].y);
+            } else {
+                bstore1(r, a ? (base + c) * 8 : kNowhere, f * v[q].x);
+                bstore1(r, b ? (base + c + 1) * 8 : kNowhere, f * v[q].y);
+            }
+        }
+    }
+};
+
+template <int WPE>
+__global__ void __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(WPE))) k_conv_rows_inv(const ConvRowsInv P)
+{
+    extern __shared__ double2 zl[];
+    __shared__ int roff[kConvMaxTb];
+    const int tid = (int)threadIdx.x, M = P.F.N, NT = P.F.NT, tb = 1 << P.ltb;
+    unsigned blk = xcd_block(blockIdx.x, gridDim.x);
+    int which = 0;
+    while (which + 1 < P.nset && blk >= P.set[which].groups) blk -= P.set[which++].groups;
+    const ConvRowInvSet &A = P.set[which];
+    const ConvSpec S = A.S;
+    const long long q0 = (long long)blk * tb;
+    const int nrow = (int)(A.rows - q0 < tb ? A.rows - q0 : tb);
+    const long long img0 = q0 / S.rows;
+    if (tid < nrow) roff[tid] = conv_row_off(S, q0 + tid, img0);
+    __syncthreads();
+    const int nthr = tb * NT, lc = S.lcb + P.ltb;
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(P.rtw, ((long long)(M / 2) + 1) * 16);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(S.p + S.block(img0, 0), A.span);
+    const int top = M / 2;
+    const int total = ((top >> S.lcb) + 1) << lc;
+    // Z[k] = E + i O, E = X[k] + conj X[M-k], O = (X[k] - conj X[M-k]) conj(W^k), and Z[M-k] =
+    // conj(E) + i conj(O); the imaginary parts of X[0] and X[M] are ignored, as c2r does
+    for (int e0 = tid; e0 < total; e0 += 4 * nthr) {
+        double2 w[4], x[4], m[4];
+        int kk[4], tt[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int e = e0 + c * nthr;
+            tt[c] = (e >> S.lcb) & (tb - 1);
+            kk[c] = (e >> lc << S.lcb) + (e & ((1 << S.lcb) - 1));
+            const int k = min(kk[c], top);
+            const int off = tt[c] < nrow ? roff[tt[c]] : kNowhere / 2;
+            w[c] = bload2(rw, k * 16);
+            x[c] = bload2(rs, off + conv_bin_off(S, k));
+            m[c] = bload2(rs, off + conv_bin_off(S, M - k));
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int k = kk[c];
+            if (k > top || tt[c] >= nrow) continue;
+            double2 a = x[c], b = m[c];
+            if (k == 0) a.y = b.y = 0.0;
+            const double2 ev = cadd(a, cconj(b)), o = cmul(csub(a, cconj(b)), cconj(w[c]));
+            double2 *zr = zl + tt[c] * M;
+            zr[k] = make_double2(ev.x - o.y, ev.y + o.x);
+            if (k && 2 * k != M) zr[M - k] = make_double2(ev.x + o.y, o.x - ev.y);
+        }
+    }
+    __syncthreads();
+    const int t = tid / NT, i = tid - t * NT;
+    const int es = P.f32 ? 4 : 8;
+    double2 *row = zl + t * M;
+    ConvRowOut out;
+    out.r = make_rsrc((char *)A.dst + q0 * A.Wout * es, (long long)nrow * A.Wout * es);
+    out.base = t * A.Wout;
+    out.Wout = t < nrow ? A.Wout : 0;
+    out.ox = A.ox;
+    out.f32 = P.f32;
+    out.f = P.scale;
+    mix_fft<true, false, 1>(P.F, row, i, true, row, i, true, 1.0, MixLds{row}, out);
+}
+
+// column `t` of a block: rows [r0, r0 + rows) of the grid, zeros elsewhere
+struct ConvColIn {
+    __amdgpu_buffer_rsrc_t r;
+    int t, lcb, rows, r0;
+    template <int R> __device__ __forceinline__ void load(double2 *v, int b, int nb) const
+    {
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const int m = b + q * nb - r0;
+            v[q] = bload2(r, (unsigned)m < (unsigned)rows ? ((m << lcb) + t) * 16 : kNowhere);
+        }
+    }
+};
+
+// the same from a pointer of the thread's own (x and g columns side by side in one workgroup)
+struct ConvColIn2 {
+    const double2 *col;
+    int lcb, rows, r0;
+    template <int R> __device__ __forceinline__ void load(double2 *v, int b, int nb) const
+    {
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const int m = b + q * nb - r0;
+            const bool ok = (unsigned)m < (unsigned)rows;
+            const double2 x = col[(ok ? m : 0) << lcb];
+            v[q] = ok ? x : make_double2(0.0, 0.0);
+        }
+    }
+};
+
+// grid rows [oy, oy + rows) of column `t`
+struct ConvColOut {
+    __amdgpu_buffer_rsrc_t r;
+    int t, lcb, rows, oy;
+    template <int R, class G> __device__ __forceinline__ void store(const double2 *v, int n, int dn, G) const
+    {
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const int m = n + q * dn - oy;
+            bstore2(r, (unsigned)m < (unsigned)rows ? ((m << lcb) + t) * 16 : kNowhere, v[q]);
+        }
+    }
+};
+
+// v[q] times K^ (or conj K^) at column positions b + q nb
+struct ConvColMul {
+    __amdgpu_buffer_rsrc_t r;
+    int t, lcb;
+    double cj;
+    template <int R> __device__ __forceinline__ void apply(double2 *v, int b, int nb) const
+    {
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            double2 k = bload2(r, (((b + q * nb) << lcb) + t) * 16);
+            k.y *= cj;
+            v[q] = cmul(v[q], k);
+        }
+    }
+};
+
+// sum of the chunks' partial spectra of column `t`
+struct ConvAccIn {
+    const double2 *acc;
+    long long step;   // elements from one chunk to the next
+    int n, t, lcb;
+    template <int R> __device__ __forceinline__ void load(double2 *v, int b, int nb) const
+    {
+#pragma unroll
+        for (int q = 0; q < R; ++q) v[q] = make_double2(0.0, 0.0);
+        for (int c = 0; c < n; ++c)
+#pragma unroll
+            for (int q = 0; q < R; ++q) v[q] = cadd(v[q], acc[c * step + ((b + q * nb) << lcb) + t]);
+    }
+};
+
+template <int MODE, int WPE>
+__global__ void __launch_bounds__(MODE == CC_GK && WPE == 4 ? 2 * kConvThreads : kConvThreads)
+__attribute__((amdgpu_waves_per_eu(WPE))) k_conv_cols(const ConvCols C)
+{
+    extern __shared__ double2 zl[];
+    const int P = C.F.N, NT = C.F.NT, lcb = C.Sa.lcb, cb = 1 << lcb, nblk = C.Sa.nblk;
+    const int tid = (int)threadIdx.x;
+    const unsigned logical = xcd_block(blockIdx.x, gridDim.x);
+    // LDS row stride: lanes that walk across columns meet distinct bank groups
+    const int cols = MODE == CC_GK ? 2 * C.sub : cb;
+    const int t = tid & (cols - 1), i = tid / cols;
+    const int ld = cols > 1 ? P + ((8 / cols - P) & 7) : P;
+    double2 *row = zl + t * ld;
+    const long long span = ((long long)P << lcb) * 16;   // one block of kernel or partial spectrum
 
     if constexpr (MODE == CC_SPECTRUM) {
-        load(zl, C.Sa, 0, C.ra);
-        lds_fft_inline<kConvPPT, true>(zl, P, cnt, -1.0, kConvOrder, tw);
-        for (int e = tid; e < n; e += T) {
-            const int t = e & (cnt - 1), m = e >> lc, j = group * cnt + t;
-            if (j < Qh) C.Sout[(long long)j * P + m] = zl[lpad(t * P + m)];
-        }
+        const int blk = (int)logical;
+        const ConvColIn in{make_rsrc(C.Sa.p + C.Sa.block(0, blk), ((long long)C.Sa.rows << lcb) * 16), t, lcb, C.Sa.rows, C.ra};
+        const ConvColOut out{make_rsrc(C.KT + ((long long)blk * P << lcb), span), t, lcb, P, 0};
+        mix_fft<false, false, -1>(C.F, row, i, true, row, i, true, -1.0, in, out);
     } else if constexpr (MODE == CC_CONV) {
-        double2 kr[NQ];
-        kernel_values(kr, C.conjk != 0);
-        const int b1 = min(C.nimg, (chunk + 1) * C.chunk);
-        for (int b = chunk * C.chunk; b < b1; ++b) {
-            load(zl, C.Sa, b, C.ra);
-            lds_fft_inline<kConvPPT, true>(zl, P, cnt, -1.0, kConvOrder, tw);
-#pragma unroll
-            for (int q = 0; q < NQ; ++q) {
-                const int e = tid + q * T;
-                if (e < n) {
-                    const int p = lpad((e & (cnt - 1)) * P + (e >> lc));
-                    zl[p] = cmul(zl[p], kr[q]);
-                }
-            }
-            __syncthreads();
-            lds_fft_inline<kConvPPT, true>(zl, P, cnt, 1.0, kConvOrder, tw);
-            store(zl, b);
-        }
+        // images fastest: neighbouring workgroups share their block of K^ in the L2
+        const int img = (int)(logical % (unsigned)C.nimg), blk = (int)(logical / (unsigned)C.nimg);
+        const ConvColIn in{make_rsrc(C.Sa.p + C.Sa.block(img, blk), ((long long)C.Sa.rows << lcb) * 16), t, lcb, C.Sa.rows, C.ra};
+        const ConvColMul mul{make_rsrc(C.KT + ((long long)blk * P << lcb), span), t, lcb, C.conjk ? -1.0 : 1.0};
+        const ConvColOut out{make_rsrc(C.So.p + C.So.block(img, blk), ((long long)C.So.rows << lcb) * 16), t, lcb, C.So.rows, C.oy};
+        mix_conv(C.F, C.I, row, i, in, mul, out);
     } else if constexpr (MODE == CC_GK) {
-        // x and g spectra of the column group in one LDS batch (lines 0 .. cnt-1 and cnt .. 2cnt-1),
-        // transformed together; the chunk's sum of conj(X^) G^ in registers
-        constexpr int NQG = kConvPPT * T / 2 / T + 1;
-        double2 acc[NQG];
+        // x and g columns transformed together (slots 0 .. sub-1 and sub .. 2 sub - 1), `sub` columns
+        // of a block per workgroup; the chunk's sum of conj(X^) G^ in registers
+        const int nsub = cb / C.sub;
+        const int part = (int)(logical % (unsigned)nsub);
+        const int blk = (int)(logical / (unsigned)nsub % (unsigned)nblk), chunk = (int)(logical / (unsigned)(nsub * nblk));
+        const bool isg = t >= C.sub;
+        const int nthr = cols * NT, n = C.sub * P;
+        double2 acc[kConvAcc];
 #pragma unroll
-        for (int q = 0; q < NQG; ++q) acc[q] = make_double2(0.0, 0.0);
+        for (int q = 0; q < kConvAcc; ++q) acc[q] = make_double2(0.0, 0.0);
         const int b1 = min(C.nimg, (chunk + 1) * C.chunk);
         for (int b = chunk * C.chunk; b < b1; ++b) {
-            for (int e = tid; e < 2 * n; e += T) {
-                const int half = e >= n ? 1 : 0, f = e - half * n;
-                const int t = f & (cnt - 1), m = f >> lc, j = group * cnt + t, r = m - (half ? C.rg : C.ra);
-                double2 v = make_double2(0.0, 0.0);
-                if (j < Qh && r >= 0 && r < C.Ha) v = (half ? C.Sg : C.Sa)[((long long)b * C.Ha + r) * Qh + j];
-                zl[lpad((half * cnt + t) * P + m)] = v;
-            }
-            __syncthreads();
-            lds_fft_inline<kConvPPT, true>(zl, P, 2 * cnt, -1.0, kConvOrder, tw);
+            const ConvColIn2 in{(isg ? C.Sg.p : C.Sa.p) + C.Sa.block(b, blk) + part * C.sub + (t & (C.sub - 1)), lcb,
+                                C.Sa.rows, isg ? C.rg : C.ra};
+            mix_fft<false, true, -1>(C.F, row, i, true, row, i, true, -1.0, in, MixLds{row});
+            const int e0 = opaque(tid);   // the LDS addresses are not worth registers across the transform
 #pragma unroll
-            for (int q = 0; q < NQG; ++q) {
-                const int e = tid + q * T;
+            for (int q = 0; q < kConvAcc; ++q) {
+                const int e = e0 + q * nthr;
                 if (e < n) {
-                    const int t = e & (cnt - 1), m = e >> lc;
-                    acc[q] = cadd(acc[q], cmul(cconj(zl[lpad(t * P + m)]), zl[lpad((cnt + t) * P + m)]));
+                    const int tt = e & (C.sub - 1), m = e / C.sub;
+                    acc[q] = cadd(acc[q], cmul(cconj(zl[tt * ld + m]), zl[(C.sub + tt) * ld + m]));
                 }
             }
             __syncthreads();
         }
+        double2 *out = C.acc + ((((long long)chunk * nblk + blk) * P) << lcb);
 #pragma unroll
-        for (int q = 0; q < NQG; ++q) {
-            const int e = tid + q * T, t = e & (cnt - 1), m = e >> lc, j = group * cnt + t;
-            if (e < n && j < Qh) C.acc[((long long)chunk * Qh + j) * P + m] = acc[q];
+        for (int q = 0; q < kConvAcc; ++q) {
+            const int e = tid + q * nthr;
+            if (e < n) out[((e / C.sub) << lcb) + part * C.sub + (e & (C.sub - 1))] = acc[q];
         }
     } else {   // CC_GK_FINAL
-        for (int e = tid; e < n; e += T) {
-            const int t = e & (cnt - 1), m = e >> lc, j = group * cnt + t;
-            double2 v = make_double2(0.0, 0.0);
-            if (j < Qh)
-                for (int c = 0; c < C.nchunk; ++c) v = cadd(v, C.acc[((long long)c * Qh + j) * P + m]);
-            zl[lpad(t * P + m)] = v;
-        }
-        __syncthreads();
-        lds_fft_inline<kConvPPT, true>(zl, P, cnt, 1.0, kConvOrder, tw);
-        store(zl, 0);
+        const int blk = (int)logical;
+        const ConvAccIn in{C.acc + ((long long)blk * P << lcb), (long long)nblk * P << lcb, C.nchunk, t, lcb};
+        const ConvColOut out{make_rsrc(C.So.p + C.So.block(0, blk), ((long long)C.So.rows << lcb) * 16), t, lcb, C.So.rows, C.oy};
+        mix_fft<false, false, 1>(C.F, row, i, true, row, i, true, 1.0, in, out);
     }
+}
+
+static MixShape mix_shape(int N, const std::vector<int> &rad, int nt, const double2 *tw)
+{
+    MixShape S{N, (int)rad.size(), 0, nt, tw};
+    for (size_t k = 0; k < rad.size(); ++k) S.codes |= (unsigned)(rad[k] - 1) << (4 * k);
+    return S;
 }
 
 static unsigned blocks_for(long long total)
@@ -362,39 +547,37 @@ struct Conv2d {
     DevBuf pad, spec_a, spec_b, kspec, kpad;
     // fused path
     bool fused = false;
-    int row_count = 1, row_lc = 0, col_count = 1, col_lc = 0, gk_count = 1, gk_lc = 0, nchunk = 1, chunk = 1;
-    DevBuf tq, tp;          // W_Q^j (j < Q), W_P^j (j < P)
-    DevBuf sx, sg, sk, kt;  // half spectra [B][H][Qh] (two), kernel rows [KH][Qh], kernel spectrum [Qh][P]
-    DevBuf acc;             // kernel-gradient partial sums [nchunk][Qh][P]
+    int lcb = 0, ltb = 0, sub = 1, nblk = 1, nchunk = 1, chunk = 1;
+    MixShape Ff{}, Fi{};    // columns: forward, inverse with reversed radices
+    MixShape Rf{}, Ri{};    // rows: forward, inverse
+    DevBuf tab;             // their stage tables and W_Q^k, k <= Q/4
+    const double2 *rtw = nullptr;
+    DevBuf sx, sg, sk, kt;  // half spectra of the images (two) and of the kernel rows, kernel spectrum
+    DevBuf acc;             // kernel-gradient partial sums [nchunk][block][P][cb]
 };
 
-static int pow2_floor_int(long long v)
+// the cheapest length of at least `need` points the mixed-radix stages take (within 1/16, or the
+// first one found), by the operation count of a whole transform
+static long long conv_fused_len(long long need)
 {
-    int c = 1;
-    while (2LL * c <= v) c *= 2;
-    return c;
-}
-
-static int ilog2_int(int v)
-{
-    int l = 0;
-    while ((1 << l) < v) ++l;
-    return l;
-}
-
-// Fused path set-up for grids the LDS kernels hold: line counts per workgroup
-// (powers of two, at most 8 points per thread), image chunks, tables and
-// workspaces.  Leaves c.fused false for larger grids.
-static long long smooth7_at_least(long long n)
-{
-    for (;; ++n) {
-        long long r = n;
-        for (int p : {2, 3, 5, 7})
-            while (r % p == 0) r /= p;
-        if (r == 1) return n;
+    long long best = 0;
+    double cost = 0.0;
+    for (long long n = std::max<long long>(need, 4); n <= kConvMaxLen; ++n) {
+        if (best && n > need + need / 16) break;
+        std::vector<int> rad;
+        int nt;
+        double c;
+        if (!smooth13_c(n) || !mix_factor((int)n, kConvThreads / 2, rad, nt, &c)) continue;
+        if (!best || c < cost) {
+            best = n;
+            cost = c;
+        }
     }
+    return best;
 }
 
+// Fused path set-up for grids the kernels hold: block widths, image chunks,
+// tables and workspaces.  Leaves c.fused false for larger grids.
 static int conv_fused_setup(Conv2d &c, Error &err)
 {
     // A circular convolution of period P gives the 'same' rows [cy, cy + H) of the linear one when
@@ -402,102 +585,166 @@ static int conv_fused_setup(Conv2d &c, Error &err)
     // correlations of the backward pass need the same bound (their wrapped terms land outside
     // [0, KH) and [0, H)).  Likewise for the columns.
     const int cy = (c.KH - 1) / 2, cx = (c.KW - 1) / 2;
-    const long long P = smooth7_at_least((long long)c.H + std::max(cy, c.KH - 1 - cy));
-    const long long M = smooth7_at_least(((long long)c.W + std::max(cx, c.KW - 1 - cx) + 1) / 2), Qh = M + 1;
-    // rows of M complex points and, in the kernel-gradient pass, two columns of P points per LDS batch
-    if (M > (long long)kConvPPT * kConvRowThreads || 2 * P > kConvColPoints) return OK;
+    const long long P = conv_fused_len((long long)c.H + std::max(cy, c.KH - 1 - cy));
+    const long long M = conv_fused_len(((long long)c.W + std::max(cx, c.KW - 1 - cx) + 1) / 2), Qh = M + 1;
+    if (!P || !M) return OK;
+    std::vector<int> rc, rr;
+    int ntc = 0, ntr = 0;
+    if (!mix_factor((int)P, kConvThreads / 2, rc, ntc) || !mix_factor((int)M, kConvThreads / 2, rr, ntr)) return OK;
     c.P = P;
     c.Q = 2 * M;
     c.nspec = c.P * Qh;
-    c.row_count = std::min(64, pow2_floor_int((long long)kConvPPT * kConvRowThreads / M));
-    c.row_lc = ilog2_int(c.row_count);
-    c.col_count = std::min(64, pow2_floor_int(kConvColPoints / c.P));
-    c.col_lc = ilog2_int(c.col_count);
-    // the kernel-gradient pass transforms x and g columns together: 2 count P <= kConvColPoints
-    c.gk_count = std::min(32, pow2_floor_int(kConvColPoints / (2 * c.P)));
-    c.gk_lc = ilog2_int(c.gk_count);
-    const long long ngroups = (Qh + c.col_count - 1) / c.col_count;
-    // enough workgroups for four per CU of a 256-CU device, in chunks of images
-    c.nchunk = (int)std::max<long long>(1, std::min<long long>(c.B, (4 * 256 + ngroups - 1) / ngroups));
+    // Columns per block: a wavefront's worth of threads.  One column where it fills one leaves
+    // small workgroups, several to a CU (backward of 8 x 1024^2, 31 x 31: 0.304 ms with four columns,
+    // 0.257 ms with one); half-filled wavefronts cost more than that (21 x 439 x 1713, 13 x 9: 448
+    // points by 32 threads, forward 0.221 -> 0.255 ms).  The kernel gradient holds x and g columns.
+    const long long lds = 80 * 1024 - 1024;
+    while (c.lcb < 3 && (1 << c.lcb) * ntc < 64 && (2LL << c.lcb) * (P + 8) * 16 <= lds) ++c.lcb;
+    c.sub = std::max(1, (1 << c.lcb) / 2);
+    c.nblk = (int)((Qh + (1 << c.lcb) - 1) >> c.lcb);
+    // rows per workgroup: whole 128-byte lines of a block, a wavefront at least
+    while ((1 << (c.lcb + c.ltb)) * 16 < 128 || (1 << c.ltb) * ntr < 64) {
+        if ((2LL << c.ltb) * M * 16 > lds || (2 << c.ltb) * ntr > kConvThreads || (2 << c.ltb) > kConvMaxTb) break;
+        ++c.ltb;
+    }
+    // kernel gradient: chunks of images that make three rounds of two workgroups per CU, eight at
+    // most (the final pass sums them one after the other)
+    const long long ng = (long long)c.nblk * ((1 << c.lcb) / c.sub);
+    c.nchunk = (int)std::max<long long>(1, std::min<long long>(std::min(c.B, 8), (3 * 512 + ng - 1) / ng));
     c.chunk = (c.B + c.nchunk - 1) / c.nchunk;
     c.nchunk = (c.B + c.chunk - 1) / c.chunk;
-    std::vector<double2> h;
-    twiddle_table(h, (uint64_t)c.Q, (uint64_t)c.Q, 1);
-    if (c.tq.alloc(h.size() * sizeof(double2)) ||
-        hipMemcpy(c.tq.p, h.data(), h.size() * sizeof(double2), hipMemcpyHostToDevice) != hipSuccess) {
+    // tables
+    std::vector<double2> all, h;
+    size_t at[5];
+    std::vector<int> rci(rc.rbegin(), rc.rend());
+    auto add = [&](size_t k) { at[k] = all.size(); all.insert(all.end(), h.begin(), h.end()); };
+    mix_table(h, rc, -1); add(0);
+    mix_table(h, rci, 1); add(1);
+    mix_table(h, rr, -1); add(2);
+    mix_table(h, rr, 1); add(3);
+    twiddle_table(h, (uint64_t)c.Q, (uint64_t)(M / 2 + 1), 1); add(4);
+    if (c.tab.alloc(all.size() * sizeof(double2)) ||
+        hipMemcpy(c.tab.p, all.data(), all.size() * sizeof(double2), hipMemcpyHostToDevice) != hipSuccess) {
         (void)hipGetLastError();
         err = {E_NOMEM, "convolution table allocation failed"};
         return E_NOMEM;
     }
-    twiddle_table(h, (uint64_t)c.P, (uint64_t)c.P, 1);
-    if (c.tp.alloc(h.size() * sizeof(double2)) ||
-        hipMemcpy(c.tp.p, h.data(), h.size() * sizeof(double2), hipMemcpyHostToDevice) != hipSuccess) {
-        (void)hipGetLastError();
-        err = {E_NOMEM, "convolution table allocation failed"};
-        return E_NOMEM;
-    }
-    const size_t spec = (size_t)c.B * c.H * Qh * sizeof(double2);
-    if (c.sx.alloc(spec) || c.sg.alloc(spec) || c.sk.alloc((size_t)c.KH * Qh * sizeof(double2)) ||
-        c.kt.alloc((size_t)Qh * c.P * sizeof(double2)) ||
-        c.acc.alloc((size_t)c.nchunk * Qh * c.P * sizeof(double2))) {
+    const double2 *tab = (const double2 *)c.tab.p;
+    c.Ff = mix_shape((int)P, rc, ntc, tab + at[0]);
+    c.Fi = mix_shape((int)P, rci, ntc, tab + at[1]);
+    c.Rf = mix_shape((int)M, rr, ntr, tab + at[2]);
+    c.Ri = mix_shape((int)M, rr, ntr, tab + at[3]);
+    c.rtw = tab + at[4];
+    const size_t qp = (size_t)c.nblk << c.lcb;   // bins per row, whole blocks
+    const size_t spec = (size_t)c.B * c.H * qp * sizeof(double2);
+    if (c.sx.alloc(spec) || c.sg.alloc(spec) || c.sk.alloc((size_t)c.KH * qp * sizeof(double2)) ||
+        c.kt.alloc(qp * c.P * sizeof(double2)) || c.acc.alloc((size_t)c.nchunk * qp * c.P * sizeof(double2))) {
         err = {E_NOMEM, "convolution workspace allocation failed"};
         return E_NOMEM;
     }
     static std::once_flag attr_once;
     std::call_once(attr_once, [] {
-        for (const void *f : {(const void *)k_conv_cols<CC_SPECTRUM>, (const void *)k_conv_cols<CC_CONV>,
-                              (const void *)k_conv_cols<CC_GK>, (const void *)k_conv_cols<CC_GK_FINAL>})
-            if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 1024) != hipSuccess)
+        for (const void *f :
+             {(const void *)k_conv_cols<CC_SPECTRUM, 3>, (const void *)k_conv_cols<CC_SPECTRUM, 4>,
+              (const void *)k_conv_cols<CC_CONV, 3>, (const void *)k_conv_cols<CC_CONV, 4>,
+              (const void *)k_conv_cols<CC_GK, 3>, (const void *)k_conv_cols<CC_GK, 4>,
+              (const void *)k_conv_cols<CC_GK_FINAL, 3>, (const void *)k_conv_cols<CC_GK_FINAL, 4>,
+              (const void *)k_conv_rows<3>, (const void *)k_conv_rows<4>, (const void *)k_conv_rows_inv<3>,
+              (const void *)k_conv_rows_inv<4>})
+            if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 2048) != hipSuccess)
                 (void)hipGetLastError();
     });
     c.fused = true;
     return OK;
 }
 
-static size_t row_lds(const Conv2d &c) { return (size_t)lds_points_padded(c.row_count * (int)(c.Q / 2)) * sizeof(double2); }
-
-static hipError_t rows_fwd(const Conv2d &c, const void *src, bool f32, long long rows, int W, int rx, double2 *S,
-                           hipStream_t s)
+static ConvSpec conv_spec(const Conv2d &c, const DevBuf &b, int rows)
 {
-    ConvRows R{src, S, (const double2 *)c.tq.p, rows, W, (int)c.Q, rx, f32 ? 1 : 0, c.row_count, c.row_lc};
-    const long long groups = (rows + c.row_count - 1) / c.row_count;
-    const unsigned grid = (unsigned)std::max<long long>(1, std::min<long long>(groups, 65536));
-    hipLaunchKernelGGL(k_conv_rows<kConvRowThreads>, dim3(grid), dim3(kConvRowThreads), row_lds(c), s, R);
+    return ConvSpec{(double2 *)b.p, rows, c.nblk, c.lcb};
+}
+
+// bytes from the first image of a workgroup's rows to the end of its last one
+static long long conv_row_span(const Conv2d &c, const ConvSpec &S)
+{
+    const long long imgs = ((1 << c.ltb) + S.rows - 1) / S.rows + 1;
+    return imgs * (((long long)S.nblk * S.rows) << S.lcb) * 16;
+}
+
+static size_t row_lds(const Conv2d &c) { return ((size_t)(c.Q / 2) << c.ltb) * sizeof(double2); }
+
+// workgroups of up to 256 threads run faster with three waves per SIMD, larger ones with four (the
+// rule of the engine's mixed-radix passes): forward of 21 x 439 x 1713, 13 x 9: 0.260 ms with four,
+// 0.227 ms with three; of 16 x 2048^2, 63 x 63: 0.96 and 1.17 ms
+static bool conv_w3(unsigned block) { return block <= 256; }
+
+static ConvRowSet row_set(const Conv2d &c, const void *src, long long rows, int W, int rx, const ConvSpec &S)
+{
+    return ConvRowSet{src, S, rows, conv_row_span(c, S), W, rx, (unsigned)((rows + (1LL << c.ltb) - 1) >> c.ltb)};
+}
+
+static hipError_t rows_fwd(const Conv2d &c, std::initializer_list<ConvRowSet> sets, hipStream_t s)
+{
+    ConvRows R{};
+    unsigned grid = 0;
+    for (const ConvRowSet &a : sets) {
+        R.set[R.nset++] = a;
+        grid += a.groups;
+    }
+    R.F = c.Rf;
+    R.rtw = c.rtw;
+    R.f32 = c.dtype == 1;
+    R.ltb = c.ltb;
+    const unsigned block = (unsigned)c.Rf.NT << c.ltb;
+    if (conv_w3(block)) hipLaunchKernelGGL(k_conv_rows<3>, dim3(grid), dim3(block), row_lds(c), s, R);
+    else hipLaunchKernelGGL(k_conv_rows<4>, dim3(grid), dim3(block), row_lds(c), s, R);
     return hipGetLastError();
 }
 
-static hipError_t rows_inv(const Conv2d &c, const double2 *S, long long rows, void *dst, bool f32, int Wout, int ox,
-                           double scale, hipStream_t s)
+static ConvRowInvSet row_inv_set(const Conv2d &c, const ConvSpec &S, long long rows, void *dst, int Wout, int ox)
 {
-    ConvRowsInv R{S, dst, (const double2 *)c.tq.p, rows, Wout, (int)c.Q, ox, f32 ? 1 : 0, c.row_count, c.row_lc,
-                  scale};
-    const long long groups = (rows + c.row_count - 1) / c.row_count;
-    const unsigned grid = (unsigned)std::max<long long>(1, std::min<long long>(groups, 65536));
-    hipLaunchKernelGGL(k_conv_rows_inv<kConvRowThreads>, dim3(grid), dim3(kConvRowThreads), row_lds(c), s, R);
+    return ConvRowInvSet{S, dst, rows, conv_row_span(c, S), Wout, ox, (unsigned)((rows + (1LL << c.ltb) - 1) >> c.ltb)};
+}
+
+static hipError_t rows_inv(const Conv2d &c, std::initializer_list<ConvRowInvSet> sets, hipStream_t s)
+{
+    ConvRowsInv R{};
+    unsigned grid = 0;
+    for (const ConvRowInvSet &a : sets)
+        if (a.dst) {
+            R.set[R.nset++] = a;
+            grid += a.groups;
+        }
+    if (!grid) return hipSuccess;
+    R.F = c.Ri;
+    R.rtw = c.rtw;
+    R.f32 = c.dtype == 1;
+    R.ltb = c.ltb;
+    R.scale = 1.0 / ((double)c.P * c.Q);
+    const unsigned block = (unsigned)c.Ri.NT << c.ltb;
+    if (conv_w3(block)) hipLaunchKernelGGL(k_conv_rows_inv<3>, dim3(grid), dim3(block), row_lds(c), s, R);
+    else hipLaunchKernelGGL(k_conv_rows_inv<4>, dim3(grid), dim3(block), row_lds(c), s, R);
     return hipGetLastError();
 }
 
-static hipError_t cols(const Conv2d &c, int mode, ConvCols C, hipStream_t s)
+template <int MODE>
+static hipError_t cols(const Conv2d &c, ConvCols C, hipStream_t s)
 {
-    const bool gk = mode == CC_GK;
-    C.P = (int)c.P;
-    C.Qh = (int)(c.Q / 2 + 1);
-    C.count = gk ? c.gk_count : c.col_count;
-    C.lc = gk ? c.gk_lc : c.col_lc;
-    C.tp = (const double2 *)c.tp.p;
+    C.KT = (double2 *)c.kt.p;
+    C.acc = (double2 *)c.acc.p;
+    C.F = MODE == CC_GK_FINAL ? c.Fi : c.Ff;
+    C.I = c.Fi;
     C.nchunk = c.nchunk;
     C.chunk = c.chunk;
-    const int n = C.count * (int)c.P * (gk ? 2 : 1);   // points of one LDS batch
-    const unsigned ngroups = (unsigned)((C.Qh + C.count - 1) / C.count);
-    const bool chunked = mode == CC_CONV || gk;
-    const dim3 grid(chunked ? ngroups * (unsigned)c.nchunk : ngroups), block(kConvColThreads);
-    const size_t lds = (size_t)lds_points_padded(n) * sizeof(double2);
-    switch (mode) {
-        case CC_SPECTRUM: hipLaunchKernelGGL(k_conv_cols<CC_SPECTRUM>, grid, block, lds, s, C); break;
-        case CC_CONV: hipLaunchKernelGGL(k_conv_cols<CC_CONV>, grid, block, lds, s, C); break;
-        case CC_GK: hipLaunchKernelGGL(k_conv_cols<CC_GK>, grid, block, lds, s, C); break;
-        default: hipLaunchKernelGGL(k_conv_cols<CC_GK_FINAL>, grid, block, lds, s, C); break;
-    }
+    C.sub = c.sub;
+    const unsigned cb = 1u << c.lcb, nblk = (unsigned)c.nblk;
+    const unsigned ncol = MODE == CC_GK ? 2u * (unsigned)c.sub : cb;
+    const unsigned grid = MODE == CC_CONV ? nblk * (unsigned)C.nimg
+                          : MODE == CC_GK ? nblk * (cb / (unsigned)c.sub) * (unsigned)c.nchunk
+                                          : nblk;
+    const unsigned block = ncol * (unsigned)c.Ff.NT;
+    const size_t lds = (size_t)ncol * (size_t)(c.P + 8) * sizeof(double2);
+    if (conv_w3(block)) hipLaunchKernelGGL((k_conv_cols<MODE, 3>), dim3(grid), dim3(block), lds, s, C);
+    else hipLaunchKernelGGL((k_conv_cols<MODE, 4>), dim3(grid), dim3(block), lds, s, C);
     return hipGetLastError();
 }
 
@@ -585,39 +832,21 @@ static int kernel_spectrum(Conv2d &c, const void *k, hipStream_t s, Error &err)
     return plan_execute(*c.r2c_1, c.kpad.p, c.kspec.p, 1.0, s, err);
 }
 
-// fused path: K^ into kt ([Qh][P]) from the kernel's rows
-static hipError_t fused_kernel_spectrum(Conv2d &c, const void *k, hipStream_t s)
-{
-    hipError_t e = rows_fwd(c, k, c.dtype == 1, c.KH, c.KW, 0, (double2 *)c.sk.p, s);
-    if (e != hipSuccess) return e;
-    ConvCols C{};
-    C.Sa = (const double2 *)c.sk.p;
-    C.Ha = c.KH;
-    C.ra = 0;
-    C.Sout = (double2 *)c.kt.p;
-    return cols(c, CC_SPECTRUM, C, s);
-}
-
 // y = crop_c(c2r(K^ . r2c(pad_0 x))) / (P Q)
 static int fused_forward(Conv2d &c, const void *x, const void *k, void *y, hipStream_t s, Error &err)
 {
-    const bool f32 = c.dtype == 1;
     const int cy = (c.KH - 1) / 2, cx = (c.KW - 1) / 2;
-    IFFT_TRY_HIP(fused_kernel_spectrum(c, k, s));
-    IFFT_TRY_HIP(rows_fwd(c, x, f32, (long long)c.B * c.H, c.W, 0, (double2 *)c.sx.p, s));
-    ConvCols C{};
-    C.Sa = (const double2 *)c.sx.p;
-    C.Ha = c.H;
-    C.ra = 0;
-    C.Sout = (double2 *)c.sx.p;   // in place: a workgroup reads its columns before it writes them
+    const long long rows = (long long)c.B * c.H;
+    const ConvSpec S = conv_spec(c, c.sx, c.H), Sk = conv_spec(c, c.sk, c.KH);
+    IFFT_TRY_HIP(rows_fwd(c, {row_set(c, k, c.KH, c.KW, 0, Sk), row_set(c, x, rows, c.W, 0, S)}, s));
+    ConvCols K{}, C{};
+    K.Sa = Sk;
+    IFFT_TRY_HIP(cols<CC_SPECTRUM>(c, K, s));
+    C.Sa = C.So = S;   // in place: a workgroup reads its columns before it writes them
     C.oy = cy;
-    C.Ho = c.H;
-    C.KT = (const double2 *)c.kt.p;
     C.nimg = c.B;
-    C.conjk = 0;
-    IFFT_TRY_HIP(cols(c, CC_CONV, C, s));
-    IFFT_TRY_HIP(rows_inv(c, (const double2 *)c.sx.p, (long long)c.B * c.H, y, f32, c.W, cx,
-                          1.0 / ((double)c.P * c.Q), s));
+    IFFT_TRY_HIP(cols<CC_CONV>(c, C, s));
+    IFFT_TRY_HIP(rows_inv(c, {row_inv_set(c, S, rows, y, c.W, cx)}, s));
     return OK;
 }
 
@@ -626,46 +855,41 @@ static int fused_forward(Conv2d &c, const void *x, const void *k, void *y, hipSt
 static int fused_backward(Conv2d &c, const void *x, const void *k, const void *gy, void *gx, void *gk, hipStream_t s,
                           Error &err)
 {
-    const bool f32 = c.dtype == 1;
     const int cy = (c.KH - 1) / 2, cx = (c.KW - 1) / 2;
-    const double inv = 1.0 / ((double)c.P * c.Q);
-    if (gx) IFFT_TRY_HIP(fused_kernel_spectrum(c, k, s));   // K^ into kt before the kernel rows' workspace is reused
-    IFFT_TRY_HIP(rows_fwd(c, gy, f32, (long long)c.B * c.H, c.W, cx, (double2 *)c.sg.p, s));
+    const long long rows = (long long)c.B * c.H;
+    const ConvSpec Sx = conv_spec(c, c.sx, c.H), Sg = conv_spec(c, c.sg, c.H), Sk = conv_spec(c, c.sk, c.KH);
+    const ConvRowSet rg = row_set(c, gy, rows, c.W, cx, Sg), rk = row_set(c, k, c.KH, c.KW, 0, Sk),
+                     rx = row_set(c, x, rows, c.W, 0, Sx);
+    if (gx && gk) IFFT_TRY_HIP(rows_fwd(c, {rk, rg, rx}, s));
+    else if (gx) IFFT_TRY_HIP(rows_fwd(c, {rk, rg}, s));
+    else if (gk) IFFT_TRY_HIP(rows_fwd(c, {rg, rx}, s));
+    if (gx) {   // K^ before the kernel rows' workspace is reused
+        ConvCols K{};
+        K.Sa = Sk;
+        IFFT_TRY_HIP(cols<CC_SPECTRUM>(c, K, s));
+    }
     if (gk) {
         // sum_b conj(X^_b) G^_b per chunk of images, then the chunks' sum transformed back
-        IFFT_TRY_HIP(rows_fwd(c, x, f32, (long long)c.B * c.H, c.W, 0, (double2 *)c.sx.p, s));
         ConvCols C{};
-        C.Sa = (const double2 *)c.sx.p;
-        C.Sg = (const double2 *)c.sg.p;
-        C.Ha = c.H;
-        C.ra = 0;
+        C.Sa = Sx;
+        C.Sg = Sg;
         C.rg = cy;
-        C.acc = (double2 *)c.acc.p;
         C.nimg = c.B;
-        IFFT_TRY_HIP(cols(c, CC_GK, C, s));
+        IFFT_TRY_HIP(cols<CC_GK>(c, C, s));
         ConvCols F{};
-        F.acc = (double2 *)c.acc.p;
-        F.Sout = (double2 *)c.sk.p;
-        F.oy = 0;
-        F.Ho = c.KH;
-        IFFT_TRY_HIP(cols(c, CC_GK_FINAL, F, s));
-        IFFT_TRY_HIP(rows_inv(c, (const double2 *)c.sk.p, c.KH, gk, f32, c.KW, 0, inv, s));
+        F.Sa = F.So = Sk;
+        IFFT_TRY_HIP(cols<CC_GK_FINAL>(c, F, s));
     }
     if (gx) {
         // the convolution pass with conj(K^), G^'s rows at cy, result rows from 0, in place
         ConvCols C{};
-        C.Sa = (const double2 *)c.sg.p;
-        C.Ha = c.H;
+        C.Sa = C.So = Sg;
         C.ra = cy;
-        C.Sout = (double2 *)c.sg.p;
-        C.oy = 0;
-        C.Ho = c.H;
-        C.KT = (const double2 *)c.kt.p;
         C.nimg = c.B;
         C.conjk = 1;
-        IFFT_TRY_HIP(cols(c, CC_CONV, C, s));
-        IFFT_TRY_HIP(rows_inv(c, (const double2 *)c.sg.p, (long long)c.B * c.H, gx, f32, c.W, 0, inv, s));
+        IFFT_TRY_HIP(cols<CC_CONV>(c, C, s));
     }
+    IFFT_TRY_HIP(rows_inv(c, {row_inv_set(c, Sk, c.KH, gk, c.KW, 0), row_inv_set(c, Sg, rows, gx, c.W, 0)}, s));
     return OK;
 }
 

@@ -19,6 +19,7 @@
 #pragma once
 
 #include <type_traits>
+#include <utility>
 
 #include "butterflies.h"
 #include "fft_common.h"
@@ -107,6 +108,17 @@ template <int R> __device__ __forceinline__ void dftm(double2 *v, double s)
 
 constexpr int kMixMaxStages = 4;
 
+// f(std::integral_constant<int, 0>{}), ..., f(std::integral_constant<int, N - 1>{})
+template <int N, class F, int... I>
+__device__ __forceinline__ void each_of(F &&f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F> __device__ __forceinline__ void each(F &&f)
+{
+    each_of<N>(f, std::make_integer_sequence<int, N>{});
+}
+
 // butterflies of radix R a thread may own (16 points in registers at most)
 __host__ __device__ constexpr int mix_nb(int R) { return R > 8 ? 1 : 16 / R; }
 
@@ -156,24 +168,26 @@ struct MixLds {
 #pragma unroll
         for (int q = 0; q < R; ++q) v[q] = buf[b + q * nb];
     }
-    template <int R> __device__ __forceinline__ void store(const double2 *v, int j, int p) const
+    template <int R, class G> __device__ __forceinline__ void store(const double2 *v, int j, int p, G) const
     {
 #pragma unroll
         for (int q = 0; q < R; ++q) buf[j + q * p] = v[q];
     }
 };
 
-// One stage: `ld` delivers inputs b, b + nb, ..., `st` takes outputs j, j + p, ...
+// One stage: `ld` delivers inputs b, b + nb, ..., `st` takes outputs j, j + p, ... (and the number of
+// the butterfly within the thread).
 // SYNC separates the reads from the writes when both ends are the same LDS
 // rows.  lim is the number of butterflies this thread's transform runs (N / R,
-// or 0 for an idle slot).  Twiddle W_{pR}^{qk} sits at tw[(q - 1) p + k].
-template <int R, bool FIRST, bool SYNC, class LD, class ST>
+// or 0 for an idle slot).  Twiddle W_{pR}^{qk} sits at tw[(q - 1) p + k].  SG is
+// the sign of the transform where it is known at compile time, else 0 and in s.
+template <int R, bool FIRST, bool SYNC, int SG = 0, class LD, class ST>
 __device__ __forceinline__ void mix_stage(int nb, int lim, int p, int i, int NT, double s, const double2 *tw,
                                           const LD &ld, const ST &st)
 {
     constexpr int G = mix_nb(R);
     double2 v[G][R];
-    s = opaque(s);
+    s = SG ? (double)SG : opaque(s);
     i = opaque(i);
 #pragma unroll
     for (int g = 0; g < G; ++g) {
@@ -183,8 +197,8 @@ __device__ __forceinline__ void mix_stage(int nb, int lim, int p, int i, int NT,
     if constexpr (SYNC) __syncthreads();
     const float rp = FIRST ? 1.0f : __builtin_amdgcn_rcpf((float)p);
     const __amdgpu_buffer_rsrc_t rtw = make_rsrc(tw, FIRST ? 0 : (long long)(R - 1) * p * 16);
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
+    each<G>([&](auto gc) __attribute__((always_inline)) {
+        constexpr int g = decltype(gc)::value;
         const int b = i + g * NT;
         if (b < lim) {
             const int k = FIRST ? 0 : mod_small(b, p, rp);
@@ -193,9 +207,9 @@ __device__ __forceinline__ void mix_stage(int nb, int lim, int p, int i, int NT,
                 for (int q = 1; q < R; ++q) v[g][q] = cmul(v[g][q], bload2(rtw, (k + (q - 1) * p) * 16));
             }
             dftm<R>(v[g], s);
-            st.template store<R>(v[g], (b - k) * R + k, p);
+            st.template store<R>(v[g], (b - k) * R + k, p, gc);
         }
-    }
+    });
 }
 
 // Radices of a length and its stage-ordered twiddle table, as kernels take them
@@ -212,7 +226,7 @@ struct MixShape {
 // and store side, which may differ when lanes walk another way there.
 // LD_LDS: the inputs already sit in the LDS rows (behind a barrier).  ST_LDS: the
 // outputs stay in LDS rows, natural order; a barrier follows.
-template <bool LD_LDS, bool ST_LDS, class LD, class ST>
+template <bool LD_LDS, bool ST_LDS, int SG = 0, class LD, class ST>
 __device__ __forceinline__ void mix_fft(const MixShape &S, double2 *buf, int i, bool on_in, double2 *obuf, int o,
                                         bool on_out, double s, const LD &ld, const ST &st)
 {
@@ -220,8 +234,8 @@ __device__ __forceinline__ void mix_fft(const MixShape &S, double2 *buf, int i, 
     unsigned codes = S.codes;
     mix_radix((int)(codes & 15u) + 1, [&](auto rc) __attribute__((always_inline)) {
         constexpr int R = decltype(rc)::value;
-        const int nb = N / R;
-        mix_stage<R, true, LD_LDS>(nb, on_in ? nb : 0, 1, i, NT, s, nullptr, ld, MixLds{buf});
+        const int nb = opaque_scalar(N) / R;
+        mix_stage<R, true, LD_LDS, SG>(nb, on_in ? nb : 0, 1, i, NT, s, nullptr, ld, MixLds{buf});
     });
     __syncthreads();
     int p = (int)(codes & 15u) + 1;
@@ -233,7 +247,7 @@ __device__ __forceinline__ void mix_fft(const MixShape &S, double2 *buf, int i, 
         mix_radix(r, [&](auto rc) __attribute__((always_inline)) {
             constexpr int R = decltype(rc)::value;
             const int nb = opaque_scalar(N) / R;
-            mix_stage<R, false, true>(nb, nb, p, i, NT, s, tw, MixLds{buf}, MixLds{buf});
+            mix_stage<R, false, true, SG>(nb, nb, p, i, NT, s, tw, MixLds{buf}, MixLds{buf});
         });
         __syncthreads();
         tw += (r - 1) * p;
@@ -244,9 +258,77 @@ __device__ __forceinline__ void mix_fft(const MixShape &S, double2 *buf, int i, 
         mix_radix((int)(codes & 15u) + 1, [&](auto rc) __attribute__((always_inline)) {
             constexpr int R = decltype(rc)::value;
             const int nb = N / R;
-            mix_stage<R, false, false>(nb, on_out ? nb : 0, p, o, NT, s, tw, MixLds{obuf}, st);
+            mix_stage<R, false, false, SG>(nb, on_out ? nb : 0, p, o, NT, s, tw, MixLds{obuf}, st);
         });
     }
+}
+
+// The turn of mix_conv: the forward outputs of a butterfly times `mul`'s values, and the first
+// inverse stage (outputs b R + q) into the LDS row.
+template <class MUL>
+struct MixTurn {
+    const MixLds &row;
+    const MUL &mul;
+    template <int R, class G> __device__ __forceinline__ void store(double2 *v, int b, int nb, G g) const
+    {
+        mul.template apply<R>(v, b, nb);
+        dftm<R>(v, 1.0);
+        row.template store<R>(v, b * R, 1, g);
+    }
+};
+
+// Forward transform, pointwise product and inverse transform of one LDS row.  The inverse takes the
+// forward radices in reverse, so its first stage has its inputs b + q N/R where the forward's last
+// stage leaves its outputs: that radix is transformed, multiplied (mul) and transformed back in
+// registers, and the spectrum never passes through LDS.  F: forward shape (sign -1 table), I: the
+// reversed one (sign +1 table), of the same threads.
+template <class LD, class MUL, class ST>
+__device__ __forceinline__ void mix_conv(const MixShape &F, const MixShape &I, double2 *buf, int i, const LD &ld,
+                                         const MUL &mul, const ST &st)
+{
+    const int N = F.N, NT = F.NT;
+    const MixLds row{buf};
+    unsigned codes = F.codes;
+    mix_radix((int)(codes & 15u) + 1, [&](auto rc) __attribute__((always_inline)) {
+        constexpr int R = decltype(rc)::value;
+        const int nb = N / R;
+        mix_stage<R, true, false, -1>(nb, nb, 1, i, NT, -1.0, nullptr, ld, row);
+    });
+    __syncthreads();
+    int p = (int)(codes & 15u) + 1;
+    const double2 *tw = F.tw;
+    auto middle = [&](auto sg) __attribute__((always_inline)) {
+        constexpr int SG = decltype(sg)::value;
+        for (int k = 1; k < F.nst - 1; ++k) {
+            codes >>= 4;
+            const int r = (int)(codes & 15u) + 1;
+            mix_radix(r, [&](auto rc) __attribute__((always_inline)) {
+                constexpr int R = decltype(rc)::value;
+                const int nb = opaque_scalar(N) / R;
+                mix_stage<R, false, true, SG>(nb, nb, p, i, NT, (double)SG, tw, row, row);
+            });
+            __syncthreads();
+            tw += (r - 1) * p;
+            p *= r;
+        }
+        codes >>= 4;
+    };
+    middle(std::integral_constant<int, -1>{});
+    mix_radix((int)(codes & 15u) + 1, [&](auto rc) __attribute__((always_inline)) {
+        constexpr int R = decltype(rc)::value;
+        const int nb = N / R;
+        mix_stage<R, false, true, -1>(nb, nb, nb, i, NT, -1.0, tw, row, MixTurn<MUL>{row, mul});
+    });
+    __syncthreads();
+    codes = I.codes;
+    p = (int)(codes & 15u) + 1;
+    tw = I.tw;
+    middle(std::integral_constant<int, 1>{});
+    mix_radix((int)(codes & 15u) + 1, [&](auto rc) __attribute__((always_inline)) {
+        constexpr int R = decltype(rc)::value;
+        const int nb = N / R;
+        mix_stage<R, false, false, 1>(nb, nb, p, i, NT, 1.0, tw, row, st);
+    });
 }
 
 }  // namespace ifft

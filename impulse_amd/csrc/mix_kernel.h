@@ -192,7 +192,7 @@ struct MixOut {
         else bstore2(r, o, z);
     }
 
-    template <int R> __device__ __forceinline__ void store(const double2 *v, int n, int dn) const
+    template <int R, class G> __device__ __forceinline__ void store(const double2 *v, int n, int dn, G) const
     {
         const int pos = p0 + n * dp, dpos = dn * dp;
         if constexpr (SM == ST_C2C) {

@@ -71,7 +71,7 @@ static int dft_ops(int R)
 // accesses of each stage with the bank conflicts of the first stage's writes (their stride is the
 // radix: 16-byte words fall on 8 bank groups, so an odd first radix has none), and the
 // per-stage overhead of every thread.
-bool mix_factor(int N, int max_threads, std::vector<int> &radices, int &threads)
+bool mix_factor(int N, int max_threads, std::vector<int> &radices, int &threads, double *cost_out)
 {
     if (N < 4) return false;
     double best = -1.0;
@@ -106,6 +106,7 @@ bool mix_factor(int N, int max_threads, std::vector<int> &radices, int &threads)
             }
     };
     rec(rec, N);
+    if (cost_out) *cost_out = best;
     return best >= 0.0;
 }
 
