@@ -190,6 +190,7 @@ size_t mfma_workspace_bytes(const Mfma &m);
 void mfma_destroy(Mfma *m);
 
 // mixed-radix shapes (twiddle.hip)
+int mix_ops(int R);   // VALU operations of one radix-R butterfly
 bool mix_factor(int N, int max_threads, std::vector<int> &radices, int &threads, double *cost = nullptr);
 void mix_table(std::vector<double2> &out, const std::vector<int> &radices, int sign);
 

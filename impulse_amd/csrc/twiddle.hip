@@ -60,7 +60,7 @@ void twiddle_table(std::vector<double2> &out, uint64_t n, uint64_t count, uint64
 // ---------------------------------------------------------------------------
 
 // VALU operations of one radix-R butterfly, counted from the code
-static int dft_ops(int R)
+int mix_ops(int R)
 {
     static const int ops[17] = {0, 0, 4, 16, 16, 40, 44, 72, 60, 120, 100, 160, 112, 216, 172, 200, 170};
     return ops[R];
@@ -85,7 +85,7 @@ bool mix_factor(int N, int max_threads, std::vector<int> &radices, int &threads,
             double cost = 0.0;
             for (size_t k = 0; k < cur.size(); ++k) {
                 const int R = cur[k];
-                cost += (double)(N / R) * (dft_ops(R) + (k ? 4 * (R - 1) : 0) + 10 * R) + 60.0 * nt;
+                cost += (double)(N / R) * (mix_ops(R) + (k ? 4 * (R - 1) : 0) + 10 * R) + 60.0 * nt;
             }
             int g = cur[0];
             g = (g & 1) ? 1 : (g & 2) ? 2 : (g & 4) ? 4 : 8;   // gcd with the 8 bank groups
