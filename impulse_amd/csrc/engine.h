@@ -88,11 +88,7 @@ struct Pass {
     size_t bytes_in = 0, bytes_out = 0;   // bytes the launch must move at least once
     const char *name = "";
     std::string kname;                    // kernel instantiation of the last execute, as rocprof names it
-    // even-length real input at unit stride read as complex pairs (used when the
-    // source pointer is 16-byte aligned at execute time)
-    bool has_alt = false;
-    FftParams fp_alt{};
-    // FFT_MIX: the half-length real side moves as complex words when its pointer is aligned to them
+    // a half-length real side moves as complex words when its pointer is aligned to them
     bool in_words = false, out_words = false;
 };
 

@@ -65,8 +65,8 @@ template <int N, int MAP> constexpr int pow2_ld() { return N + N / 16 + (MAP == 
 // products of those, and each twiddle is used as soon as it is formed so that
 // at most five are live at a time.
 // IO_BLUE_IN / IO_BLUE_OUT: the Bluestein column passes with direct buffer
-// accesses -- chirp-in loads (complex or odd real pairs) with a twiddled store,
-// and plain loads with a chirp-out complex store (rows and columns mappings)
+// accesses -- chirp-in loads (complex, odd real pairs or odd c2r pairs) with a twiddled store,
+// and plain loads with a chirp-out complex or odd-pair store (rows and columns mappings)
 // IO_W4 (added to IO_CONV or a Bluestein mode) selects the instance held to four waves per
 // SIMD, for grids of a few rounds.  IO_S32 / IO_D32 (added to IO_PLAIN, or IO_S32 to
 // IO_TWIDDLE) select the instances whose source / destination array holds complex float: widened
@@ -75,8 +75,12 @@ template <int N, int MAP> constexpr int pow2_ld() { return N + N / 16 + (MAP == 
 // passes 1-2 %).
 // IO_R2C_HALF: a whole even-length r2c signal per transform (its half-length complex sequence,
 // per-point loads), the real post-process fused into the store.
+// IO_C2R (added to IO_TWIDDLE): the first pass of an even-length four-step c2r, whose loads take the
+// bin pair X[p], X[M - p] through buffers.  Per-point loads (a mode switch, 64-bit indices) took 0.517
+// ms for c2r 2^22 x16; these take 0.35 ms, with the mirror bins' lines shared in the L2 (1.6 GB
+// requested, 1.07 GB from memory).  Its second pass stores complex words: 0.408 -> 0.266 ms.
 enum Pow2Io { IO_GENERIC = 0, IO_PLAIN = 1, IO_TWIDDLE = 2, IO_R2C_ROWPAIR = 3, IO_CONV = 4, IO_BLUE_IN = 5,
-              IO_BLUE_OUT = 6, IO_R2C_HALF = 7, IO_W4 = 8, IO_S32 = 16, IO_D32 = 32 };
+              IO_BLUE_OUT = 6, IO_R2C_HALF = 7, IO_W4 = 8, IO_S32 = 16, IO_D32 = 32, IO_C2R = 64 };
 
 // Row assignment of the fused real post-process (ST_R2C_ROWPAIR, rows of L1 = N
 // points, L2 rows per signal, Z[j + L2 n] in row j).  Z[M - k] for k = j + L2 n
@@ -217,7 +221,7 @@ template <int N, int MAP, int IOW>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(pow2_wpe<MAP, IOW>()))) k_fft_pow2(const FftParams P)
 {
     constexpr int IO = IOW & (IO_W4 - 1);
-    constexpr bool S32 = IOW & IO_S32, D32 = IOW & IO_D32;
+    constexpr bool S32 = IOW & IO_S32, D32 = IOW & IO_D32, C2R = IOW & IO_C2R;
     extern __shared__ double lds[];
     __shared__ TfInfo info[MAP == MAP_ROWCOL ? kMaxTB : 1];
     constexpr bool COL = MAP == MAP_COL;
@@ -236,6 +240,12 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(pow2_w
         RG = rowpair_group(xcd_block(blockIdx.x, gridDim.x), TB, P.ni);
         const long long g = rowpair_transform(RG, t, TB, P.ni);
         gidx = g < 0 ? P.ntf : g;
+    } else if constexpr (C2R) {
+        // Column groups g and G - 1 - g of a signal in turn: each reads the lines the other reads as
+        // mirror bins, and neighbouring workgroups run on one XCD at about the same time.
+        const unsigned blk = xcd_block(blockIdx.x, gridDim.x), G = (unsigned)P.ni / TB;
+        const unsigned u = blk / G, k = blk - u * G;
+        gidx = (long long)(u * G + ((k & 1) ? G - 1 - (k >> 1) : k >> 1)) * TB + t;
     } else {
         gidx = (long long)xcd_block(blockIdx.x, gridDim.x) * TB + t;
     }
@@ -263,6 +273,37 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(pow2_w
         const int ilim = (int)P.ilim;
         const double cj = P.conj_in ? -1.0 : 1.0;
         const bool hasb = T.flags & 2;
+        if (P.load_mode == LD_C2R_PAIR) {
+            // the odd c2r pair A + i B, Hermitian-extended past L/2; Im of bin 0 is ignored
+            const int L = P.M;
+            const double fw = P.fwd_flag ? -1.0 : 1.0;
+            auto ld = [&](int off) -> double2 {
+                if constexpr (S32) {
+                    const float2 f = bloadf2(rin, off);
+                    return make_double2((double)f.x, (double)f.y);
+                } else {
+                    return bload2(rin, off);
+                }
+            };
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const int pos = (int)T.ip0 + (i + q * (N / 16)) * (int)P.in.pst;
+                const bool ok = valid && pos < ilim;
+                const int pc = ok ? pos : 0;
+                const bool mirror = 2 * pc > L;
+                const int k = mirror ? L - pc : pc;
+                double2 a = ld(ba + k * estep), c = ld(bb + k * estep);
+                const double sg = pc == 0 ? 0.0 : (mirror ? -fw : fw);
+                a.y = pc == 0 ? 0.0 : a.y * sg;
+                c.y = pc == 0 ? 0.0 : c.y * sg;
+                if (!hasb) c = make_double2(0.0, 0.0);
+                double2 z = make_double2(a.x - c.y, a.y + c.x);
+                if (P.adj_w && pc != 0) z = cscale(z, 0.5);
+                z.y *= cj;
+                const double2 w = bload2(rch, pc * 16);
+                v[q] = ok ? cmul(z, w) : make_double2(0.0, 0.0);
+            }
+        } else {
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
             const int pos = (int)T.ip0 + (i + q * (N / 16)) * (int)P.in.pst;
@@ -287,6 +328,46 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(pow2_w
             const double2 w = bload2(rch, pc * 16);
             v[q] = ok ? cmul(z, w) : make_double2(0.0, 0.0);
         }
+        }
+    } else if constexpr (C2R) {
+        // z[p] = (X[p] + X*[M-p]) + i (X[p] - X*[M-p]) W_{2M}^{-p} at p = j + L1 (i + q N/16).  The
+        // step between a thread's points is a multiple of the low table's length (pow2_c2r_in), so
+        // they share its entry.  Im of bins 0 and M is ignored.  Idle slots read the first signal.
+        const __amdgpu_buffer_rsrc_t rin = make_rsrc((const char *)P.src + P.src_lo, P.src_span);
+        constexpr int es = S32 ? 8 : 16;
+        const int estep = (int)P.in.sax * es, ba = (int)(T.ia * es - P.src_lo), M = P.M;
+        const int p0 = (int)T.ip0 + i * (int)P.in.pst, dp = (N / 16) * (int)P.in.pst;
+        const long long rS = 1LL << P.rtw_logS;
+        const __amdgpu_buffer_rsrc_t rhi = make_rsrc(P.rtw_hi, (2LL * M / rS + 2) * 16);
+        const double2 wlo = bload2(make_rsrc(P.rtw_lo, rS * 16), (int)(p0 & (rS - 1)) * 16);
+        const int hi0 = (p0 >> P.rtw_logS) * 16, dhi = (dp >> P.rtw_logS) * 16;
+        const double cj = P.fwd_flag ? -1.0 : 1.0;
+        auto ld = [&](int off) -> double2 {
+            if constexpr (S32) {
+                const float2 f = bloadf2(rin, off);
+                return make_double2((double)f.x, (double)f.y);
+            } else {
+                return bload2(rin, off);
+            }
+        };
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int p = p0 + q * dp;
+            double2 x = ld(ba + p * estep), m = ld(ba + (M - p) * estep);
+            x.y *= cj;
+            m.y *= cj;
+            if (q == 0) {   // bin 0 keeps weight 1 in the adjoint, which halves all others below
+                const double d = P.adj_w ? 2.0 : 1.0;
+                x = make_double2(p ? x.x : d * x.x, p ? x.y : 0.0);
+                m = make_double2(p ? m.x : d * m.x, p ? m.y : 0.0);
+            }
+            const double2 e = cadd(x, cconj(m));
+            const double2 o = cmul(csub(x, cconj(m)), cconj(cmul(wlo, bload2(rhi, hi0 + q * dhi))));
+            v[q] = make_double2(e.x - o.y, e.y + o.x);
+        }
+        if (P.adj_w)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) v[q] = cscale(v[q], 0.5);
     } else if constexpr (FAST) {
         // The r2c row-pair pass reads whole rows that no other workgroup touches: its loads are
         // non-temporal, which keeps the L2 for merging its short strided stores (pass time
@@ -485,6 +566,19 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(pow2_w
                 const long long tS = 1LL << P.tw_logS;
                 const __amdgpu_buffer_rsrc_t rlo = make_rsrc(P.tw_lo, tS * 16);
                 const __amdgpu_buffer_rsrc_t rhi = make_rsrc(P.tw_hi, (P.tw_L / tS + 2) * 16);
+                // c2r passes read both levels for every point, one product from exact (they did when
+                // their loads were per point; products of powers put 4 % on the transform's error)
+                if (C2R || (IO == IO_BLUE_IN && P.load_mode == LD_C2R_PAIR)) {
+#pragma unroll
+                    for (int c = 0; c < NB; ++c)
+#pragma unroll
+                        for (int q = 0; q < RL; ++q) {
+                            const int n = i + c * NT + q * (N / RL);
+                            const double2 w = twolevel_b(rlo, rhi, P.tw_logS, T.j * (long long)n);
+                            put(obase + n * ostep, cmul(v[c * RL + q], tw_sign(w, so)));
+                        }
+                    return;
+                }
                 const double2 step1 = twolevel_b(rlo, rhi, P.tw_logS, T.j * (long long)(N / RL));
                 double2 pw[4];
                 pw[0] = step1;
@@ -511,6 +605,15 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(pow2_w
                 const __amdgpu_buffer_rsrc_t rch = make_rsrc(P.chirp, P.olim * 16);
                 const int olim = (int)P.olim, op0 = (int)T.op0, opst = (int)P.out.pst;
                 const double cj = P.conj_out ? -1.0 : 1.0;
+                const bool pairs = P.store_mode == ST_C2R_PAIR;   // Re z to real row a, Im z to row b
+                constexpr int res = D32 ? 4 : 8;
+                const int ra = (int)(T.oa * res - P.dst_lo), rb = (int)(T.ob * res - P.dst_lo);
+                const int rstep = (int)P.out.sax * res;
+                const bool hasb = T.flags & 4;
+                auto putr = [&](int off, double x) {
+                    if constexpr (D32) bstoref1(rout, off, x);
+                    else bstore1(rout, off, x);
+                };
 #pragma unroll
                 for (int c = 0; c < NB; ++c) {
                     const int b = i + c * NT;
@@ -521,7 +624,15 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(pow2_w
                         const double2 w = bload2(rch, (pos < olim ? pos : 0) * 16);
                         double2 z = cmul(v[c * RL + q], w);
                         z.y *= cj;
-                        if (pos < olim) put(obase + n * ostep, cscale(z, P.fct));
+                        if (pos < olim) {
+                            z = cscale(z, P.fct);
+                            if (!pairs) {
+                                put(obase + n * ostep, z);
+                            } else {
+                                putr(ra + pos * rstep, z.x);
+                                if (hasb) putr(rb + pos * rstep, z.y);
+                            }
+                        }
                     }
                 }
             } else {
@@ -727,6 +838,21 @@ static hipError_t launch_conv(const FftParams &P, unsigned grid, unsigned block,
     return hipGetLastError();
 }
 
+// the first pass of a four-step c2r, on the column mapping
+template <int N, int IOW>
+static hipError_t launch_c2r(const FftParams &P, unsigned grid, unsigned block, size_t lds, hipStream_t s)
+{
+    static bool attr_done = false;
+    if (!attr_done) {
+        if (hipFuncSetAttribute((const void *)k_fft_pow2<N, MAP_COL, IOW>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 8192) != hipSuccess)
+            (void)hipGetLastError();
+        attr_done = true;
+    }
+    hipLaunchKernelGGL((k_fft_pow2<N, MAP_COL, IOW>), dim3(grid), dim3(block), lds, s, P);
+    return hipGetLastError();
+}
+
 template <int N>
 static hipError_t launch_n(const FftParams &P, int map, int io, unsigned grid, unsigned block, size_t lds,
                            hipStream_t s)
@@ -737,6 +863,9 @@ static hipError_t launch_n(const FftParams &P, int map, int io, unsigned grid, u
         return (io & IO_W4) ? launch_conv<N, IO_CONV | IO_W4>(P, grid, block, lds, s)
                             : launch_conv<N, IO_CONV>(P, grid, block, lds, s);
     }
+    if (io & IO_C2R)
+        return (io & IO_S32) ? launch_c2r<N, IO_TWIDDLE | IO_C2R | IO_S32>(P, grid, block, lds, s)
+                             : launch_c2r<N, IO_TWIDDLE | IO_C2R>(P, grid, block, lds, s);
     switch (io) {
         case IO_PLAIN: return launch_io<N, IO_PLAIN>(P, map, grid, block, lds, s);
         case IO_TWIDDLE: return launch_io<N, IO_TWIDDLE>(P, map, grid, block, lds, s);
@@ -795,20 +924,31 @@ static bool blue_windows(const FftParams &P)
            P.in.ipos >= 0 && P.in.pst > 0 && P.out.ipos >= 0 && P.out.pst > 0;
 }
 
-// chirp-in loads (complex or odd real pairs) with the plain four-step twiddle store
+// chirp-in loads (complex, odd real pairs or odd c2r pairs) with the plain four-step twiddle store
 static bool pow2_blue_in(const FftParams &P)
 {
     const long long omax = (P.ni - 1) * P.out.ipos + (long long)(P.N - 1) * P.out.pst;
-    return blue_windows(P) && !P.dst32 && P.chirp_in && (P.load_mode == LD_C2C || P.load_mode == LD_R2C_PAIR) &&
+    return blue_windows(P) && !P.dst32 && P.chirp_in && (P.load_mode == LD_C2C || P.load_mode == LD_R2C_PAIR || P.load_mode == LD_C2R_PAIR) &&
            P.ilim <= 0x7fffffffLL / 16 && P.store_mode == ST_TWIDDLE && P.tw_mul == 1 && !P.chirp_out &&
            !P.conj_out && omax < P.olim;
 }
 
-// plain loads with the chirp-out complex store
+// the first pass of an even-length four-step c2r: columns j of L1 = ni, positions j + L1 n of M = N L1
+static bool pow2_c2r_in(const FftParams &P, int tb)
+{
+    const long long omax = (P.ni - 1) * P.out.ipos + (long long)(P.N - 1) * P.out.pst;
+    const long long win = 0x7fffffffLL;
+    return P.load_mode == LD_C2R_HALF && P.store_mode == ST_TWIDDLE && P.tw_mul == 1 && !P.dst32 && !P.chirp_in &&
+           !P.conj_in && !P.chirp_out && !P.conj_out && P.rtw_lo && P.ni % tb == 0 && P.in.ipos == 1 &&
+           P.in.pst == P.ni && (long long)P.M == P.ni * P.N && P.M < P.ilim && omax < P.olim && P.src_span > 0 &&
+           P.src_span <= win && P.dst_span > 0 && P.dst_span <= win && (P.N / 16) * P.in.pst % (1LL << P.rtw_logS) == 0;
+}
+
+// plain loads with the chirp-out complex or odd-real-pair store
 static bool pow2_blue_out(const FftParams &P)
 {
     return blue_windows(P) && pow2_fast_load(P) && P.chirp_out && P.olim <= 0x7fffffffLL / 16 &&
-           P.store_mode == ST_C2C;
+           (P.store_mode == ST_C2C || P.store_mode == ST_C2R_PAIR);
 }
 
 // compute units of the current device (read once per device)
@@ -856,6 +996,7 @@ int pow2_io(const FftParams &P, int map, unsigned grid, unsigned block, size_t l
         // the twiddled store writes a workspace: no complex float instance for it
         return (io & IO_D32) && (io & (IO_W4 - 1)) == IO_TWIDDLE ? IO_GENERIC : io;
     }
+    else if (map == MAP_COL && pow2_c2r_in(P, pow2_tb(P.N, MAP_COL))) return IO_TWIDDLE | IO_C2R | (P.src32 ? IO_S32 : 0);
     else if (map != MAP_ROWCOL && pow2_blue_in(P)) io = IO_BLUE_IN | (P.src32 ? IO_S32 : 0);
     else if (map != MAP_ROWCOL && pow2_blue_out(P)) io = IO_BLUE_OUT | (P.dst32 ? IO_D32 : 0);
     else return IO_GENERIC;

@@ -381,18 +381,13 @@ struct Builder {
         return true;
     }
 
-    // LD_REAL_HALF with unit position stride reads x[2 pos], x[2 pos + 1]: the
-    // same bytes as one complex word, so the pass can run as a plain complex
-    // load when all batch strides are even and the pointer is 16-byte aligned
+    // A half-length real side with unit position stride moves x[2 pos], x[2 pos + 1]: the same bytes
+    // as one complex word, so the pass runs as a plain complex load or store when all batch strides
+    // are even and the pointer is aligned to complex words at execute time.
     static void make_alt(Pass &ps)
     {
-        const FftParams &P = ps.fp;
-        if (P.load_mode != LD_REAL_HALF || !even_side(P.in)) return;
-        ps.fp_alt = P;
-        ps.fp_alt.load_mode = LD_C2C;
-        for (int d = 0; d < P.in.nbd; ++d) ps.fp_alt.in.str[d] /= 2;
-        ps.fp_alt.in.isig /= 2;
-        ps.has_alt = true;
+        ps.in_words = ps.fp.load_mode == LD_REAL_HALF && even_side(ps.fp.in);
+        ps.out_words = ps.fp.store_mode == ST_C2R_HALF && even_side(ps.fp.out);
     }
 
     // bytes of the array behind `r` that a pass may address (the workspace of a linear side: its
@@ -483,8 +478,7 @@ struct Builder {
         ps.name = "k_fft_mix";
         ps.bytes_in = side_bytes(P, true);
         ps.bytes_out = side_bytes(P, false);
-        ps.in_words = P.load_mode == LD_REAL_HALF && even_side(P.in);
-        ps.out_words = P.store_mode == ST_C2R_HALF && even_side(P.out);
+        make_alt(ps);
         plan.passes.push_back(ps);
         return 1;
     }
@@ -1375,6 +1369,21 @@ int plan_execute_noalloc(Plan &P, const void *in, void *out, double fct, hipStre
     return plan_execute_ws(P, in, out, fct, stream, W, err);
 }
 
+// real sides that move as complex words (in_words, out_words) as complex sides
+static void as_words(FftParams &P)
+{
+    if (P.in_words) {
+        P.load_mode = LD_C2C;
+        for (int d = 0; d < P.in.nbd; ++d) P.in.str[d] /= 2;
+        P.in.isig /= 2;
+    }
+    if (P.out_words) {
+        P.store_mode = ST_C2C;
+        for (int d = 0; d < P.out.nbd; ++d) P.out.str[d] /= 2;
+        P.out.isig /= 2;
+    }
+}
+
 static int plan_execute_ws(Plan &P, const void *in, void *out, double fct, hipStream_t stream, const Workspace &W,
                            Error &err)
 {
@@ -1438,16 +1447,16 @@ static int plan_execute_ws(Plan &P, const void *in, void *out, double fct, hipSt
         hipError_t e;
         if (prof) (void)hipEventRecord(ev[2 * pi], stream);
         if (ps.kind == Pass::FFT_LDS || ps.kind == Pass::FFT_POW2 || ps.kind == Pass::FFT_MIX) {
-            const void *srcp = resolve(ps.src);
-            FftParams fp = (ps.has_alt && ((uintptr_t)srcp % (ps.fp_alt.src32 ? 8 : 16)) == 0) ? ps.fp_alt : ps.fp;
-            fp.src = srcp;
+            FftParams fp = ps.fp;
+            fp.src = resolve(ps.src);
             fp.dst = resolve(ps.dst);
+            fp.in_words = ps.in_words && (uintptr_t)fp.src % (fp.src32 ? 8 : 16) == 0;
+            fp.out_words = ps.out_words && (uintptr_t)fp.dst % (fp.dst32 ? 8 : 16) == 0;
+            if (ps.kind == Pass::FFT_POW2) as_words(fp);
             window(ps.src, fp.src_lo, fp.src_span);
             window(ps.dst, fp.dst_lo, fp.dst_span);
             fp.fct = ps.uses_fct ? fct : 1.0;
             if (ps.kind == Pass::FFT_MIX) {
-                fp.in_words = ps.in_words && (uintptr_t)srcp % (fp.src32 ? 8 : 16) == 0;
-                fp.out_words = ps.out_words && (uintptr_t)fp.dst % (fp.dst32 ? 8 : 16) == 0;
                 e = launch_fft_mix(fp, ps.grid, ps.block, ps.lds, stream);
                 ps.kname = "k_fft_mix<" + std::to_string(fp.load_mode) + ", " + std::to_string(fp.store_mode) + ", " +
                            std::to_string(mix_wpe(ps.grid, ps.block)) + ">";
