@@ -249,7 +249,7 @@ __global__ void __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_
     in.f32 = P.f32;
     in.pairs = !(A.rx & 1) && !(A.W & 1) && (uintptr_t)A.src % (2 * es) == 0;
     double2 *row = zl + t * M;
-    mix_fft<false, true, -1>(P.F, row, i, true, row, i, true, -1.0, in, MixLds{row});   // ends with a barrier
+    mix_fft<false, true, -1>(P.F, MixLds{row}, i, true, MixLds{row}, i, true, -1.0, in, MixLds{row});   // ends with a barrier
     // X[k] = E + W_{2M}^k O and X[M-k] = conj(E) - conj(W^k O), E = (Z[k] + conj Z[M-k]) / 2,
     // O = (Z[k] - conj Z[M-k]) / 2i.  Lanes walk a block's columns, then the rows; four bin pairs
     // in flight per thread.
@@ -367,7 +367,7 @@ __global__ void __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_
     out.ox = A.ox;
     out.f32 = P.f32;
     out.f = P.scale;
-    mix_fft<true, false, 1>(P.F, row, i, true, row, i, true, 1.0, MixLds{row}, out);
+    mix_fft<true, false, 1>(P.F, MixLds{row}, i, true, MixLds{row}, i, true, 1.0, MixLds{row}, out);
 }
 
 // column `t` of a block: rows [r0, r0 + rows) of the grid, zeros elsewhere
@@ -464,7 +464,7 @@ __attribute__((amdgpu_waves_per_eu(WPE))) k_conv_cols(const ConvCols C)
         const int blk = (int)logical;
         const ConvColIn in{make_rsrc(C.Sa.p + C.Sa.block(0, blk), ((long long)C.Sa.rows << lcb) * 16), t, lcb, C.Sa.rows, C.ra};
         const ConvColOut out{make_rsrc(C.KT + ((long long)blk * P << lcb), span), t, lcb, P, 0};
-        mix_fft<false, false, -1>(C.F, row, i, true, row, i, true, -1.0, in, out);
+        mix_fft<false, false, -1>(C.F, MixLds{row}, i, true, MixLds{row}, i, true, -1.0, in, out);
     } else if constexpr (MODE == CC_CONV) {
         // images fastest: neighbouring workgroups share their block of K^ in the L2
         const int img = (int)(logical % (unsigned)C.nimg), blk = (int)(logical / (unsigned)C.nimg);
@@ -487,7 +487,7 @@ __attribute__((amdgpu_waves_per_eu(WPE))) k_conv_cols(const ConvCols C)
         for (int b = chunk * C.chunk; b < b1; ++b) {
             const ConvColIn2 in{(isg ? C.Sg.p : C.Sa.p) + C.Sa.block(b, blk) + part * C.sub + (t & (C.sub - 1)), lcb,
                                 C.Sa.rows, isg ? C.rg : C.ra};
-            mix_fft<false, true, -1>(C.F, row, i, true, row, i, true, -1.0, in, MixLds{row});
+            mix_fft<false, true, -1>(C.F, MixLds{row}, i, true, MixLds{row}, i, true, -1.0, in, MixLds{row});
             const int e0 = opaque(tid);   // the LDS addresses are not worth registers across the transform
 #pragma unroll
             for (int q = 0; q < kConvAcc; ++q) {
@@ -509,7 +509,7 @@ __attribute__((amdgpu_waves_per_eu(WPE))) k_conv_cols(const ConvCols C)
         const int blk = (int)logical;
         const ConvAccIn in{C.acc + ((long long)blk * P << lcb), (long long)nblk * P << lcb, C.nchunk, t, lcb};
         const ConvColOut out{make_rsrc(C.So.p + C.So.block(0, blk), ((long long)C.So.rows << lcb) * 16), t, lcb, C.So.rows, C.oy};
-        mix_fft<false, false, 1>(C.F, row, i, true, row, i, true, 1.0, in, out);
+        mix_fft<false, false, 1>(C.F, MixLds{row}, i, true, MixLds{row}, i, true, 1.0, in, out);
     }
 }
 

@@ -33,7 +33,7 @@
 //   DST-IV   as DCT-IV                            forward   y[k] = -2 Im(e^{-i pi k/2N} Z[k])
 // (each follows from writing the cosine / sine as the real / imaginary part of
 // one exponential and collecting the DFT kernel).  The half-length forms take
-// their pre / post twiddles, and the fused kernel its LDS-stage roots, from
+// their pre / post twiddles, and the one-kernel path its stage twiddles, from
 // per-axis tables written by the long-double host generator (one length per
 // axis, so one table serves every line); the full-length forms use FP64
 // sincospi.
@@ -43,11 +43,12 @@
 // across lines, which keeps the strided gathers and scatters coalesced; the
 // c2c then runs over the workspace's strided axis).
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "butterflies.h"
 #include "engine.h"
-#include "lds_fft.h"
+#include "mix_fft.h"
 
 namespace ifft {
 
@@ -73,9 +74,8 @@ struct R2rParams {
     double fct;
     // half-length lines: the twiddles of the pre / post steps, L + 1 entries each
     // (types 2, 3: e1[k] = exp(i pi 2k / N), e2[k] = exp(i pi k / 2N);
-    //  type 4: e1[k] = exp(i pi k / N), e2[k] = exp(i pi (4k + 1) / 4N)),
-    // and W_L^j (j < L) for the fused kernel's LDS stages
-    const double2 *e1, *e2, *ftw;
+    //  type 4: e1[k] = exp(i pi k / N), e2[k] = exp(i pi (4k + 1) / 4N))
+    const double2 *e1, *e2;
 };
 
 // (line, point) of work item e and the workspace index of that point
@@ -312,46 +312,254 @@ __global__ void k_r2r_post(const R2rParams P)
     }
 }
 
-// Types 2-4 at even N with the N/2-point transform in LDS: `count` lines per
-// workgroup (count M <= 8 THREADS points), each loaded, transformed and stored
-// by THREADS / count threads, so HBM sees each line read once and written once.
-// One instance per type keeps only that type's pre- and post-processing in
-// the kernel; three waves per SIMD (168 registers) let three 256-thread
-// workgroups share a CU.
-constexpr int kR2rFusedMax = 4096;   // longest N/2 the fused kernel takes (512 threads)
-#ifndef DCT_FUSED_WPE
-#define DCT_FUSED_WPE 3
-#endif
+// ---------------------------------------------------------------------------
+// types 2-4 at even N in one kernel per axis
+// ---------------------------------------------------------------------------
 
-// SMALL: a 7-smooth M, transformed by inlined radix-2..8 stages (no call frames in
-// scratch memory); other lengths call the per-radix stage functions.
-template <int TYPE, int THREADS, bool SMALL>
-__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(DCT_FUSED_WPE)))
-k_r2r_fused(const R2rParams P, int count)
+// A workgroup takes `tb` lines along or across which its lanes walk (col), builds each line's
+// N/2-point sequence in an LDS row, runs the mixed-radix stages (mix_fft.h) there and forms the
+// outputs from the row, so HBM sees each line read once and written once whatever its stride.
+// The half-length forms are symmetric in (k, M - k): one pair of points shares its inputs, roots and
+// products, and along a unit-stride line the real words move in aligned pairs.
+//
+// Measured on one MI355X (DCT-II unless said, one axis, one launch):
+//   2160 x 3840 columns  0.189 -> 0.056 ms (three passes before: build, c2c, form), DCT-III 0.187 -> 0.054
+//   2160 x 3840 rows     0.053 -> 0.042 ms (3.2 TB/s), DCT-III 0.072 -> 0.037
+//   4096 x 4096 rows     0.078 -> 0.068 ms, columns 0.237 -> 0.115
+//   8 x 1080 x 1920, the middle axis  0.366 -> 0.074 ms
+// Bound now: the LDS rows (16 bytes a point) hold ten wavefronts a CU, each one load-to-store chain.
+struct R2rMix {
+    const double *src;
+    double *dst;
+    long long src_lo, src_span, dst_lo, dst_span;   // byte windows of the arrays around src / dst
+    LineMap in, out;
+    long long sa_in, sa_out;   // element stride along the axis
+    long long lines;
+    MixShape S;                // M = N/2 points
+    const double2 *e1, *e2;    // as R2rParams
+    int tb, ld, col, cosine, ortho;
+    int in_pairs, out_pairs;   // words 2j, 2j + 1 of every line are one aligned 16-byte word
+    double fct;
+};
+
+template <int TYPE, class ROW>
+__device__ __forceinline__ void r2r_mix_load(const R2rMix &P, const ROW &row, int base, int i)
 {
-    extern __shared__ double2 zl[];
-    const int M = (int)P.L;
-    const int NT = THREADS / count;
-    const int t = threadIdx.x / NT, i = threadIdx.x % NT;
-    const long long cnt = r2r_post_count(1, TYPE, P.N);
-    const double s = TYPE == 3 ? 1.0 : -1.0;
-    for (long long l0 = (long long)blockIdx.x * count; l0 < P.lines; l0 += (long long)gridDim.x * count) {
-        const long long line = l0 + t;
-        const bool valid = line < P.lines;
-        if (valid) {
-            const double *x = P.src + line_off(P.in, line);
-            for (int m = i; m < M; m += NT) zl[lpad(t * M + m)] = half_pre<TYPE>(P, x, m);
+    const int M = P.S.N, N = 2 * M, NT = P.S.NT;
+    const int step = (int)P.sa_in * 8;
+    const __amdgpu_buffer_rsrc_t r = make_rsrc((const char *)P.src + P.src_lo, P.src_span);
+    auto pair = [&](int j) -> double2 {   // x[2j], x[2j + 1]
+        const int o = base + 2 * j * step;
+        return P.in_pairs ? bload2(r, o) : make_double2(bload1(r, o), bload1(r, o + step));
+    };
+    constexpr int C = 4;   // items in flight per thread
+    if constexpr (TYPE == 2) {
+        // v[j] = x'[2j], v[N-1-j] = x'[2j+1]; the DST alternates signs
+        const double so = P.cosine ? 1.0 : -1.0;
+        for (int j0 = i; j0 < M; j0 += C * NT) {
+            double2 x[C];
+#pragma unroll
+            for (int c = 0; c < C; ++c) x[c] = pair(min(j0 + c * NT, M - 1));
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const int j = j0 + c * NT;
+                if (j < M) {
+                    row.word(j) = x[c].x;
+                    row.word(N - 1 - j) = so * x[c].y;
+                }
+            }
         }
-        __syncthreads();
-        if constexpr (SMALL) lds_fft_inline<kPointsPerThread, true>(zl, M, count, s, 2, TwTable{P.ftw, M});
-        else lds_fft(zl, M, count, s, 0, TwTable{P.ftw, M});   // both end with a barrier
-        if (valid) {
-            double *yl = P.dst + line_off(P.out, line);
-            auto Zat = [&](long long m) { return zl[lpad(t * M + (int)m)]; };
-            for (long long k = i; k < cnt; k += NT) half_post<TYPE>(P, yl, k, Zat);
+    } else if constexpr (TYPE == 3) {
+        // z[k] = (V(k) + conj V(M-k)) + i e1[k] (V(k) - conj V(M-k)), V(k) = e2[k] (x'[k] - i x'[N-k]);
+        // z[M-k] has the same sum and product conjugated
+        const __amdgpu_buffer_rsrc_t r1 = make_rsrc(P.e1, (M + 1LL) * 16), r2 = make_rsrc(P.e2, (M + 1LL) * 16);
+        const int o = P.cosine ? 0 : N - 1;   // the ortho end point as the DCT indexes it
+        auto off = [&](int n) { return base + (P.cosine ? n : N - 1 - n) * step; };
+        const int top = M / 2;
+        for (int k0 = i; k0 <= top; k0 += 2 * NT) {
+            double x[2][4];
+            double2 w1[2], wk[2], wm[2];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int k = min(k0 + c * NT, top);
+                x[c][0] = bload1(r, off(k));
+                x[c][1] = bload1(r, off(k ? N - k : N - 1));
+                x[c][2] = bload1(r, off(M - k));
+                x[c][3] = bload1(r, off(M + k < N ? M + k : N - 1));
+                w1[c] = bload2(r1, k * 16);
+                wk[c] = bload2(r2, k * 16);
+                wm[c] = bload2(r2, (M - k) * 16);
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int k = k0 + c * NT;
+                if (k > top) continue;
+                double a0 = x[c][0], a1 = k ? x[c][1] : 0.0, b0 = x[c][2], b1 = M + k < N ? x[c][3] : 0.0;
+                if (P.ortho) {
+                    if (k == o) a0 *= kSqrt2;
+                    if (k && N - k == o) a1 *= kSqrt2;
+                    if (M - k == o) b0 *= kSqrt2;
+                    if (M + k == o) b1 *= kSqrt2;
+                }
+                const double2 vk = cmul(wk[c], make_double2(a0, -a1));
+                const double2 vm = cconj(cmul(wm[c], make_double2(b0, -b1)));
+                const double2 s = cadd(vk, vm), d = cmul(w1[c], csub(vk, vm));
+                row.at(k) = make_double2(s.x - d.y, s.y + d.x);
+                if (k && 2 * k != M) row.at(M - k) = make_double2(s.x + d.y, d.x - s.y);
+            }
         }
-        __syncthreads();
+    } else {
+        // z[p] = (x'[2p] + i x'[N-1-2p]) conj(e1[p]) from the words (2p, 2p + 1) and their mirrors
+        const __amdgpu_buffer_rsrc_t r1 = make_rsrc(P.e1, (M + 1LL) * 16);
+        const int top = (M - 1) / 2;
+        for (int p0 = i; p0 <= top; p0 += 2 * NT) {
+            double2 a[2], b[2], wa[2], wb[2];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int p = min(p0 + c * NT, top);
+                a[c] = pair(p);
+                b[c] = pair(M - 1 - p);
+                wa[c] = bload2(r1, p * 16);
+                wb[c] = bload2(r1, (M - 1 - p) * 16);
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int p = p0 + c * NT;
+                if (p > top) continue;
+                // x[2p] = a.x, x[2p+1] = a.y, x[N-2-2p] = b.x, x[N-1-2p] = b.y; the DST reads reversed
+                const double2 za = P.cosine ? make_double2(a[c].x, b[c].y) : make_double2(b[c].y, a[c].x);
+                const double2 zb = P.cosine ? make_double2(b[c].x, a[c].y) : make_double2(a[c].y, b[c].x);
+                row.at(p) = cmul(za, cconj(wa[c]));
+                if (2 * p != M - 1) row.at(M - 1 - p) = cmul(zb, cconj(wb[c]));
+            }
+        }
     }
+}
+
+template <int TYPE, class ROW>
+__device__ __forceinline__ void r2r_mix_store(const R2rMix &P, const ROW &row, int base, int i)
+{
+    const int M = P.S.N, N = 2 * M, NT = P.S.NT;
+    const int step = (int)P.sa_out * 8;
+    const double f = P.fct;
+    const __amdgpu_buffer_rsrc_t r = make_rsrc((char *)P.dst + P.dst_lo, P.dst_span);
+    auto put = [&](int n, double v) { bstore1(r, base + n * step, v); };
+    auto put_pair = [&](int j, double a, double b) {   // y[2j], y[2j + 1]
+        const int o = base + 2 * j * step;
+        if (P.out_pairs) {
+            bstore2(r, o, make_double2(a, b));
+        } else {
+            bstore1(r, o, a);
+            bstore1(r, o + step, b);
+        }
+    };
+    if constexpr (TYPE == 2) {
+        // V[k] = E + conj(e1[k]) O, V[M-k] from the same pair; y[k] = 2 Re, y[N-k] = -2 Im of conj(e2) V
+        const __amdgpu_buffer_rsrc_t r1 = make_rsrc(P.e1, (M + 1LL) * 16), r2 = make_rsrc(P.e2, (M + 1LL) * 16);
+        const int o = P.cosine ? 0 : N - 1;
+        const int top = M / 2;
+        auto out = [&](int n, double v) {   // output n as the DCT forms it (the DST stores it reversed)
+            if (P.ortho && n == o) v *= 0.5 * kSqrt2;
+            put(P.cosine ? n : N - 1 - n, v * f);
+        };
+        for (int k0 = i; k0 <= top; k0 += 2 * NT) {
+            double2 w1[2], wk[2], wm[2], zk[2], zm[2];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int k = min(k0 + c * NT, top);
+                w1[c] = bload2(r1, k * 16);
+                wk[c] = bload2(r2, k * 16);
+                wm[c] = bload2(r2, (M - k) * 16);
+                zk[c] = row.at(k);
+                zm[c] = cconj(row.at(k ? M - k : 0));
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int k = k0 + c * NT;
+                if (k > top) continue;
+                const double2 ev = cscale(cadd(zk[c], zm[c]), 0.5), d = csub(zk[c], zm[c]);
+                const double2 od = cmul(cconj(w1[c]), make_double2(0.5 * d.y, -0.5 * d.x));
+                const double2 wa = cmul(cconj(wk[c]), cadd(ev, od));
+                const double2 wb = cmul(cconj(wm[c]), make_double2(ev.x - od.x, od.y - ev.y));
+                out(k, 2.0 * wa.x);
+                if (k) out(N - k, -2.0 * wa.y);
+                if (2 * k != M) {
+                    out(M - k, 2.0 * wb.x);
+                    if (k) out(M + k, -2.0 * wb.y);
+                }
+            }
+        }
+    } else if constexpr (TYPE == 3) {
+        // y[2j] = v[j], y[2j+1] = v[N-1-j], v the real view of the row; the DST alternates signs
+        const double so = P.cosine ? f : -f;
+        for (int j = i; j < M; j += NT) put_pair(j, f * row.word(j), so * row.word(N - 1 - j));
+    } else {
+        // S = conj(e2[k]) Z[k]; y[2k] = 2 Re S[k], y[2k+1] = -2 Im S[M-1-k]
+        const __amdgpu_buffer_rsrc_t r2 = make_rsrc(P.e2, (M + 1LL) * 16);
+        const int top = (M - 1) / 2;
+        const double se = 2.0 * f, so = P.cosine ? -2.0 * f : 2.0 * f;
+        for (int k0 = i; k0 <= top; k0 += 2 * NT) {
+            double2 wa[2], wb[2];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int k = min(k0 + c * NT, top);
+                wa[c] = bload2(r2, k * 16);
+                wb[c] = bload2(r2, (M - 1 - k) * 16);
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int k = k0 + c * NT;
+                if (k > top) continue;
+                const double2 sa = cmul(row.at(k), cconj(wa[c])), sb = cmul(row.at(M - 1 - k), cconj(wb[c]));
+                put_pair(k, se * sa.x, so * sb.y);
+                if (2 * k != M - 1) put_pair(M - 1 - k, se * sb.x, so * sa.y);
+            }
+        }
+    }
+}
+
+template <int TYPE, int WPE, bool PAD>
+__global__ void __launch_bounds__(kMixMaxThreads) __attribute__((amdgpu_waves_per_eu(WPE))) k_r2r_mix(const R2rMix P)
+{
+    using ROW = typename std::conditional<PAD, MixLdsPad, MixLds>::type;
+    extern __shared__ double2 zl[];
+    __shared__ int off[2][kMaxTB];
+    const int tid = (int)threadIdx.x, tb = P.tb, NT = P.S.NT;
+    const long long l0 = (long long)xcd_block(blockIdx.x, gridDim.x) * tb;
+    if (tid < tb && l0 + tid < P.lines) {
+        off[0][tid] = (int)(line_off(P.in, l0 + tid) * 8 - P.src_lo);
+        off[1][tid] = (int)(line_off(P.out, l0 + tid) * 8 - P.dst_lo);
+    }
+    const int t = P.col ? tid % tb : tid / NT, i = P.col ? tid / tb : tid % NT;
+    const bool valid = l0 + t < P.lines;
+    const ROW row{zl + t * P.ld};
+    __syncthreads();
+    if (valid) r2r_mix_load<TYPE>(P, row, off[0][t], i);
+    __syncthreads();
+    if (P.S.nst) mix_fft<true, true, TYPE == 3 ? 1 : -1>(P.S, row, i, true, row, i, true, 1.0, row, row);
+    if (valid) r2r_mix_store<TYPE>(P, row, off[1][t], i);
+}
+
+template <int TYPE, int WPE>
+static void launch_r2r_mix_tw(const R2rMix &Q, bool pad, unsigned grid, unsigned block, size_t lds, hipStream_t s)
+{
+    if (pad) hipLaunchKernelGGL((k_r2r_mix<TYPE, WPE, true>), dim3(grid), dim3(block), lds, s, Q);
+    else hipLaunchKernelGGL((k_r2r_mix<TYPE, WPE, false>), dim3(grid), dim3(block), lds, s, Q);
+}
+
+template <int TYPE>
+static hipError_t launch_r2r_mix(const R2rMix &Q, bool pad, unsigned grid, unsigned block, size_t lds, hipStream_t s)
+{
+    static std::once_flag attr_once;
+    std::call_once(attr_once, [] {
+        for (const void *f : {(const void *)k_r2r_mix<TYPE, 3, false>, (const void *)k_r2r_mix<TYPE, 3, true>,
+                              (const void *)k_r2r_mix<TYPE, 4, false>, (const void *)k_r2r_mix<TYPE, 4, true>})
+            if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 2048) != hipSuccess)
+                (void)hipGetLastError();
+    });
+    if (mix_wpe(grid, block) == 3) launch_r2r_mix_tw<TYPE, 3>(Q, pad, grid, block, lds, s);
+    else launch_r2r_mix_tw<TYPE, 4>(Q, pad, grid, block, lds, s);
+    return hipGetLastError();
 }
 
 static bool smooth13_r2r(long long n)
@@ -361,50 +569,7 @@ static bool smooth13_r2r(long long n)
     return n == 1;
 }
 
-static bool smooth7_r2r(long long n)
-{
-    for (int p : {2, 3, 5, 7})
-        while (n % p == 0) n /= p;
-    return n == 1;
-}
-
-// workgroup size of the fused kernel for N/2 = M, and lines per workgroup: the
-// largest power of two <= 64 with count M <= 8 threads
-static int fused_threads(long long M) { return M <= 2048 ? 256 : 512; }
-static int fused_count(long long M)
-{
-    const long long budget = 8LL * fused_threads(M);
-    int c = 1;
-    while (2 * c <= 64 && 2 * c * M <= budget) c *= 2;
-    return c;
-}
-
-template <int THREADS, bool SMALL>
-static hipError_t launch_fused_ts(int type, const R2rParams &Q, unsigned grid, size_t lds, int count, hipStream_t s)
-{
-    switch (type) {
-        case 2: hipLaunchKernelGGL((k_r2r_fused<2, THREADS, SMALL>), dim3(grid), dim3(THREADS), lds, s, Q, count); break;
-        case 3: hipLaunchKernelGGL((k_r2r_fused<3, THREADS, SMALL>), dim3(grid), dim3(THREADS), lds, s, Q, count); break;
-        default: hipLaunchKernelGGL((k_r2r_fused<4, THREADS, SMALL>), dim3(grid), dim3(THREADS), lds, s, Q, count); break;
-    }
-    return hipGetLastError();
-}
-
-template <int THREADS>
-static hipError_t launch_fused_t(int type, bool small, const R2rParams &Q, unsigned grid, size_t lds, int count,
-                                 hipStream_t s)
-{
-    static std::once_flag attr_once;
-    std::call_once(attr_once, [] {
-        for (const void *f : {(const void *)k_r2r_fused<2, THREADS, false>, (const void *)k_r2r_fused<3, THREADS, false>,
-                              (const void *)k_r2r_fused<4, THREADS, false>, (const void *)k_r2r_fused<2, THREADS, true>,
-                              (const void *)k_r2r_fused<3, THREADS, true>, (const void *)k_r2r_fused<4, THREADS, true>})
-            if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) != hipSuccess)
-                (void)hipGetLastError();
-    });
-    return small ? launch_fused_ts<THREADS, true>(type, Q, grid, lds, count, s)
-                 : launch_fused_ts<THREADS, false>(type, Q, grid, lds, count, s);
-}
+constexpr int kR2rMixMax = 4096;   // longest N/2 of the one-kernel path
 
 struct R2r {
     int cosine = 1, type = 2, ortho = 0;
@@ -412,8 +577,11 @@ struct R2r {
         int axis;
         long long N, L, lines;
         int forward, half, col;
-        int fused;                        // one LDS kernel per line batch (no sub-plan)
-        std::shared_ptr<DevBuf> tab;      // half lines: e1 | e2 (L + 1 each) | W_L^j (fused, L)
+        int fused;                        // one kernel (no sub-plan)
+        MixShape S;                       // ... its stages, lines per workgroup and LDS row length
+        int tb, ld, pad;
+        std::vector<int> rad;
+        std::shared_ptr<DevBuf> tab;      // half lines: e1 | e2 (L + 1 each) | stage twiddles (fused)
         LineMap in_first, in_next, out;
         long long sa_in_first, sa_in_next, sa_out;
         std::unique_ptr<Plan> fft;
@@ -440,7 +608,7 @@ static LineMap line_map(const std::vector<size_t> &shape, const std::vector<ptrd
 static int half_tables(R2r::Axis &A, int type, Error &err)
 {
     const long long N = A.N, L = A.L;
-    std::vector<double2> t((size_t)(2 * (L + 1) + (A.fused ? L : 0)));
+    std::vector<double2> t((size_t)(2 * (L + 1))), stages;
     auto cj = [](double2 w) { return make_double2(w.x, -w.y); };   // exp(+i..) from W = exp(-i..)
     for (long long k = 0; k <= L; ++k) {
         if (type == 4) {
@@ -451,8 +619,10 @@ static int half_tables(R2r::Axis &A, int type, Error &err)
             t[(size_t)(L + 1 + k)] = cj(twiddle_at((uint64_t)k, (uint64_t)(4 * N)));
         }
     }
-    if (A.fused)
-        for (long long j = 0; j < L; ++j) t[(size_t)(2 * (L + 1) + j)] = twiddle_at((uint64_t)j, (uint64_t)L);
+    if (A.fused && !A.rad.empty()) {
+        mix_table(stages, A.rad, type == 3 ? 1 : -1);
+        t.insert(t.end(), stages.begin(), stages.end());
+    }
     A.tab = std::make_shared<DevBuf>();
     if (A.tab->alloc(t.size() * sizeof(double2))) { err = {E_NOMEM, "DCT/DST table allocation failed"}; return E_NOMEM; }
     if (hipMemcpy(A.tab->p, t.data(), t.size() * sizeof(double2), hipMemcpyHostToDevice) != hipSuccess) {
@@ -460,7 +630,58 @@ static int half_tables(R2r::Axis &A, int type, Error &err)
         err = {E_HIP, "hipMemcpy of a DCT/DST table failed"};
         return E_HIP;
     }
+    A.S.tw = (const double2 *)A.tab->p + 2 * (L + 1);
     return OK;
+}
+
+// The stages, lines per workgroup and LDS rows of the one-kernel path (M = N/2 points): as the
+// engine's mixed-radix passes, one line where it fills a wavefront along rows.
+static bool mix_axis(R2r::Axis &A)
+{
+    if (!A.half || A.L > kR2rMixMax || !smooth13_r2r(A.L)) return false;
+    int nt = 1;
+    A.S = MixShape{(int)A.L, 0, 0, 1, nullptr};
+    if (A.L > 1) {
+        if (!mix_factor((int)A.L, kMixMaxThreads, A.rad, nt, nullptr, 1)) return false;
+        if (!A.col && (A.L & (A.L - 1)) == 0) {
+            // powers of two along rows: radix-8 stages with one butterfly a thread, twice the wavefronts
+            // per LDS row of the radix-16 plan (4096 rows of 4096 points: 86 us with 8 16 16, 68 us so)
+            A.rad.clear();
+            long long m = A.L;
+            while (m % 8 == 0) { A.rad.push_back(8); m /= 8; }
+            if (m > 1) A.rad.insert(A.rad.begin(), (int)m);
+            nt = (int)std::max<long long>(1, A.L / 8);
+        }
+        A.S.NT = nt;
+        A.S.nst = (int)A.rad.size();
+        for (size_t k = 0; k < A.rad.size(); ++k) A.S.codes |= (unsigned)(A.rad[k] - 1) << (4 * k);
+    }
+    A.pad = !A.rad.empty() && A.rad[0] % 2 == 0;
+    const long long len = A.pad ? A.L + A.L / 16 + 1 : A.L;
+    const long long row = len * 16, fit = kMixMaxThreads / nt;
+    long long tb;
+    if (A.col) {
+        // about 40 KiB of LDS a workgroup, four to a CU, and two lines at least: small workgroups
+        // overlap one's loads with another's stages (1080-line columns 66 us with four lines of 32-byte
+        // runs, 56 us with two; 540-point columns 92 us with eight, 73 us with four).  Lines too long
+        // for two take four in one workgroup a CU (2048 points: 248 us alone, 136 with two, 116 with four).
+        tb = std::min<long long>(8, 40 * 1024 / row);
+        if (tb < 2) tb = 2 * row <= 53 * 1024 ? 2 : std::min<long long>(4, 150 * 1024 / row);
+        tb = std::max<long long>(tb, std::min<long long>(256 / nt, 40 * 1024 / row));
+    } else {
+        tb = nt >= 64 ? 1 : std::min<long long>(128 / nt, 80 * 1024 / row);
+    }
+    tb = std::min<long long>(std::min<long long>(tb, kMaxTB), fit);
+    tb = std::max<long long>(1, std::min(tb, std::max<long long>(A.col ? 2 : 1, A.lines / 512)));
+    if (A.col)
+        while (tb & (tb - 1)) tb &= tb - 1;
+    A.tb = (int)tb;
+    A.ld = (int)len;
+    if (A.col && tb > 1) {   // lanes across lines meet distinct bank groups
+        const int o = tb >= 8 ? 1 : 8 / (int)tb;
+        while (A.ld % 8 != o) ++A.ld;
+    }
+    return true;
 }
 
 int r2r_plan_create(std::unique_ptr<Plan> &out, int kind, int type, int ortho, int dtype, size_t ndim,
@@ -530,8 +751,8 @@ int r2r_plan_create(std::unique_ptr<Plan> &out, int kind, int type, int ortho, i
         A.sa_in_next = A.sa_out = P.sout[A.axis] / 8;
         // threads walk along lines when the axis is the input's unit-stride dimension, else across lines
         A.col = A.lines > 1 && std::llabs(a == 0 ? A.sa_in_first : A.sa_in_next) != 1;
-        // lines along the unit-stride axis, N/2 13-smooth and within the LDS budget: one fused kernel
-        A.fused = A.half && !A.col && A.L <= kR2rFusedMax && smooth13_r2r(A.L);
+        // one kernel where N/2 splits into its radices and all offsets fit 31 bits
+        A.fused = P.in_hi - P.in_lo <= 0x7fffffff && P.out_hi - P.out_lo <= 0x7fffffff && mix_axis(A);
         if (A.half && (rc = half_tables(A, type, err)) != OK) return rc;
         if (A.fused) {
             R->ax.push_back(std::move(A));
@@ -560,6 +781,14 @@ int r2r_num_launches(const R2r &R)
     return n;
 }
 
+// every line starts at an even element
+static bool even_lines(const LineMap &m)
+{
+    for (int d = 0; d < m.nd; ++d)
+        if (m.cnt[d] > 1 && m.st[d] % 2) return false;
+    return true;
+}
+
 int r2r_execute(Plan &P, const void *in, void *out, double fct, hipStream_t s, Error &err)
 {
     R2r &R = *P.r2r;
@@ -585,15 +814,35 @@ int r2r_execute(Plan &P, const void *in, void *out, double fct, hipStream_t s, E
         const double2 *tb = A.tab ? (const double2 *)A.tab->p : nullptr;
         Q.e1 = tb;
         Q.e2 = tb ? tb + (A.L + 1) : nullptr;
-        Q.ftw = tb && A.fused ? tb + 2 * (A.L + 1) : nullptr;
         if (A.fused) {
-            const int count = fused_count(A.L);
-            const long long groups = (A.lines + count - 1) / count;
-            const size_t lds = (size_t)lds_points_padded((int)(count * A.L)) * sizeof(double2);
-            const unsigned grid = (unsigned)std::min<long long>(groups, 1 << 20);
-            const bool small = smooth7_r2r(A.L);
-            hipError_t e = fused_threads(A.L) == 256 ? launch_fused_t<256>(R.type, small, Q, grid, lds, count, s)
-                                                     : launch_fused_t<512>(R.type, small, Q, grid, lds, count, s);
+            R2rMix F{};
+            F.src = Q.src;
+            F.dst = Q.dst;
+            F.src_lo = a == 0 ? P.in_lo : P.out_lo;
+            F.src_span = a == 0 ? P.in_hi - P.in_lo : P.out_hi - P.out_lo;
+            F.dst_lo = P.out_lo;
+            F.dst_span = P.out_hi - P.out_lo;
+            F.in = Q.in;
+            F.out = Q.out;
+            F.sa_in = Q.sa_in;
+            F.sa_out = Q.sa_out;
+            F.lines = A.lines;
+            F.S = A.S;
+            F.e1 = Q.e1;
+            F.e2 = Q.e2;
+            F.tb = A.tb;
+            F.ld = A.ld;
+            F.col = A.col && A.tb > 1;
+            F.cosine = R.cosine;
+            F.ortho = R.ortho;
+            F.in_pairs = F.sa_in == 1 && even_lines(F.in) && (uintptr_t)F.src % 16 == 0;
+            F.out_pairs = F.sa_out == 1 && even_lines(F.out) && (uintptr_t)F.dst % 16 == 0;
+            F.fct = Q.fct;
+            const unsigned grid = (unsigned)((A.lines + A.tb - 1) / A.tb), block = (unsigned)(A.tb * A.S.NT);
+            const size_t lds = (size_t)A.ld * (size_t)A.tb * sizeof(double2);
+            hipError_t e = R.type == 2   ? launch_r2r_mix<2>(F, A.pad, grid, block, lds, s)
+                           : R.type == 3 ? launch_r2r_mix<3>(F, A.pad, grid, block, lds, s)
+                                         : launch_r2r_mix<4>(F, A.pad, grid, block, lds, s);
             if (e != hipSuccess) { err = {E_HIP, std::string("DCT/DST launch: ") + hipGetErrorString(e)}; return E_HIP; }
             continue;
         }

@@ -187,7 +187,8 @@ void mfma_destroy(Mfma *m);
 
 // mixed-radix shapes (twiddle.hip)
 int mix_ops(int R);   // VALU operations of one radix-R butterfly
-bool mix_factor(int N, int max_threads, std::vector<int> &radices, int &threads, double *cost = nullptr);
+bool mix_factor(int N, int max_threads, std::vector<int> &radices, int &threads, double *cost = nullptr,
+                int min_stages = 2);
 void mix_table(std::vector<double2> &out, const std::vector<int> &radices, int sign);
 
 // host FP64 twiddles (twiddle.hip)

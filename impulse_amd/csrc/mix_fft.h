@@ -2,7 +2,7 @@
 // first stage's inputs and the last stage's outputs going straight between
 // registers and the caller's loads and stores.
 //
-// A length N = R0 R1 ... (2 to 4 stages, any radices 2..16) is factored on the
+// A length N = R0 R1 ... (two or three stages mostly, any radices 2..16) is factored on the
 // host (mix_factor).  Stage s of radix R, with p the product of the earlier
 // radices, takes butterflies b in [0, N/R), k = b mod p:
 //   inputs  x[b + q N/R] W_{pR}^{q k},  outputs y[(b - k) R + k + q p],  q < R,
@@ -106,7 +106,7 @@ template <int R> __device__ __forceinline__ void dftm(double2 *v, double s)
 // stages
 // ---------------------------------------------------------------------------
 
-constexpr int kMixMaxStages = 4;
+constexpr int kMixMaxStages = 6;
 
 // f(std::integral_constant<int, 0>{}), ..., f(std::integral_constant<int, N - 1>{})
 template <int N, class F, int... I>
@@ -163,6 +163,8 @@ __device__ __forceinline__ void mix_radix(int r, F &&f)
 // LDS end of a stage: point idx at buf[idx]
 struct MixLds {
     double2 *buf;
+    __device__ __forceinline__ double2 &at(int idx) const { return buf[idx]; }
+    __device__ __forceinline__ double &word(int d) const { return ((double *)buf)[d]; }   // real view
     template <int R> __device__ __forceinline__ void load(double2 *v, int b, int nb) const
     {
 #pragma unroll
@@ -172,6 +174,25 @@ struct MixLds {
     {
 #pragma unroll
         for (int q = 0; q < R; ++q) buf[j + q * p] = v[q];
+    }
+};
+
+// The same with one word skipped every 16, for lengths with no odd radix to put first: the first
+// stage's writes, whose stride is the radix, then spread over the banks.
+struct MixLdsPad {
+    double2 *buf;
+    static constexpr __host__ __device__ int pad(int idx) { return idx + (idx >> 4); }
+    __device__ __forceinline__ double2 &at(int idx) const { return buf[pad(idx)]; }
+    __device__ __forceinline__ double &word(int d) const { return ((double *)(buf + pad(d >> 1)))[d & 1]; }
+    template <int R> __device__ __forceinline__ void load(double2 *v, int b, int nb) const
+    {
+#pragma unroll
+        for (int q = 0; q < R; ++q) v[q] = buf[pad(b + q * nb)];
+    }
+    template <int R, class G> __device__ __forceinline__ void store(const double2 *v, int j, int p, G) const
+    {
+#pragma unroll
+        for (int q = 0; q < R; ++q) buf[pad(j + q * p)] = v[q];
     }
 };
 
@@ -221,13 +242,13 @@ struct MixShape {
 };
 
 // A whole transform: `ld` is the source of the first stage, `st` the
-// destination of the last one (or the LDS rows themselves), `buf` this thread's
-// LDS row.  (i, lim_in) and (o, obuf, lim_out) are the thread's slot on the load
+// destination of the last one (or the LDS rows themselves), `row` this thread's
+// LDS row.  (i, on_in) and (o, orow, on_out) are the thread's slot on the load
 // and store side, which may differ when lanes walk another way there.
 // LD_LDS: the inputs already sit in the LDS rows (behind a barrier).  ST_LDS: the
 // outputs stay in LDS rows, natural order; a barrier follows.
-template <bool LD_LDS, bool ST_LDS, int SG = 0, class LD, class ST>
-__device__ __forceinline__ void mix_fft(const MixShape &S, double2 *buf, int i, bool on_in, double2 *obuf, int o,
+template <bool LD_LDS, bool ST_LDS, int SG = 0, class ROW, class LD, class ST>
+__device__ __forceinline__ void mix_fft(const MixShape &S, const ROW &row, int i, bool on_in, const ROW &orow, int o,
                                         bool on_out, double s, const LD &ld, const ST &st)
 {
     const int N = S.N, NT = S.NT;
@@ -235,7 +256,7 @@ __device__ __forceinline__ void mix_fft(const MixShape &S, double2 *buf, int i, 
     mix_radix((int)(codes & 15u) + 1, [&](auto rc) __attribute__((always_inline)) {
         constexpr int R = decltype(rc)::value;
         const int nb = opaque_scalar(N) / R;
-        mix_stage<R, true, LD_LDS, SG>(nb, on_in ? nb : 0, 1, i, NT, s, nullptr, ld, MixLds{buf});
+        mix_stage<R, true, LD_LDS, SG>(nb, on_in ? nb : 0, 1, i, NT, s, nullptr, ld, row);
     });
     __syncthreads();
     int p = (int)(codes & 15u) + 1;
@@ -247,7 +268,7 @@ __device__ __forceinline__ void mix_fft(const MixShape &S, double2 *buf, int i, 
         mix_radix(r, [&](auto rc) __attribute__((always_inline)) {
             constexpr int R = decltype(rc)::value;
             const int nb = opaque_scalar(N) / R;
-            mix_stage<R, false, true, SG>(nb, nb, p, i, NT, s, tw, MixLds{buf}, MixLds{buf});
+            mix_stage<R, false, true, SG>(nb, nb, p, i, NT, s, tw, row, row);
         });
         __syncthreads();
         tw += (r - 1) * p;
@@ -258,7 +279,7 @@ __device__ __forceinline__ void mix_fft(const MixShape &S, double2 *buf, int i, 
         mix_radix((int)(codes & 15u) + 1, [&](auto rc) __attribute__((always_inline)) {
             constexpr int R = decltype(rc)::value;
             const int nb = N / R;
-            mix_stage<R, false, false, SG>(nb, on_out ? nb : 0, p, o, NT, s, tw, MixLds{obuf}, st);
+            mix_stage<R, false, false, SG>(nb, on_out ? nb : 0, p, o, NT, s, tw, orow, st);
         });
     }
 }

@@ -279,9 +279,9 @@ k_fft_mix(const FftParams P)
                 for (int k = il; k <= top; k += 4 * NT) in.template pairs<4>(bl, k, NT, top);
             }
             __syncthreads();
-            mix_fft<true, ST_LDS>(S, bl, il, true, bs, is, vout, s, MixLds{bl}, st);
+            mix_fft<true, ST_LDS>(S, MixLds{bl}, il, true, MixLds{bs}, is, vout, s, MixLds{bl}, st);
         } else {
-            mix_fft<false, ST_LDS>(S, bl, il, vin, bs, is, vout, s, in, st);
+            mix_fft<false, ST_LDS>(S, MixLds{bl}, il, vin, MixLds{bs}, is, vout, s, in, st);
         }
     };
     if constexpr (!ST_LDS) {

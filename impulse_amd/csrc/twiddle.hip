@@ -66,19 +66,23 @@ int mix_ops(int R)
     return ops[R];
 }
 
-// Factors N into 2 .. 4 radices of 2 .. 16 and the threads per transform they take, or returns
+// Factors N into min_stages .. 6 radices of 2 .. 16 and the threads per transform they take, or returns
 // false.  The cheapest order by operation count wins: butterflies, twiddle products, the LDS
 // accesses of each stage with the bank conflicts of the first stage's writes (their stride is the
 // radix: 16-byte words fall on 8 bank groups, so an odd first radix has none), and the
 // per-stage overhead of every thread.
-bool mix_factor(int N, int max_threads, std::vector<int> &radices, int &threads, double *cost_out)
+bool mix_factor(int N, int max_threads, std::vector<int> &radices, int &threads, double *cost_out,
+                int min_stages)
 {
-    if (N < 4) return false;
+    if (N < (min_stages > 1 ? 4 : 2)) return false;
     double best = -1.0;
     std::vector<int> cur;
     auto nb_of = [](int R) { return R > 8 ? 1 : 16 / R; };   // mix_nb
+    int most = 2;   // two stages over the fewest there could be reach every 13-smooth length (5^5, 7^4, ...)
+    for (long long v = 1; v < N; v *= 16) ++most;
+    most = std::min(most, 6);   // kMixMaxStages
     auto rec = [&](auto &&self, int n) -> void {
-        if (n == 1 && cur.size() >= 2) {
+        if (n == 1 && (int)cur.size() >= min_stages) {
             int nt = 1;
             for (int R : cur) nt = std::max(nt, (N / R + nb_of(R) - 1) / nb_of(R));
             if (nt > max_threads) return;
@@ -97,7 +101,7 @@ bool mix_factor(int N, int max_threads, std::vector<int> &radices, int &threads,
             }
             return;
         }
-        if (cur.size() >= 4) return;
+        if ((int)cur.size() >= most) return;
         for (int R = 2; R <= 16; ++R)
             if (n % R == 0) {
                 cur.push_back(R);

@@ -17,6 +17,14 @@ pytestmark = pytest.mark.gpu
 TOL = {"f64": 1e-12, "f32": 2.0 ** -24 + 2e-15}
 
 
+@pytest.fixture(scope="module", autouse=True)
+def _device():
+    import torch   # before the library: both then share one HIP runtime
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
+    yield
+    torch.cuda.synchronize()
+
+
 def _names(plan):
     out = []
     for k in range(plan.num_launches):

@@ -14,6 +14,14 @@ pytestmark = pytest.mark.gpu
 TOL = {"f64": 1e-12, "f32": 2.0 ** -24 + 1e-12}
 
 
+@pytest.fixture(scope="module", autouse=True)
+def _device():
+    import torch   # before the library: both then share one HIP runtime
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
+    yield
+    torch.cuda.synchronize()
+
+
 def _reference(x, k, g):
     (B, H, W), (KH, KW) = x.shape, k.shape
     s = (H + KH - 1, W + KW - 1)

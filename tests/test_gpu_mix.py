@@ -25,6 +25,14 @@ LENGTHS = [18, 20, 21, 24, 26, 33, 36, 91, 96, 120, 121, 125, 143, 169, 200, 231
            1080, 1331, 1536, 1920, 2197, 2250, 3003, 3072, 4095, 4290, 5000, 6000]
 
 
+@pytest.fixture(scope="module", autouse=True)
+def _device():
+    import torch   # before the library: both then share one HIP runtime
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
+    yield
+    torch.cuda.synchronize()
+
+
 def _rand(shape, cplx, dt, seed):
     x = synth.complex_normal(shape, seed=seed) if cplx else synth.uniform(shape, -1.0, 1.0, seed=seed)
     if dt == "f32":

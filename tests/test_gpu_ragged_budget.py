@@ -12,6 +12,14 @@ from tests.conftest import rel_l2
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(scope="module", autouse=True)
+def _device():
+    import torch   # before the library: both then share one HIP runtime
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
+    yield
+    torch.cuda.synchronize()
+
+
 # 2^22: M = 2^21 = 2048 x 1024, the longest power of two of the small budget; 2^23 is beyond it
 @pytest.mark.parametrize("longest,points", [(2048, 2048), (1 << 22, 2048), (1 << 23, 4096)])
 def test_starting_budget(longest, points):
