@@ -101,6 +101,71 @@ __global__ void __launch_bounds__(256) k_upfirdn_tile(const double *__restrict__
     }
 }
 
+// Polyphase kernel with the taps in registers: a workgroup has T threads, T a multiple of `up`, and
+// thread i computes the R outputs J0 + i + k T, which share one phase.  Each tap is read once (from
+// the caches: `up` neighbouring taps per step) for R outputs, so an FMA takes one LDS read, of the
+// signal, instead of two, and the taps take no LDS and no copy into it.  The sum of an output runs in
+// ufd_output's order.  The first workgroups take the outputs whose taps meet either end of the signal,
+// and those past the last whole tile, T each by ufd_output itself: [0, lead) and [tail, nout).  2^22
+// samples on one MI355X: 160/147 with 1,601 taps 28.7 -> 23.0 us, with 6,401 taps 98 -> 46 us; 4/1 with 81
+// taps 72 -> 41 us; 320/441 with 17,641 taps 210 -> 61 us.  Bound now by the LDS reads of the signal (one
+// an FMA) and, at few taps, by HBM (3 TB/s).
+template <int R>
+__global__ void __launch_bounds__(512) k_upfirdn_phase(const double *__restrict__ t, const double *__restrict__ h,
+                                                       double *__restrict__ y, long long nt, int nh, int up, int down,
+                                                       long long nout, long long lead, long long tail)
+{
+    extern __shared__ double ts[];
+    const int T = (int)blockDim.x, i = (int)threadIdx.x;
+    const double *tb = t + (long long)blockIdx.y * nt;
+    double *yb = y + (long long)blockIdx.y * nout;
+    const long long nlead = (lead + T - 1) / T, nedge = nlead + (nout - tail + T - 1) / T;
+    if (blockIdx.x < nedge) {
+        const bool front = blockIdx.x < nlead;
+        const long long j = (front ? 0 : tail - nlead * T) + (long long)blockIdx.x * T + i;
+        if (j < (front ? lead : nout)) yb[j] = ufd_output(tb, 0, h, j, nt, nh, up, down);
+        return;
+    }
+    const long long J0 = lead + ((long long)blockIdx.x - nedge) * (T * R);
+    const long long first = J0 * down - (nh - 1), q1 = (J0 + (long long)T * R - 1) * down / up;
+    const long long q0 = first / up;
+    const int nseg = (int)(q1 - q0 + 1);
+    for (int e = i; e < nseg; e += T) ts[e] = tb[q0 + e];
+    __syncthreads();
+    const long long m = (J0 + i) * down;
+    const long long qhi = m / up;
+    const int r = (int)(m - qhi * up);
+    const int step = T / up * down;               // signal points from one output of the thread to the next
+    int c = r < nh ? (nh - 1 - r) / up + 1 : 0;   // taps of the phase
+    const double *tp = ts + (int)(qhi - q0);
+    const double *hp = h + r;
+    double a[R][4];
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) a[k][u] = 0.0;
+    for (; c >= 4; c -= 4) {
+        double w[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) w[u] = hp[u * up];
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) a[k][u] = fma(tp[k * step - u], w[u], a[k][u]);
+        tp -= 4;
+        hp += 4 * up;
+    }
+    for (; c > 0; --c) {
+        const double w = *hp;
+#pragma unroll
+        for (int k = 0; k < R; ++k) a[k][0] = fma(tp[k * step], w, a[k][0]);
+        --tp;
+        hp += up;
+    }
+#pragma unroll
+    for (int k = 0; k < R; ++k) yb[J0 + i + (long long)k * T] = (a[k][0] + a[k][1]) + (a[k][2] + a[k][3]);
+}
+
 // Fallback for filters or rate ratios whose tile does not fit LDS: taps and
 // signal read from global memory, one output per thread.
 __global__ void __launch_bounds__(256) k_upfirdn_direct(const double *__restrict__ t, const double *__restrict__ h,
@@ -173,6 +238,8 @@ struct Upfirdn {
     int up = 1, down = 1, algo = 1;
     DevBuf h;                                  // taps (direct)
     int seg_cap = 0;                           // signal points per tile in LDS (0: untiled direct kernel)
+    long long phase_lead = 0, phase_tail = 0, phase_grid = 0;
+    int phase_t = 0, phase_r = 0, phase_seg = 0;   // k_upfirdn_phase: threads, outputs per thread, LDS points (0: not taken)
     long long P = 0, B = 0, nblk = 0, nspec = 0;
     std::unique_ptr<Plan> r2c, c2r;
     DevBuf hspec, seg, spec;
@@ -204,6 +271,44 @@ static void fft_shape(Upfirdn &U)
     }
     U.B = U.P - nh1;
     U.nspec = U.P / 2 + 1;
+}
+
+// Threads (the multiple of `up` up to 512 that fills its wavefronts best, near 256 on a tie), outputs per
+// thread and LDS segment of the phase kernel.  Eight outputs a thread where that leaves 1,024 whole tiles,
+// four where that leaves 512; smaller problems are bound by one workgroup's latency and stay with the
+// tile kernel (65,536 samples, 147/160, 41 taps a phase: 11.7 us there, 20 us here), as do rates above
+// 512 and segments over the LDS budget.
+static void phase_shape(Upfirdn &U)
+{
+    int best = 0;
+    double score = -1.0;
+    for (int T = U.up; T <= 512; T += U.up) {
+        const double f = (double)T / (64 * ((T + 63) / 64)) - 0.0002 * std::abs(T - 256);
+        if (f > score) {
+            score = f;
+            best = T;
+        }
+    }
+    if (!best) return;
+    for (int R : {8, 4}) {
+        const long long per = (long long)best * R;
+        const long long span = ((per - 1) * U.down) / U.up + (U.nh - 1) / U.up + 3;
+        // whole tiles from the first output with all its taps (a multiple of T) to the last one
+        const long long lead = ((U.nh - 1 + U.down - 1) / U.down + best - 1) / best * best;
+        const long long good = std::min(U.nout, ((U.nt - 1) * U.up + U.up - 1) / U.down + 1);   // outputs with qhi <= nt - 1
+        const long long tiles = good > lead ? (good - lead) / per : 0;
+        const long long edges = (lead + best - 1) / best + (U.nout - (lead + tiles * per) + best - 1) / best;
+        if (span * 8 > (R == 8 ? kUfdLdsBytes / 2 : kUfdLdsBytes) || tiles * U.batch < (R == 8 ? 1024 : 512) ||
+            tiles + edges >= (1LL << 31))
+            continue;
+        U.phase_t = best;
+        U.phase_r = R;
+        U.phase_seg = (int)span;
+        U.phase_lead = lead;
+        U.phase_tail = lead + tiles * per;
+        U.phase_grid = tiles + edges;
+        return;
+    }
 }
 
 static bool tiles_fit(const Upfirdn &U)
@@ -246,6 +351,7 @@ int upfirdn_create(Upfirdn **out, size_t batch, size_t nt, const double *h, size
         // signal points a tile of 256 R outputs reads: floor(J1 down / up) - floor((J0 down - nh + 1) / up) + 1
         const long long span = ((256LL * kUfdTileR - 1) * down + U->nh - 1) / up + 2;
         if ((U->nh + span) * 8 <= kUfdLdsBytes && tiles_fit(*U)) U->seg_cap = (int)span;
+        phase_shape(*U);
     }
     if (U->algo == 1) {
         if (U->h.alloc(nh * 8) || hipMemcpy(U->h.p, h, nh * 8, hipMemcpyHostToDevice) != hipSuccess) {
@@ -304,7 +410,16 @@ int upfirdn_execute(Upfirdn &U, const double *t, double *y, hipStream_t s, Error
     }
     const long long total = U.batch * U.nout;
     if (U.algo == 1) {
-        if (U.seg_cap > 0) {
+        if (U.phase_t > 0) {
+            const dim3 grid((unsigned)U.phase_grid, (unsigned)U.batch), block((unsigned)U.phase_t);
+            const size_t lds = (size_t)U.phase_seg * 8;
+            if (U.phase_r == 8)
+                hipLaunchKernelGGL(k_upfirdn_phase<8>, grid, block, lds, s, t, (const double *)U.h.p, y, U.nt, (int)U.nh, U.up,
+                                   U.down, U.nout, U.phase_lead, U.phase_tail);
+            else
+                hipLaunchKernelGGL(k_upfirdn_phase<4>, grid, block, lds, s, t, (const double *)U.h.p, y, U.nt, (int)U.nh, U.up,
+                                   U.down, U.nout, U.phase_lead, U.phase_tail);
+        } else if (U.seg_cap > 0) {
             const long long tiles = (U.nout + 256 * kUfdTileR - 1) / (256 * kUfdTileR);
             const size_t lds = (size_t)(U.nh + U.seg_cap) * 8;
             hipLaunchKernelGGL(k_upfirdn_tile<kUfdTileR>, dim3((unsigned)tiles, (unsigned)U.batch), dim3(256), lds, s,
