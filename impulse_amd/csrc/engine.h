@@ -31,6 +31,7 @@ hipError_t launch_fft_pow2(const FftParams &P, int map, unsigned grid, unsigned 
 // fft_mix.hip
 int mix_wpe(unsigned grid, unsigned block);   // waves per SIMD of the instance a launch takes
 hipError_t launch_fft_mix(const FftParams &P, unsigned grid, unsigned block, size_t lds, hipStream_t s);
+hipError_t launch_fft_mix_blue(const FftParams &P, unsigned grid, unsigned block, size_t lds, hipStream_t s);
 
 // status codes (mirror impulse_fft_status)
 enum Status { OK = 0, E_INVALID = 1, E_NOMEM = 2, E_HIP = 3, E_UNSUPPORTED = 4, E_NODEVICE = 5 };
@@ -77,7 +78,7 @@ struct HostStage {
 enum BufRef : int { REF_IN = 0, REF_OUT = 1, REF_S0 = 2, REF_S1 = 3, REF_TMP = 4, REF_NONE = 5 };
 
 struct Pass {
-    enum Kind { FFT_LDS, FFT_POW2, FFT_MIX, REAL_POST } kind;
+    enum Kind { FFT_LDS, FFT_POW2, FFT_MIX, FFT_MIX_BLUE, REAL_POST } kind;
     int map = 0;                          // FFT_POW2 lane mapping (0 row, 1 col, 2 row load / col store)
     FftParams fp{};
     RealPostParams rp{};

@@ -76,6 +76,7 @@ struct FftParams {
     int nst;                   // number of Stockham stages
     int radix[kMaxStages];
     unsigned codes;            // mixed-radix kernel: radix - 1 of stage k in bits 4k .. 4k + 3
+    unsigned codes_inv;        // ... of the inverse transform of a Bluestein pass (the radices reversed)
     int NT;                    // threads per transform
     int TB;                    // transforms per workgroup
     int LD;                    // LDS words (double2) per transform
@@ -107,7 +108,8 @@ struct FftParams {
     void *dst;
     long long src_lo, src_span;   // byte window of the source array around src (lo <= 0)
     long long dst_lo, dst_span;   // byte window of the destination array around dst
-    const double2 *tw;         // W_N^j (forward sign), j < N
+    const double2 *tw;         // W_N^j (forward sign), j < N; mixed-radix kernels: the stage tables
+    const double2 *tw_inv;     // mixed-radix Bluestein: stage tables of the inverse transform
     const double2 *chirp;      // w[n] = exp(-i pi n^2 / nsig), n < nsig
     const double2 *spec;       // Bluestein kernel spectrum / N, N entries
     const double2 *rtw;        // W_{2M}^k, k <= M (real-half modes)

@@ -303,7 +303,8 @@ struct MixTurn {
 // stage leaves its outputs: that radix is transformed, multiplied (mul) and transformed back in
 // registers, and the spectrum never passes through LDS.  F: forward shape (sign -1 table), I: the
 // reversed one (sign +1 table), of the same threads.
-template <class LD, class MUL, class ST>
+// LD_LDS / ST_LDS as for mix_fft.
+template <bool LD_LDS = false, bool ST_LDS = false, class LD, class MUL, class ST>
 __device__ __forceinline__ void mix_conv(const MixShape &F, const MixShape &I, double2 *buf, int i, const LD &ld,
                                          const MUL &mul, const ST &st)
 {
@@ -313,7 +314,7 @@ __device__ __forceinline__ void mix_conv(const MixShape &F, const MixShape &I, d
     mix_radix((int)(codes & 15u) + 1, [&](auto rc) __attribute__((always_inline)) {
         constexpr int R = decltype(rc)::value;
         const int nb = N / R;
-        mix_stage<R, true, false, -1>(nb, nb, 1, i, NT, -1.0, nullptr, ld, row);
+        mix_stage<R, true, LD_LDS, -1>(nb, nb, 1, i, NT, -1.0, nullptr, ld, row);
     });
     __syncthreads();
     int p = (int)(codes & 15u) + 1;
@@ -348,8 +349,9 @@ __device__ __forceinline__ void mix_conv(const MixShape &F, const MixShape &I, d
     mix_radix((int)(codes & 15u) + 1, [&](auto rc) __attribute__((always_inline)) {
         constexpr int R = decltype(rc)::value;
         const int nb = N / R;
-        mix_stage<R, false, false, 1>(nb, nb, p, i, NT, 1.0, tw, row, st);
+        mix_stage<R, false, ST_LDS, 1>(nb, nb, p, i, NT, 1.0, tw, row, st);
     });
+    if constexpr (ST_LDS) __syncthreads();
 }
 
 }  // namespace ifft

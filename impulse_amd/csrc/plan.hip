@@ -423,19 +423,32 @@ struct Builder {
         std::vector<int> rad;
         int nt = 0;
         if (!mix_factor(P.N, kMixMaxThreads, rad, nt)) return 0;
-        const auto key = std::make_pair(P.N, P.sign);
-        auto it = mix_tw.find(key);
-        if (it == mix_tw.end()) {
-            std::vector<double2> v;
-            mix_table(v, rad, P.sign);
-            auto b = upload(v);
-            if (!b) return -1;
-            it = mix_tw.emplace(key, (const double2 *)b->p).first;
-        }
-        P.tw = it->second;
+        if (!(P.tw = mix_stage_table(rad, P.N, P.sign))) return -1;
+        return push_mix(Pass::FFT_MIX, P, src, dst, uses_fct, colL, colS, rad, nt);
+    }
+
+    // the stage tables of a length and sign (sign 2: backward, radices reversed), one upload per plan
+    const double2 *mix_stage_table(const std::vector<int> &rad, int N, int sign)
+    {
+        const auto key = std::make_pair(N, sign);
+        const auto it = mix_tw.find(key);
+        if (it != mix_tw.end()) return it->second;
+        std::vector<double2> v;
+        mix_table(v, sign == 2 ? std::vector<int>(rad.rbegin(), rad.rend()) : rad, sign < 0 ? -1 : 1);
+        const auto b = upload(v);
+        return b ? mix_tw.emplace(key, (const double2 *)b->p).first->second : nullptr;
+    }
+
+    // Completes and adds a mixed-radix pass: 1, or 0 where it does not fit.
+    int push_mix(Pass::Kind kind, FftParams P, BufRef src, BufRef dst, bool uses_fct, bool colL, bool colS,
+                 const std::vector<int> &rad, int nt)
+    {
         P.nst = (int)rad.size();
-        P.codes = 0;
-        for (size_t k = 0; k < rad.size(); ++k) P.codes |= (unsigned)(rad[k] - 1) << (4 * k);
+        P.codes = P.codes_inv = 0;
+        for (size_t k = 0; k < rad.size(); ++k) {
+            P.codes |= (unsigned)(rad[k] - 1) << (4 * k);
+            P.codes_inv |= (unsigned)(rad[rad.size() - 1 - k] - 1) << (4 * k);
+        }
         P.NT = nt;
         // Transforms per workgroup.  Along rows one where it fills a wavefront, else two wavefronts'
         // worth: small workgroups overlap one's loads with another's stages (float r2c rows of 1920
@@ -464,8 +477,9 @@ struct Builder {
         if ((long long)P.LD * tb * (long long)sizeof(double2) > cap) return 0;
         P.col_load = tb > 1 && colL;
         P.col_store = tb > 1 && colS;
+        if (kind == Pass::FFT_MIX_BLUE) P.col_load = P.col_store = tb > 1 && col;   // one mapping
         Pass ps;
-        ps.kind = Pass::FFT_MIX;
+        ps.kind = kind;
         ps.fp = P;
         ps.block = (unsigned)(tb * nt);
         const long long grid = (P.ntf + tb - 1) / tb;
@@ -475,7 +489,7 @@ struct Builder {
         ps.src = src;
         ps.dst = dst;
         ps.uses_fct = uses_fct;
-        ps.name = "k_fft_mix";
+        ps.name = kind == Pass::FFT_MIX ? "k_fft_mix" : "k_fft_mix_blue";
         ps.bytes_in = side_bytes(P, true);
         ps.bytes_out = side_bytes(P, false);
         make_alt(ps);
@@ -646,7 +660,39 @@ struct Builder {
         return true;
     }
 
-    bool bluestein_single(const Job &J, long long Ls, long long n2)
+    // The cheapest length of at least `need` points that the mixed-radix kernel takes in one pass, within
+    // 1/16 or the first sixteen smooth ones; 0 if there is none.
+    static long long mix_blue_len(long long need)
+    {
+        long long best = 0;
+        double least = 0.0;
+        int seen = 0;
+        for (long long n = std::max<long long>(need, kMixMinLen); n <= kMaxLdsLen && seen < 16; ++n) {
+            if (best && n > need + need / 16) break;
+            if (!smooth13(n)) continue;
+            ++seen;
+            std::vector<int> rad;
+            int nt;
+            double cost;
+            if (!mix_factor((int)n, kMixMaxThreads, rad, nt, &cost)) continue;
+            if (!best || cost < least) {
+                best = n;
+                least = cost;
+            }
+        }
+        return best;
+    }
+
+    // whether the mixed-radix Bluestein pass can address the job's arrays
+    bool mix_blue_fits(const Job &J) const
+    {
+        const FftParams P{};
+        const Side S{};
+        const long long win = 0x7fffff00LL;
+        return ref_bytes(J.src, S, P) <= win && ref_bytes(J.dst, S, P) <= win;
+    }
+
+    bool bluestein_single(const Job &J, long long Ls, long long n2, bool mix)
     {
         // Ls: complex signal length the chirp-z runs on (L, L/2 for even real)
         const double2 *chirp = nullptr, *spec = nullptr;
@@ -654,8 +700,6 @@ struct Builder {
         const bool real = J.kind != J_C2C;
         const bool pair = real && (J.L & 1);
         FftParams P = base(n2);
-        P.tw = table_direct(n2);
-        if (!P.tw) return false;
         P.chirp = chirp;
         P.spec = spec;
         P.chirp_in = P.conv = P.chirp_out = 1;
@@ -696,6 +740,19 @@ struct Builder {
         }
         const bool colL = !J.cnt.empty() && std::llabs(J.istr[0]) < std::llabs(J.is_ax);
         const bool colS = !J.cnt.empty() && std::llabs(J.ostr[0]) < std::llabs(J.os_ax);
+        if (mix) {
+            io_flags(P, J.src, J.dst);
+            std::vector<int> rad;
+            int nt = 0;
+            if (!mix_factor((int)n2, kMixMaxThreads, rad, nt)) return false;   // mix_blue_len found it
+            if (!(P.tw = mix_stage_table(rad, (int)n2, -1)) || !(P.tw_inv = mix_stage_table(rad, (int)n2, 2))) return false;
+            if (push_mix(Pass::FFT_MIX_BLUE, P, J.src, J.dst, J.fct, colL, colS, rad, nt) != 1) {
+                err = {E_UNSUPPORTED, "batch too large for one launch"};
+                return false;
+            }
+            return true;
+        }
+        if (!(P.tw = table_direct(n2))) return false;
         P.TB = choose_tb(P, P.ntf, colL || colS);
         P.col_load = P.TB > 1 && colL;
         P.col_store = P.TB > 1 && colS;
@@ -1079,8 +1136,10 @@ struct Builder {
         const long long Ls = real ? ((J.L & 1) ? J.L : J.L / 2) : J.L;
         if (lds_len_ok(Ls)) return single_pass(J);
         if (!smooth13(Ls)) {
+            const long long nm = mix_blue_fits(J) ? mix_blue_len(2 * Ls - 1) : 0;
+            if (nm) return bluestein_single(J, Ls, nm, true);
             const long long n2 = bluestein_n2(Ls);
-            if (lds_len_ok(n2)) return bluestein_single(J, Ls, n2);
+            if (lds_len_ok(n2)) return bluestein_single(J, Ls, n2, false);
         }
         return four_step(J);
     }
@@ -1446,7 +1505,8 @@ static int plan_execute_ws(Plan &P, const void *in, void *out, double fct, hipSt
         auto &ps = P.passes[pi];
         hipError_t e;
         if (prof) (void)hipEventRecord(ev[2 * pi], stream);
-        if (ps.kind == Pass::FFT_LDS || ps.kind == Pass::FFT_POW2 || ps.kind == Pass::FFT_MIX) {
+        if (ps.kind == Pass::FFT_LDS || ps.kind == Pass::FFT_POW2 || ps.kind == Pass::FFT_MIX ||
+            ps.kind == Pass::FFT_MIX_BLUE) {
             FftParams fp = ps.fp;
             fp.src = resolve(ps.src);
             fp.dst = resolve(ps.dst);
@@ -1456,9 +1516,10 @@ static int plan_execute_ws(Plan &P, const void *in, void *out, double fct, hipSt
             window(ps.src, fp.src_lo, fp.src_span);
             window(ps.dst, fp.dst_lo, fp.dst_span);
             fp.fct = ps.uses_fct ? fct : 1.0;
-            if (ps.kind == Pass::FFT_MIX) {
-                e = launch_fft_mix(fp, ps.grid, ps.block, ps.lds, stream);
-                ps.kname = "k_fft_mix<" + std::to_string(fp.load_mode) + ", " + std::to_string(fp.store_mode) + ", " +
+            if (ps.kind == Pass::FFT_MIX || ps.kind == Pass::FFT_MIX_BLUE) {
+                e = ps.kind == Pass::FFT_MIX ? launch_fft_mix(fp, ps.grid, ps.block, ps.lds, stream)
+                                             : launch_fft_mix_blue(fp, ps.grid, ps.block, ps.lds, stream);
+                ps.kname = std::string(ps.name) + "<" + std::to_string(fp.load_mode) + ", " + std::to_string(fp.store_mode) + ", " +
                            std::to_string(mix_wpe(ps.grid, ps.block)) + ">";
             } else if (ps.kind == Pass::FFT_POW2) {
                 e = launch_fft_pow2(fp, ps.map, ps.grid, ps.block, ps.lds, stream);

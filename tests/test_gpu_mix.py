@@ -166,3 +166,43 @@ def test_four_step(n):
     Y = F.r2c(r, [1])
     assert rel_l2(Y, oracle.r2c(r, [1], True, 1.0)) <= TOL["f64"]
     assert rel_l2(F.c2r(Y, n, [1], False, 1.0 / n), r) <= TOL["f64"]
+
+
+@pytest.mark.parametrize("dt", ["f64", "f32"])
+@pytest.mark.parametrize("n", [17, 19, 34, 51, 101, 289, 509, 1021, 1999, 2999])
+def test_bluestein(n, dt):
+    """Chirp-z lengths in one pass: c2c of n, r2c and c2r of 2 n (half length) and n (odd pairs, a last
+    row without a partner), rows and columns, and an odd row pitch (no complex words)."""
+    import torch
+    cdt, rdt = (torch.complex64, torch.float32) if dt == "f32" else (torch.complex128, torch.float64)
+    for batch in (1, 6, 7):
+        for axis in (0, 1):
+            shape = (n, batch) if axis == 0 else (batch, n)
+            x = _rand(shape, True, dt, n + batch)
+            for fwd in (True, False):
+                y, ker = _run(_lib.C2C, x, shape, cdt, [axis], fwd, 0.5)
+                assert all(k.startswith("k_fft_mix_blue") for k in ker), (n, axis, ker)
+                assert rel_l2(y, oracle.c2c(_wide(x), [axis], fwd, 0.5)) <= TOL[dt], (n, batch, axis, fwd)
+            for m in ((n, 2 * n) if n % 2 else (2 * n,)):
+                shape = (m, batch) if axis == 0 else (batch, m)
+                half = [v // 2 + 1 if a == axis else v for a, v in enumerate(shape)]
+                x = _rand(shape, False, dt, m + batch)
+                for fwd in (True, False):
+                    y, ker = _run(_lib.R2C, x, half, cdt, [axis], fwd, 1.0)
+                    assert all(k.startswith("k_fft_mix_blue") for k in ker), (m, axis, ker)
+                    assert rel_l2(y, oracle.r2c(_wide(x), [axis], fwd, 1.0)) <= TOL[dt], (m, batch, axis)
+                    h = _rand(tuple(half), True, dt, m)
+                    z, ker = _run(_lib.C2R, h, shape, rdt, [axis], fwd, 1.0 / m)
+                    assert all(k.startswith("k_fft_mix_blue") for k in ker), (m, axis, ker)
+                    assert rel_l2(z, oracle.c2r(_wide(h), m, [axis], fwd, 1.0 / m)) <= TOL[dt], (m, batch, axis)
+    wide = _rand((5, 2 * n + 3), False, dt, 9)
+    for v in (wide[:, :2 * n], wide[:, 1:2 * n + 1], wide[::-1, :n], wide[:, 2 * n::-2][:, :n]):
+        assert rel_l2(F.r2c(v, [1], True, 1.0), oracle.r2c(_wide(v), [1], True, 1.0)) <= TOL[dt]
+    c = _rand((4, n + 1, 3), True, dt, 10)
+    got = F.c2r(c[:, ::-1, :], 2 * n, [1], False, 1.0)
+    assert rel_l2(got, oracle.c2r(_wide(c[:, ::-1, :]), 2 * n, [1], False, 1.0)) <= TOL[dt]
+
+
+@pytest.mark.parametrize("n", [101, 202, 509])
+def test_bluestein_adjoint_weights(n):
+    test_adjoint_weights(n)
