@@ -54,6 +54,14 @@ __host__ __device__ constexpr int pow2_tb(int N, int map)
     return map == MAP_ROW ? (N >= 4096 ? 1 : 4096 / N) : (N >= 8192 ? 1 : (8192 / N > 64 ? 64 : 8192 / N));
 }
 
+// The same for a grid that would leave compute units idle (pow2_tb_pick): a wavefront of threads, and
+// four transforms (64-byte runs) at least where the lanes walk across them.
+__host__ __device__ constexpr int pow2_tb_small(int N, int map)
+{
+    const int wave = N >= 1024 ? 1 : 1024 / N;
+    return map == MAP_ROW || wave > 4 ? wave : 4;
+}
+
 // doubles of LDS per transform: one padded component row plus one word so
 // that rows of neighbouring transforms start on different banks; the
 // row-load / column-store variant reuses the row as N/2 complex words with
@@ -217,8 +225,11 @@ template <int MAP, int IOW> constexpr int pow2_wpe()
     return MAP == MAP_ROW ? IFFT_ROW_WPE : (MAP == MAP_COL ? IFFT_COL_WPE : IFFT_ROWCOL_WPE);
 }
 
-template <int N, int MAP, int IOW>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(pow2_wpe<MAP, IOW>()))) k_fft_pow2(const FftParams P)
+// TB transforms per workgroup: pow2_tb, or pow2_tb_small, whose few workgroups take three waves per SIMD
+// (no spills) whatever IO_W4 says.
+template <int N, int MAP, int IOW, int TB = pow2_tb(N, MAP)>
+__global__ void __launch_bounds__(512)
+    __attribute__((amdgpu_waves_per_eu(TB == pow2_tb(N, MAP) ? pow2_wpe<MAP, IOW>() : 3))) k_fft_pow2(const FftParams P)
 {
     constexpr int IO = IOW & (IO_W4 - 1);
     constexpr bool S32 = IOW & IO_S32, D32 = IOW & IO_D32, C2R = IOW & IO_C2R;
@@ -229,7 +240,6 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(pow2_w
     constexpr int LDP = pow2_ld<N, MAP>();
     using RS = Pow2Radices<N>;
     constexpr int NST = RS::n;
-    constexpr int TB = pow2_tb(N, MAP);
     const int tid = threadIdx.x;
     const int t = COL ? tid % TB : tid / NT;
     const int i = COL ? tid / TB : tid % NT;
@@ -886,8 +896,46 @@ static hipError_t launch_n(const FftParams &P, int map, int io, unsigned grid, u
     }
 }
 
+// The pow2_tb_small instances: plain, twiddled, Bluestein, c2r and r2c passes of FP64 arrays, and the
+// per-point path for whatever else meets a mapping (a misaligned array, say).
+template <int N, int MAP, int IO>
+static hipError_t launch_one_small(const FftParams &P, unsigned grid, unsigned block, size_t lds, hipStream_t s)
+{
+    hipLaunchKernelGGL((k_fft_pow2<N, MAP, IO, pow2_tb_small(N, MAP)>), dim3(grid), dim3(block), lds, s, P);
+    return hipGetLastError();
+}
+
+template <int N>
+static hipError_t launch_small(const FftParams &P, int map, int io, unsigned grid, unsigned block, size_t lds,
+                               hipStream_t s)
+{
+    if (map == MAP_ROW) {
+        switch (io) {
+            case IO_PLAIN: return launch_one_small<N, MAP_ROW, IO_PLAIN>(P, grid, block, lds, s);
+            case IO_R2C_HALF: return launch_one_small<N, MAP_ROW, IO_R2C_HALF>(P, grid, block, lds, s);
+            case IO_CONV | IO_W4: return launch_one_small<N, MAP_ROW, IO_CONV | IO_W4>(P, grid, block, lds, s);
+            default: return launch_one_small<N, MAP_ROW, IO_GENERIC>(P, grid, block, lds, s);
+        }
+    }
+    if (map == MAP_ROWCOL)
+        return io == IO_PLAIN ? launch_one_small<N, MAP_ROWCOL, IO_PLAIN>(P, grid, block, lds, s)
+                              : launch_one_small<N, MAP_ROWCOL, IO_GENERIC>(P, grid, block, lds, s);
+    switch (io) {
+        case IO_PLAIN: return launch_one_small<N, MAP_COL, IO_PLAIN>(P, grid, block, lds, s);
+        case IO_TWIDDLE: return launch_one_small<N, MAP_COL, IO_TWIDDLE>(P, grid, block, lds, s);
+        case IO_TWIDDLE | IO_C2R: return launch_one_small<N, MAP_COL, IO_TWIDDLE | IO_C2R>(P, grid, block, lds, s);
+        case IO_BLUE_IN | IO_W4: return launch_one_small<N, MAP_COL, IO_BLUE_IN | IO_W4>(P, grid, block, lds, s);
+        case IO_BLUE_OUT | IO_W4: return launch_one_small<N, MAP_COL, IO_BLUE_OUT | IO_W4>(P, grid, block, lds, s);
+        default: return launch_one_small<N, MAP_COL, IO_GENERIC>(P, grid, block, lds, s);
+    }
+}
+
+bool pow2_small(const FftParams &P, int map)
+{
+    return P.N >= 128 && P.N <= 1024 && P.TB == pow2_tb_small(P.N, map) && P.TB != pow2_tb(P.N, map);
+}
+
 bool pow2_supported(int N) { return N >= 64 && N <= 8192 && (N & (N - 1)) == 0; }
-int pow2_tb_host(int N, int map) { return pow2_tb(N, map); }
 // LDS bytes per transform (one padded component row of doubles)
 int pow2_lds_bytes(int N, int map) { return (N + N / 16 + (map == MAP_ROWCOL ? 2 : 1)) * 8; }
 
@@ -985,7 +1033,39 @@ static bool few_rounds(unsigned grid, unsigned block, size_t lds)
     return per_cu >= 1 && (long long)grid <= 4LL * per_cu * device_cus();
 }
 
-int pow2_io(const FftParams &P, int map, unsigned grid, unsigned block, size_t lds)
+int pow2_tb_host(int N, int map) { return pow2_tb(N, map); }
+
+// A grid that would leave compute units idle takes small workgroups: the same transforms on more CUs, each
+// wavefront with its own load-to-store chain.  256 CUs, one call each: c2c of 16,384 points 18.6 -> 10.8 us,
+// 65,536 18.9 -> 11.4, 262,144 23.4 -> 15.9; Bluestein 8,191 26.5 -> 19.2, 30,011 34.8 -> 19.7; 2-D 256^2
+// 14.1 -> 10.6; rows 1,000 x 512 8.4 -> 7.4 (63 -> 500 workgroups), 5,000 x 128 7.5 -> 6.9 (157); columns 128
+// x 3,000 7.8 -> 5.9 (47), 512 x 3,000 13.4 either way (188).  1,024 points across transforms gain only up
+// to a quarter of the CUs (80 columns 9.0 -> 7.0), and lose near all of them (1,800 columns 15.4 -> 16.4):
+// their runs halve to 64 bytes.  64 to 256 threads a workgroup; float arrays and other lengths keep theirs.
+int pow2_tb_pick(const FftParams &P, int map)
+{
+    const int tb = pow2_tb(P.N, map);
+    if (P.N < 128 || P.N > 1024 || P.src32 || P.dst32) return tb;
+    const int fill = P.N == 1024 && map != MAP_ROW ? device_cus() / 4 + 1 : device_cus();
+    return (P.ntf + tb - 1) / tb < fill ? pow2_tb_small(P.N, map) : tb;
+}
+
+// the instances pow2_tb_small is built for (launch_small)
+static int small_io(int map, int io)
+{
+    switch (io) {
+        case IO_PLAIN: return io;
+        case IO_R2C_HALF:
+        case IO_CONV | IO_W4: return map == MAP_ROW ? io : IO_GENERIC;
+        case IO_TWIDDLE:
+        case IO_TWIDDLE | IO_C2R:
+        case IO_BLUE_IN | IO_W4:
+        case IO_BLUE_OUT | IO_W4: return map == MAP_COL ? io : IO_GENERIC;
+        default: return IO_GENERIC;
+    }
+}
+
+static int pow2_io_full(const FftParams &P, int map, unsigned grid, unsigned block, size_t lds)
 {
     if (P.store_mode == ST_R2C_ROWPAIR) return IO_R2C_ROWPAIR;
     if (P.store_mode == ST_R2C_HALF) return map == MAP_ROWCOL ? IO_GENERIC : IO_R2C_HALF;   // plan routes rows only
@@ -996,11 +1076,17 @@ int pow2_io(const FftParams &P, int map, unsigned grid, unsigned block, size_t l
         // the twiddled store writes a workspace: no complex float instance for it
         return (io & IO_D32) && (io & (IO_W4 - 1)) == IO_TWIDDLE ? IO_GENERIC : io;
     }
-    else if (map == MAP_COL && pow2_c2r_in(P, pow2_tb(P.N, MAP_COL))) return IO_TWIDDLE | IO_C2R | (P.src32 ? IO_S32 : 0);
+    else if (map == MAP_COL && pow2_c2r_in(P, P.TB)) return IO_TWIDDLE | IO_C2R | (P.src32 ? IO_S32 : 0);
     else if (map != MAP_ROWCOL && pow2_blue_in(P)) io = IO_BLUE_IN | (P.src32 ? IO_S32 : 0);
     else if (map != MAP_ROWCOL && pow2_blue_out(P)) io = IO_BLUE_OUT | (P.dst32 ? IO_D32 : 0);
     else return IO_GENERIC;
     return few_rounds(grid, block, lds) ? (io | IO_W4) : io;
+}
+
+int pow2_io(const FftParams &P, int map, unsigned grid, unsigned block, size_t lds)
+{
+    const int io = pow2_io_full(P, map, grid, block, lds);
+    return pow2_small(P, map) ? small_io(map, io) : io;
 }
 
 // workgroups of the fused row-pair pass: the pair groups of every signal, the self-paired rows
@@ -1013,6 +1099,14 @@ long long pow2_rowpair_grid(long long signals, long long L2, int TB)
 hipError_t launch_fft_pow2(const FftParams &P, int map, unsigned grid, unsigned block, size_t lds, hipStream_t s)
 {
     const int fast = pow2_io(P, map, grid, block, lds);
+    if (pow2_small(P, map)) {
+        switch (P.N) {
+            case 128: return launch_small<128>(P, map, fast, grid, block, lds, s);
+            case 256: return launch_small<256>(P, map, fast, grid, block, lds, s);
+            case 512: return launch_small<512>(P, map, fast, grid, block, lds, s);
+            default: return launch_small<1024>(P, map, fast, grid, block, lds, s);
+        }
+    }
     switch (P.N) {
         case 64: return launch_n<64>(P, map, fast, grid, block, lds, s);
         case 128: return launch_n<128>(P, map, fast, grid, block, lds, s);

@@ -8,10 +8,11 @@
 //   c2r : c2c over all axes but the last into a contiguous temporary, then
 //         c2r along axes.back() (temporary -> output, fct).
 // Each 1-D job picks one algorithm (see build_job):
-//   length <= 8192 and 13-smooth  : one LDS pass (real transforms fused)
-//   13-smooth, longer             : four-step, two LDS passes through a workspace
-//   otherwise                     : Bluestein chirp-z with a 7-smooth length
-//                                   n2 >= 2L-1 (one LDS pass, or four passes)
+//   length <= 8192 and 13-smooth  : one pass (real transforms fused): k_fft_pow2 for
+//                                   powers of two, else k_fft_mix where it fits, else k_fft_lds
+//   13-smooth, longer             : four-step, two passes through a workspace
+//   otherwise                     : Bluestein chirp-z with a smooth length n2 >= 2L-1:
+//                                   one pass (k_fft_mix_blue or k_fft_lds), or three or four
 #include <algorithm>
 #include <climits>
 #include <cmath>
@@ -356,8 +357,8 @@ struct Builder {
         const long long cap = max_lds_bytes() - (long long)sizeof(long long) * 8 * kMaxTB - 1024;
         long long tb;
         // the kernel fixes its transforms per workgroup: 256 threads along rows,
-        // 512 across transforms
-        tb = pow2_tb_host(P.N, map);
+        // 512 across transforms, fewer on grids that would not fill the chip
+        tb = pow2_tb_pick(P, map);
         if (tb * per > cap) return false;
         P.TB = (int)tb;
         P.NT = NT;
@@ -1020,7 +1021,7 @@ struct Builder {
     {
         io_flags(P, src, dst);
         const int map = 0;
-        const long long tb = pow2_tb_host(P.N, map);
+        const long long tb = pow2_tb_pick(P, map);
         const long long per = (long long)pow2_lds_bytes(P.N, map);
         const long long cap = max_lds_bytes() - (long long)sizeof(long long) * 8 * kMaxTB - 1024;
         if (tb * per > cap) {
@@ -1523,7 +1524,7 @@ static int plan_execute_ws(Plan &P, const void *in, void *out, double fct, hipSt
                            std::to_string(mix_wpe(ps.grid, ps.block)) + ">";
             } else if (ps.kind == Pass::FFT_POW2) {
                 e = launch_fft_pow2(fp, ps.map, ps.grid, ps.block, ps.lds, stream);
-                ps.kname = "k_fft_pow2<" + std::to_string(fp.N) + ", " + std::to_string(ps.map) + ", " +
+                ps.kname = "k_fft_pow2" + (pow2_small(fp, ps.map) ? "_tb" + std::to_string(fp.TB) : std::string()) + "<" + std::to_string(fp.N) + ", " + std::to_string(ps.map) + ", " +
                            std::to_string(pow2_io(fp, ps.map, ps.grid, ps.block, ps.lds)) + ">";
             } else {
                 e = launch_fft_lds(fp, ps.grid, ps.block, ps.lds, stream);
