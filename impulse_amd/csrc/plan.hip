@@ -218,10 +218,14 @@ struct Job {
     }
 };
 
+constexpr size_t kNoAllocScratchBytes = 64ull << 20;   // scratch of execution without allocation
+static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
+
 struct Builder {
     Plan &plan;
     Error &err;
     std::map<std::pair<int, int>, const double2 *> mix_tw;   // stage tables by length and sign
+    bool smooth_blue = false;   // long Bluestein lengths by bluestein_n2 alone (four_step_shape)
 
     std::shared_ptr<DevBuf> upload(const std::vector<double2> &v)
     {
@@ -767,15 +771,87 @@ struct Builder {
         return true;
     }
 
+    struct FourStep {
+        long long n2, L1, L2;    // L2 = 0: no split
+        long long chunk;         // signals per chunk of the batch
+        size_t s0, s1;           // workspace bytes of a chunk
+        bool three;              // Bluestein in three passes
+    };
+
+    // The lengths and workspace of a four-step job.  Bluestein takes the next power of two (three passes of
+    // the power-of-two kernels, in batch chunks of up to 2 GiB) however far above the smallest smooth length
+    // it lies; the four passes of a 7-smooth length run on the generic kernels and store one pass more.
+    // MI355X, 7-smooth -> power of two: c2c of 5,003 points 74 -> 19 us, 64 x 5,003 96 -> 42; 100,003 86 ->
+    // 33, 64 x 100,003 902 -> 377; r2c 5 x 700,001 305 -> 169; 4,194,319 (2^23, 1.99 times the smooth
+    // length) 1,007 -> 590.  `smooth`: the smallest smooth length, or the power of two within 15 % of it.
+    static FourStep four_step_shape(const Job &J, bool smooth)
+    {
+        const bool real = J.kind != J_C2C;
+        const bool pair = real && (J.L & 1);
+        const long long Ls = real ? ((J.L & 1) ? J.L : J.L / 2) : J.L;
+        const bool blue = !smooth13(Ls);
+        const long long nlog = pair ? (J.nbatch() + 1) / 2 : J.nbatch();
+        FourStep F{};
+        if (blue && !smooth) {
+            F.n2 = 1;
+            while (F.n2 < 2 * Ls - 1) F.n2 *= 2;
+            F.three = split_four(F.n2, F.L1, F.L2) && conv_rows_ok(F.L1, F.n2);
+        }
+        if (!F.three) {
+            F.n2 = blue ? bluestein_n2(Ls) : Ls;
+            split_four(F.n2, F.L1, F.L2);
+            F.three = blue && F.L2 && conv_rows_ok(F.L1, F.n2);
+        }
+        // Optional batch chunks (IMPULSE_FFT_MALL_MB): the workspace of one chunk
+        // stays within the budget so that pass A's output could still sit in the
+        // MALL (Infinity Cache) when pass B reads it.  Measured on MI355X the
+        // smaller launches lose more than the cache saves, so it is off unless set.
+        const long long mall = env_ll("IMPULSE_FFT_MALL_MB", 1LL << 30) * (1LL << 20);
+        const long long per_sig = F.n2 * (long long)sizeof(double2);
+        F.chunk = std::max<long long>(1, std::min<long long>(nlog, mall / per_sig));
+        if (F.three) F.chunk = std::max<long long>(1, std::min<long long>(F.chunk, 0x7fffffffLL / per_sig));
+        F.s0 = F.s1 = (size_t)(F.chunk * per_sig);
+        // three passes work in place; r2c adds the natural-order signal of its post-process
+        if (F.three) F.s1 = J.kind == J_R2C ? (size_t)(F.chunk * Ls) * sizeof(double2) : 0;
+        return F;
+    }
+
+    // one pass of LDS, or a four-step
+    bool is_four_step(const Job &J) const
+    {
+        const bool real = J.kind != J_C2C;
+        const long long Ls = real ? ((J.L & 1) ? J.L : J.L / 2) : J.L;
+        if (lds_len_ok(Ls)) return false;
+        return smooth13(Ls) || !((mix_blue_fits(J) && mix_blue_len(2 * Ls - 1)) || lds_len_ok(bluestein_n2(Ls)));
+    }
+
+    // The power of two takes more workspace than the smooth length in some r2c plans; where only the smooth
+    // one fits the scratch of execution without allocation (`limit` bytes), it stays.
+    bool keep_smooth(const std::vector<Job> &jobs, size_t tmp, size_t limit) const
+    {
+        size_t need[2];
+        for (int sm = 0; sm < 2; ++sm) {
+            size_t s0 = 0, s1 = 0;
+            for (auto &J : jobs) {
+                if (!is_four_step(J)) continue;
+                const FourStep F = four_step_shape(J, sm);
+                s0 = std::max(s0, F.s0);
+                s1 = std::max(s1, F.s1);
+            }
+            need[sm] = align256(s0) + align256(s1) + align256(tmp);
+        }
+        return need[0] > limit && need[1] <= limit;
+    }
+
     bool four_step(const Job &J)
     {
         const bool real = J.kind != J_C2C;
         const bool pair = real && (J.L & 1);
         const long long Ls = real ? ((J.L & 1) ? J.L : J.L / 2) : J.L;   // complex signal length
         const bool blue = !smooth13(Ls);
-        const long long n2 = blue ? bluestein_n2(Ls) : Ls;
-        long long L1, L2;
-        if (!split_four(n2, L1, L2)) {
+        const FourStep F = four_step_shape(J, smooth_blue);
+        const long long n2 = F.n2, L1 = F.L1, L2 = F.L2;
+        if (!L2) {
             err = {E_UNSUPPORTED, "transform length too long for two passes"};
             return false;
         }
@@ -794,17 +870,11 @@ struct Builder {
         const double2 *chirp = nullptr, *spec = nullptr, *spec_rows = nullptr;
         if (blue && !bluestein_tables(Ls, n2, chirp, spec)) return false;
 
-        // Optional batch chunks (IMPULSE_FFT_MALL_MB): the workspace of one chunk
-        // stays within the budget so that pass A's output could still sit in the
-        // MALL (Infinity Cache) when pass B reads it.  Measured on MI355X the
-        // smaller launches lose more than the cache saves, so it is off unless set.
-        const long long mall = env_ll("IMPULSE_FFT_MALL_MB", 1LL << 30) * (1LL << 20);
-        const long long per_sig = n2 * (long long)sizeof(double2);
-        const long long chunk = std::max<long long>(1, std::min<long long>(nlog, mall / per_sig));
+        const long long chunk = F.chunk;
         long long cn = chunk;   // signals in the current chunk (captured by the pass builders)
-        const size_t ws = (size_t)(chunk * n2) * sizeof(double2);
-        ensure_ws(plan.s0_bytes, ws);
-        ensure_ws(plan.s1_bytes, ws);
+        const size_t ws = F.s0;
+        ensure_ws(plan.s0_bytes, F.s0);
+        ensure_ws(plan.s1_bytes, F.s1);
 
         auto passA = [&](FftParams P) {
             P.N = (int)L2;
@@ -900,7 +970,7 @@ struct Builder {
                 return add_fft(B, REF_S0, J.dst, J.fct, false, true);
             }
 
-            if (conv_rows_ok(L1, n2, ws)) {
+            if (F.three) {
                 // Bluestein in three passes: A1 (chirp in, forward columns, twiddle) ->
                 // B (each row in place: forward, times the spectrum, inverse, conjugate
                 // twiddle) -> A2 (inverse columns, chirp out, natural order).  With
@@ -934,8 +1004,9 @@ struct Builder {
                 A2.olim = Ls;
                 if (J.kind == J_R2C) {
                     A2.store_mode = ST_C2C;   // natural order into the workspace, then the real post-process
+                    side_lin(A2.out, Ls, 1, L1);
                     if (!add_fft(A2, REF_S0, REF_S1, false, true, true)) return false;
-                    return add_post(J, pair, Ls, n2, rlo, rhi, rS, u0, cn);
+                    return add_post(J, pair, Ls, Ls, rlo, rhi, rS, u0, cn);
                 }
                 Side outA;
                 side_dims(outA, J, false, pair);
@@ -994,10 +1065,10 @@ struct Builder {
     // the three-pass Bluestein: the row pass runs on the power-of-two row kernel
     // (rows of L1 points), whose buffer loads address the workspace and the
     // spectrum table with 31-bit byte offsets
-    static bool conv_rows_ok(long long L1, long long n2, size_t ws)
+    static bool conv_rows_ok(long long L1, long long n2)
     {
         if (env_ll("IMPULSE_FFT_NO_CONV_ROWS", 0)) return false;
-        return pow2_supported((int)L1) && L1 >= 64 && ws <= (size_t)0x7fffffff && n2 * 16 <= 0x7fffffffLL;
+        return pow2_supported((int)L1) && L1 >= 64 && n2 * 16 <= 0x7fffffffLL;
     }
 
     // the kernel spectrum in row order of the four-step split n2 = L1 L2:
@@ -1336,6 +1407,9 @@ int plan_create(std::unique_ptr<Plan> &out, int kind, int dtype, size_t ndim, co
     Builder B{P, err};
     for (auto &J : jobs) {
         if (!merge_dims(J)) { err = {E_UNSUPPORTED, "too many batch dimensions"}; return E_UNSUPPORTED; }
+    }
+    B.smooth_blue = B.keep_smooth(jobs, P.tmp_bytes, kNoAllocScratchBytes);
+    for (auto &J : jobs) {
         if (!B.build_job(J)) return err.code ? err.code : E_UNSUPPORTED;
     }
     if (P.s0.alloc(P.s0_bytes) != OK || P.s1.alloc(P.s1_bytes) != OK || P.tmp.alloc(P.tmp_bytes) != OK) {
@@ -1375,7 +1449,6 @@ int plan_execute(Plan &P, const void *in, void *out, double fct, hipStream_t str
 // call's contents; the passes write every workspace word before reading it), so
 // calls that overlap on one GPU race.  The host uses the per-device address
 // from hipGetSymbolAddress, never the array's name.
-constexpr size_t kNoAllocScratchBytes = 64ull << 20;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -1405,8 +1478,6 @@ static int scratch_address(void **out, Error &err)
     *out = g_scratch_ptr[dev];
     return OK;
 }
-
-static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 int plan_execute_noalloc(Plan &P, const void *in, void *out, double fct, hipStream_t stream, Error &err)
 {
