@@ -33,6 +33,7 @@ hipError_t launch_fft_pow2(const FftParams &P, int map, unsigned grid, unsigned 
 // fft_mix.hip
 int mix_wpe(unsigned grid, unsigned block);   // waves per SIMD of the instance a launch takes
 hipError_t launch_fft_mix(const FftParams &P, unsigned grid, unsigned block, size_t lds, hipStream_t s);
+hipError_t launch_mix_four(const FftParams &P, unsigned grid, unsigned block, size_t lds, hipStream_t s);
 hipError_t launch_fft_mix_blue(const FftParams &P, unsigned grid, unsigned block, size_t lds, hipStream_t s);
 
 // status codes (mirror impulse_fft_status)

@@ -20,6 +20,7 @@ hipError_t launch_fft_mix(const FftParams &P, unsigned grid, unsigned block, siz
     if (P.load_mode == LD_C2C && P.store_mode == ST_C2C) return launch_mix<LD_C2C, ST_C2C>(P, grid, block, lds, s);
     if (P.load_mode == LD_C2C && P.store_mode == ST_TWIDDLE)
         return launch_mix<LD_C2C, ST_TWIDDLE>(P, grid, block, lds, s);
+    if (P.load_mode == LD_C2C || P.store_mode == ST_TWIDDLE) return launch_mix_four(P, grid, block, lds, s);
     if (P.store_mode == ST_R2C_HALF || P.store_mode == ST_R2C_PAIR) return launch_mix_r2c(P, grid, block, lds, s);
     return launch_mix_c2r(P, grid, block, lds, s);
 }

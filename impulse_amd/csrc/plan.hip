@@ -155,6 +155,7 @@ static long long good_size7(long long n)
     return best;
 }
 
+// the smallest 7-smooth chirp-z length, or the power of two within 15 % of it
 static long long bluestein_n2(long long L)
 {
     const long long need = 2 * L - 1;
@@ -405,12 +406,14 @@ struct Builder {
         return S.kind == SIDE_LINEAR ? (P.ntf / std::max<long long>(1, P.ni)) * S.lin * 16 : LLONG_MAX;
     }
 
-    // The mixed-radix kernel: plain c2c, four-step twiddled stores and single-pass real transforms
-    // of lengths that split into radices 2..16, all offsets within 31 bits.  1: added, 0: not for
+    // The mixed-radix kernel: plain c2c, single-pass real transforms and the passes of a four-step,
+    // complex or real, of lengths that split into radices 2..16, all offsets within 31 bits.  1: added, 0: not for
     // this kernel, -1: error.
     int try_mix(FftParams P, BufRef src, BufRef dst, bool uses_fct, bool colL, bool colS)
     {
-        const bool modes = (P.load_mode == LD_C2C && (P.store_mode == ST_C2C || P.store_mode == ST_TWIDDLE)) ||
+        const bool first = P.store_mode == ST_TWIDDLE, last = P.load_mode == LD_C2C;   // of a four-step
+        const bool modes = (last && (P.store_mode == ST_C2C || P.store_mode == ST_C2R_HALF || P.store_mode == ST_C2R_PAIR)) ||
+                           (first && (P.load_mode == LD_C2C || P.load_mode == LD_REAL_HALF || P.load_mode == LD_R2C_PAIR)) ||
                            (P.load_mode == LD_REAL_HALF && P.store_mode == ST_R2C_HALF) ||
                            (P.load_mode == LD_R2C_PAIR && P.store_mode == ST_R2C_PAIR) ||
                            (P.load_mode == LD_C2R_HALF && P.store_mode == ST_C2R_HALF) ||
@@ -418,7 +421,7 @@ struct Builder {
         const bool half = P.load_mode == LD_REAL_HALF || P.load_mode == LD_C2R_HALF;
         const bool real = P.load_mode != LD_C2C;
         if (!modes || P.N < kMixMinLen || P.conv || P.chirp_in || P.chirp_out || P.conj_in || P.conj_out) return 0;
-        if (P.nload != P.N || (half && !P.rtw) || (real && P.ni != 1)) return 0;
+        if (P.nload != P.N || (half && !first && !P.rtw) || (real && !first && P.ni != 1)) return 0;
         if (P.store_mode == ST_TWIDDLE && (P.tw_mul != 1 || P.dst32)) return 0;
         if ((P.ni - 1) * P.in.ipos + (long long)(P.N - 1) * P.in.pst >= P.ilim ||
             (P.ni - 1) * P.out.ipos + (long long)(P.N - 1) * P.out.pst >= P.olim)
