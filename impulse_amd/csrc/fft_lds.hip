@@ -307,11 +307,11 @@ __global__ void k_unpack_halfcomplex(const double *__restrict__ hc, double2 *__r
 // ---------------------------------------------------------------------------
 
 // Measured choice (MI355X): passes along rows with one or two transforms per
-// workgroup run faster with the larger register budget (2112-point c2c rows
-// 1.29 -> 1.07 ms over 16 x 2112^2; r2c of 4096 x 4096 rows 0.185 -> 0.162 ms;
-// 256 x 4095 0.030 -> 0.028 ms), wider row tiles and passes across transforms
-// with the higher occupancy (the rows of the 2112^2 r2c, three per workgroup:
-// 1.96 -> 1.71 ms with both passes; the 2112^2 columns 1.79 -> 1.51 ms).
+// workgroup run faster with the larger register budget, wider row tiles and
+// passes across transforms with the higher occupancy.  The lengths it was
+// measured on have kernels of their own by now (k_fft_mix, k_fft_pow2): c2c rows
+// of 16 x 2112^2 1.29 ms with four waves per SIMD, 1.07 with three; their columns
+// 1.79 with three, 1.51 with four.
 int fft_lds_wpe(const FftParams &P)
 {
     return (!P.col_load && !P.col_store && P.TB <= 2) ? 3 : 4;
