@@ -899,6 +899,28 @@ static int resident_grid(const Ragged &R, int threads, int waves, size_t lds)
     return ncu * per;
 }
 
+// Whether the batch is better off with the largest budget from the start: Bluestein units that the small
+// one splits over four phases but this one keeps in LDS, no unit that it splits itself, and at most three
+// units a CU, so that the phases' latency weighs more than the overlap of small workgroups.  Times with
+// 1,024 and with 256 threads (MI355X): 100 signals of 64 to 4,096 points 73 and 99 us, 251 of 471 to 5,082
+// 83 and 106, 600 of 500 to 4,096 94 and 115; 4,000 of 64 to 4,096 305 and 169.
+static bool single_phase_pays(const Ragged &R)
+{
+    int ncu = 0;
+    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, R.device) != hipSuccess || ncu <= 0) {
+        (void)hipGetLastError();
+        ncu = 256;
+    }
+    if (R.units.size() > 3 * (size_t)ncu) return false;
+    bool split = false;
+    for (const auto &u : R.units) {
+        const long long n = (long long)R.n[(size_t)u.first], L = transform_len(n, u.second >= 0);
+        if (L > 8192) return false;
+        split |= L > 2048 && !rg_smooth13(n % 2 == 0 ? n / 2 : n);
+    }
+    return split;
+}
+
 static int build_tasks(Ragged &R, int threads, int lds_max, int waves, Error &err)
 {
     // each unit's tasks per phase, then the units dealt to eight queues per phase (largest unit
@@ -1149,6 +1171,7 @@ int ragged_create(Ragged **out, size_t count, const size_t *lengths, const size_
     // one's loads with another's stages.  Lengths it cannot split go to the larger budgets.
     rc = E_UNSUPPORTED;
     const int budget[3][3] = {{256, 2048, 3}, {512, 4096, 4}, {1024, 8192, 0}};
+    if (single_phase_pays(*R)) rc = build_tasks(*R, budget[2][0], budget[2][1], budget[2][2], err);
     for (int k = 0; k < 3 && rc == E_UNSUPPORTED; ++k) rc = build_tasks(*R, budget[k][0], budget[k][1], budget[k][2], err);
     if (rc != OK) return rc;
     *out = R.release();

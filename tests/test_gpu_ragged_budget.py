@@ -32,3 +32,18 @@ def test_starting_budget(longest, points):
     torch.cuda.synchronize()
     for n, i, v in zip(lengths, b.in_offsets, b.output_views(y)):
         assert rel_l2(v.cpu().numpy(), np.fft.rfft(x[i:i + n].astype(np.float64))) <= 1e-12, n
+
+
+@pytest.mark.parametrize("fill,points", [(0, 8192), (767, 8192), (768, 2048)])
+def test_single_phase_budget(fill, points):
+    """A Bluestein length over the small budget's points (2206 = 2 * 1103) in a batch of at most three signals a
+    CU starts with the largest budget; one signal more, and it does not."""
+    import torch
+    lengths = [96] * fill + [2206]
+    b = RaggedBatch(lengths)
+    assert b.info()["lds_points"] == points
+    x = synth.uniform(b.in_elems, -1.0, 1.0, seed=fill).astype(np.float32)
+    y = b.execute(torch.from_numpy(x).cuda(), torch.empty(b.out_elems, dtype=torch.complex128, device="cuda"))
+    torch.cuda.synchronize()
+    for n, i, v in list(zip(lengths, b.in_offsets, b.output_views(y)))[-3:]:
+        assert rel_l2(v.cpu().numpy(), np.fft.rfft(x[i:i + n].astype(np.float64))) <= 1e-12, n
