@@ -665,7 +665,7 @@ struct Ragged {
     std::vector<std::pair<long long, long long>> spec_index;   // (2 n + pair, offset), sorted
     DevBuf spec;
     double flops = 0.0;
-    size_t in_elems = 0, out_elems = 0;
+    size_t in_elems = 0, out_elems = 0, samples = 0;   // buffer extents; samples of all signals
     // captured graph for (x, y, fct)
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -928,7 +928,7 @@ static int build_tasks(Ragged &R, int threads, int lds_max, int waves, Error &er
     std::vector<RaggedTask> ph[kPhases];      // all units' tasks back to back
     std::vector<size_t> begin[kPhases];       // unit ui's tasks: [begin[ui], begin[ui + 1])
     for (int q = 0; q < kPhases; ++q) {
-        ph[q].reserve((R.in_elems + R.units.size() * 1024) / 1024);
+        ph[q].reserve(R.samples / 1024 + R.units.size());   // of the signals held: their offsets may be far apart
         begin[q].assign(R.units.size() + 1, 0);
     }
     long long ws = 0;
@@ -1133,6 +1133,7 @@ int ragged_create(Ragged **out, size_t count, const size_t *lengths, const size_
         const long long n = (long long)lengths[i];
         if (n < 1 || n > (1LL << 28)) { err = {E_INVALID, "ragged lengths must be in [1, 2^28]"}; return E_INVALID; }
         if (n > 1) R->flops += 2.5 * (double)n * std::log2((double)n);
+        R->samples += (size_t)n;
         R->in_elems = std::max<size_t>(R->in_elems, in_off[i] + (size_t)n);
         R->out_elems = std::max<size_t>(R->out_elems, out_off[i] + (size_t)n / 2 + 1);
     }
