@@ -1169,11 +1169,13 @@ int ragged_create(Ragged **out, size_t count, const size_t *lengths, const size_
     // per SIMD was the fastest of all, or within 3 % of it, on every batch measured (100 to 4,000
     // signals of 64 to 262,144 points; 4,000: 5.06 ms against 7.27 ms with 1,024 threads and 8,192
     // points, 300 of 1,000 to 200,000 points: 0.189 against 0.314 ms): three workgroups a CU overlap
-    // one's loads with another's stages.  Lengths it cannot split go to the larger budgets.
+    // one's loads with another's stages.  Lengths it cannot split go to the larger budgets, and so
+    // do batches whose workspace does not fit: transforms a budget holds in LDS need none.
     rc = E_UNSUPPORTED;
     const int budget[3][3] = {{256, 2048, 3}, {512, 4096, 4}, {1024, 8192, 0}};
     if (single_phase_pays(*R)) rc = build_tasks(*R, budget[2][0], budget[2][1], budget[2][2], err);
-    for (int k = 0; k < 3 && rc == E_UNSUPPORTED; ++k) rc = build_tasks(*R, budget[k][0], budget[k][1], budget[k][2], err);
+    for (int k = 0; k < 3 && (rc == E_UNSUPPORTED || rc == E_NOMEM); ++k)
+        rc = build_tasks(*R, budget[k][0], budget[k][1], budget[k][2], err);
     if (rc != OK) return rc;
     *out = R.release();
     return OK;

@@ -22,3 +22,24 @@ assert L.impulse_fft_ragged_configure(h, 512, 4096, 0, 0) == 0
 report(resource.getrusage(resource.RUSAGE_SELF).ru_maxrss)
 """)
     assert kib < 256 << 10
+
+
+def test_budget_follows_device_memory(hip_host):
+    # The starting budget keeps a workspace for these transforms of 8,192 points, the largest one holds
+    # them in LDS: where the workspace does not fit, the batch is created without it.
+    roomy, tight = hip_host(CREATE + """
+n = [16384] * 1000
+ins, outs = [16384 * i for i in range(1000)], [8193 * i for i in range(1000)]
+got = []
+for limit in (1 << 40, 64 << 20):
+    S.standin_limit(limit)
+    rc, h = create(n, ins, outs)
+    assert rc == 0, L.impulse_fft_last_error()
+    t, b, w = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
+    L.impulse_fft_ragged_info(h, ctypes.byref(t), ctypes.byref(b), None, None, None, None, ctypes.byref(w))
+    got.append([t.value, b.value, w.value, S.standin_used()])
+    L.impulse_fft_ragged_destroy(h)
+report(got)
+""")
+    assert roomy[1] == 2048 and roomy[2] >= 1000 * 8192 * 16
+    assert tight[1] == 8192 and tight[2] < 1024
