@@ -679,6 +679,14 @@ struct Ragged {
         exec = nullptr;
         graph = nullptr;
     }
+    // no configuration: executes are refused until one is set
+    void unplan()
+    {
+        drop_graph();
+        tasks.clear();
+        (void)ws.alloc(0);
+        (void)dtasks.alloc(0);
+    }
     ~Ragged() { drop_graph(); }
 };
 
@@ -999,13 +1007,20 @@ static int build_tasks(Ragged &R, int threads, int lds_max, int waves, Error &er
     }
     if (all.size() > (size_t)INT_MAX) { err = {E_UNSUPPORTED, "too many ragged tasks"}; return E_UNSUPPORTED; }
     const size_t wsb = (size_t)std::max<long long>(ws, 1) * sizeof(double2);
-    if (wsb > R.ws.bytes && R.ws.alloc(wsb)) { err = {E_NOMEM, "ragged workspace allocation failed"}; return E_NOMEM; }
+    // from here on the buffers of the previous configuration are gone or overwritten
+    if (wsb > R.ws.bytes && R.ws.alloc(wsb)) {
+        R.unplan();
+        err = {E_NOMEM, "ragged workspace allocation failed"};
+        return E_NOMEM;
+    }
     if (all.size() * sizeof(RaggedTask) > R.dtasks.bytes && R.dtasks.alloc(all.size() * sizeof(RaggedTask))) {
+        R.unplan();
         err = {E_NOMEM, "ragged task table allocation failed"};
         return E_NOMEM;
     }
     if (hipMemcpy(R.dtasks.p, all.data(), all.size() * sizeof(RaggedTask), hipMemcpyHostToDevice) != hipSuccess) {
         (void)hipGetLastError();
+        R.unplan();
         err = {E_HIP, "ragged task upload failed"};
         return E_HIP;
     }
@@ -1273,6 +1288,7 @@ int ragged_execute(Ragged &R, const float *x, double2 *y, double fct, hipStream_
 {
     int rc = check_ptrs(R, x, y, err);
     if (rc != OK) return rc;
+    if (R.tasks.empty()) { err = {E_INVALID, "the last ragged configuration was refused; set one that fits"}; return E_INVALID; }
     if (!graph) {
         hipError_t e = ragged_launch(R, x, y, fct, s);
         if (e != hipSuccess) { err = {E_HIP, std::string("ragged launch: ") + hipGetErrorString(e)}; return E_HIP; }
@@ -1339,7 +1355,8 @@ int ragged_tune(Ragged &R, const float *x, double2 *y, hipStream_t s, int reps, 
     for (const Cfg &c : cands) {
         Error e2{0, ""};
         if (ragged_configure(R, c.t, c.l, c.o, c.w, e2) != OK) {
-            if (e2.code == E_UNSUPPORTED) continue;   // this batch has a length the configuration cannot split
+            // this batch has a length the configuration cannot split, or too little memory for it
+            if (e2.code == E_UNSUPPORTED || e2.code == E_NOMEM) continue;
             err = e2;
             rc = e2.code;
             break;

@@ -43,3 +43,45 @@ report(got)
 """)
     assert roomy[1] == 2048 and roomy[2] >= 1000 * 8192 * 16
     assert tight[1] == 8192 and tight[2] < 1024
+
+
+def test_refused_configuration(hip_host):
+    # A configuration whose workspace does not fit is refused, and so are executes from then on until
+    # one that fits is set; nothing is launched on buffers that are gone.
+    got = hip_host(CREATE + """
+n = [16384] * 1000
+ins, outs = [16384 * i for i in range(1000)], [8193 * i for i in range(1000)]
+S.standin_limit(64 << 20)
+rc, h = create(n, ins, outs)
+assert rc == 0
+x, y = 1 << 40, 1 << 41
+run = lambda: L.impulse_fft_ragged_execute(h, x, y, 1.0, None)
+got = [run()]
+launches()
+got.append(L.impulse_fft_ragged_configure(h, 256, 2048, 0, 3))
+got.append(run())
+got.append(len(launches()))
+got.append(L.impulse_fft_ragged_configure(h, 1024, 8192, 0, 0))
+got.append(run())
+report(got)
+""")
+    NOMEM = 2
+    assert got[0] == 0 and got[1] == NOMEM
+    assert got[2] != 0 and got[3] == 0
+    assert got[4] == 0 and got[5] == 0
+
+
+def test_tuning_passes_over_what_does_not_fit(hip_host):
+    # The candidates whose workspace does not fit are left out, as those with no split are.
+    rc, budget, run = hip_host(CREATE + """
+n = [16384] * 1000
+ins, outs = [16384 * i for i in range(1000)], [8193 * i for i in range(1000)]
+S.standin_limit(64 << 20)
+rc, h = create(n, ins, outs)
+assert rc == 0
+ms, b = ctypes.c_double(), ctypes.c_int()
+rc = L.impulse_fft_ragged_tune(h, 1 << 40, 1 << 41, None, 1, ctypes.byref(ms))
+L.impulse_fft_ragged_info(h, None, ctypes.byref(b), None, None, None, None, None)
+report([rc, b.value, L.impulse_fft_ragged_execute(h, 1 << 40, 1 << 41, 1.0, None)])
+""")
+    assert (rc, budget, run) == (0, 8192, 0)
