@@ -226,6 +226,8 @@ struct Builder {
     Plan &plan;
     Error &err;
     std::map<std::pair<int, int>, const double2 *> mix_tw;   // stage tables by length and sign
+    std::map<long long, const double2 *> direct_tw;          // W_n^j tables by length
+    mutable std::map<long long, long long> blue_lens;        // mix_blue_len by the points needed
     bool smooth_blue = false;   // long Bluestein lengths by bluestein_n2 alone (four_step_shape)
 
     std::shared_ptr<DevBuf> upload(const std::vector<double2> &v)
@@ -253,12 +255,14 @@ struct Builder {
         P.dst32 = user32(dst) ? 1 : 0;
     }
 
-    const double2 *table_direct(long long n)   // W_n^j, j < n
+    const double2 *table_direct(long long n)   // W_n^j, j < n, one upload per plan
     {
+        const auto it = direct_tw.find(n);
+        if (it != direct_tw.end()) return it->second;
         std::vector<double2> v;
         twiddle_table(v, (uint64_t)n, (uint64_t)n, 1);
         auto b = upload(v);
-        return b ? (const double2 *)b->p : nullptr;
+        return b ? direct_tw.emplace(n, (const double2 *)b->p).first->second : nullptr;
     }
 
     const double2 *table_real(long long L)   // W_L^k, k <= L/2
@@ -669,9 +673,11 @@ struct Builder {
     }
 
     // The cheapest length of at least `need` points that the mixed-radix kernel takes in one pass, within
-    // 1/16 or the first sixteen smooth ones; 0 if there is none.
-    static long long mix_blue_len(long long need)
+    // 1/16 or the first sixteen smooth ones; 0 if there is none.  Searched for once per plan.
+    long long mix_blue_len(long long need) const
     {
+        const auto it = blue_lens.find(need);
+        if (it != blue_lens.end()) return it->second;
         long long best = 0;
         double least = 0.0;
         int seen = 0;
@@ -688,6 +694,7 @@ struct Builder {
                 least = cost;
             }
         }
+        blue_lens.emplace(need, best);
         return best;
     }
 
@@ -868,8 +875,6 @@ struct Builder {
         const double2 *rlo = nullptr, *rhi = nullptr;
         long long rS = 0;
         if (real_half && !table_two_level(2 * Ls, rlo, rhi, rS)) return false;
-        const double2 *twA = table_direct(L2), *twB = table_direct(L1);
-        if (!twA || !twB) return false;
         const double2 *chirp = nullptr, *spec = nullptr, *spec_rows = nullptr;
         if (blue && !bluestein_tables(Ls, n2, chirp, spec)) return false;
 
@@ -886,7 +891,6 @@ struct Builder {
             for (size_t s = 0; s < rad.size(); ++s) P.radix[s] = rad[s];
             P.NT = threads_per_transform(L2, rad);
             P.LD = (int)L2;
-            P.tw = twA;
             P.ni = L1;
             P.ntf = L1 * cn;
             P.nload = P.nstore = (int)L2;
@@ -905,7 +909,6 @@ struct Builder {
             for (size_t s = 0; s < rad.size(); ++s) P.radix[s] = rad[s];
             P.NT = threads_per_transform(L1, rad);
             P.LD = (int)L1;
-            P.tw = twB;
             P.ni = L2;
             P.ntf = L2 * cn;
             P.nload = P.nstore = (int)L1;
@@ -1094,6 +1097,7 @@ struct Builder {
     bool add_conv_rows(FftParams P, BufRef src, BufRef dst)
     {
         io_flags(P, src, dst);
+        if (!(P.tw = table_direct(P.N))) return false;
         const int map = 0;
         const long long tb = pow2_tb_pick(P, map);
         const long long per = (long long)pow2_lds_bytes(P.N, map);
@@ -1140,6 +1144,7 @@ struct Builder {
     bool add_rowpair(FftParams P, BufRef src, BufRef dst, bool uses_fct, long long signals, long long Ls)
     {
         io_flags(P, src, dst);
+        if (!(P.tw = table_direct(P.N))) return false;
         const int map = 2;
         const long long tb = pow2_tb_host(P.N, map);
         const long long per = (long long)pow2_lds_bytes(P.N, map);

@@ -67,10 +67,12 @@ int mix_ops(int R)
 }
 
 // Factors N into min_stages .. 6 radices of 2 .. 16 and the threads per transform they take, or returns
-// false.  The cheapest order by operation count wins: butterflies, twiddle products, the LDS
-// accesses of each stage with the bank conflicts of the first stage's writes (their stride is the
-// radix: 16-byte words fall on 8 bank groups, so an odd first radix has none), and the
-// per-stage overhead of every thread.
+// false.  The cheapest order by operation count wins (of equals the one with the smaller radices first): butterflies,
+// twiddle products, the LDS accesses of each stage with the bank conflicts of the first stage's writes
+// (their stride is the radix: 16-byte words fall on 8 bank groups, so an odd first radix has none), and
+// the per-stage overhead of every thread.  A plan tries many lengths: the search leaves
+// a branch as soon as the rest needs more stages than are left or, by a bound from below, costs more
+// than the best (8 us a length on average and 40 at most, 62 and 1,200 without).
 bool mix_factor(int N, int max_threads, std::vector<int> &radices, int &threads, double *cost_out,
                 int min_stages)
 {
@@ -81,35 +83,41 @@ bool mix_factor(int N, int max_threads, std::vector<int> &radices, int &threads,
     int most = 2;   // two stages over the fewest there could be reach every 13-smooth length (5^5, 7^4, ...)
     for (long long v = 1; v < N; v *= 16) ++most;
     most = std::min(most, 6);   // kMixMaxStages
-    auto rec = [&](auto &&self, int n) -> void {
-        if (n == 1 && (int)cur.size() >= min_stages) {
-            int nt = 1;
-            for (int R : cur) nt = std::max(nt, (N / R + nb_of(R) - 1) / nb_of(R));
-            if (nt > max_threads) return;
-            double cost = 0.0;
-            for (size_t k = 0; k < cur.size(); ++k) {
-                const int R = cur[k];
-                cost += (double)(N / R) * (mix_ops(R) + (k ? 4 * (R - 1) : 0) + 10 * R) + 60.0 * nt;
-            }
+    // a stage past the first costs its butterflies at least this per bit of its radix and point
+    static const double per_bit = [] {
+        double least = 1e300;
+        for (int R = 2; R <= 16; ++R)
+            least = std::min(least, (double)(mix_ops(R) + 4 * (R - 1) + 10 * R) / (R * std::log2((double)R)));
+        return least * (1.0 - 1e-9);
+    }();
+    // n: what is left to factor; ops, nt: of the stages so far, their costs whole numbers
+    auto rec = [&](auto &&self, int n, double ops, int nt) -> void {
+        const int k = (int)cur.size();
+        if (n == 1 && k >= min_stages) {
             int g = cur[0];
             g = (g & 1) ? 1 : (g & 2) ? 2 : (g & 4) ? 4 : 8;   // gcd with the 8 bank groups
-            cost += 4.0 * N * (g - 1);
-            if (best < 0.0 || cost < best) {
+            const double cost = ops + 60.0 * nt * k + 4.0 * N * (g - 1);
+            if (best < 0.0 || cost < best || (cost == best && cur < radices)) {
                 best = cost;
                 radices = cur;
                 threads = nt;
             }
             return;
         }
-        if ((int)cur.size() >= most) return;
-        for (int R = 2; R <= 16; ++R)
+        const int left = most - k;
+        if (left <= 0 || n > 1LL << (4 * left)) return;
+        if (best >= 0.0 && k && ops + 60.0 * nt * k + per_bit * N * std::log2((double)n) > best) return;
+        // past the first stage the order costs nothing: ascending radices stand for all orders
+        for (int R = 16; R >= (k > 1 ? cur.back() : 2); --R)
             if (n % R == 0) {
+                const int t = std::max(nt, (N / R + nb_of(R) - 1) / nb_of(R));
+                if (t > max_threads) continue;
                 cur.push_back(R);
-                self(self, n / R);
+                self(self, n / R, ops + (double)(N / R) * (mix_ops(R) + (k ? 4 * (R - 1) : 0) + 10 * R), t);
                 cur.pop_back();
             }
     };
-    rec(rec, N);
+    rec(rec, N, 0.0, 1);
     if (cost_out) *cost_out = best;
     return best >= 0.0;
 }

@@ -1,0 +1,50 @@
+"""Planning on the host (no GPU): the stand-in HIP runtime of tests/cpp/hip_stand_in.cpp."""
+import pytest
+
+PLAN = """
+import time
+def strides(shape, e):
+    st = [e]
+    for n in reversed(shape[1:]):
+        st.insert(0, st[0] * n)
+    return _lib.strides(st)
+def plan(kind, dtype, shape, axes):
+    half = list(shape)
+    half[axes[-1]] = shape[axes[-1]] // 2 + 1
+    e = 4 if dtype else 8
+    h = ctypes.c_void_p()
+    rc = L.impulse_fft_plan_create(ctypes.byref(h), kind, dtype, len(shape), _lib.sizes(shape),
+                                   strides(half if kind == 2 else shape, e if kind == 1 else 2 * e),
+                                   strides(half if kind == 1 else shape, e if kind == 2 else 2 * e),
+                                   len(axes), _lib.sizes(axes), 1)
+    assert rc == 0, L.impulse_fft_last_error()
+    return h
+"""
+
+
+@pytest.mark.parametrize("n", [1999, 3851])
+def test_bluestein_length_is_searched_once(hip_host, n):
+    # The candidate lengths of a Bluestein axis are factored once, in microseconds each: such a plan
+    # takes little more than its tables (5,000 and 8,192 entries, milliseconds), not several searches.
+    best = hip_host(PLAN + f"""
+best = 1.0
+for _ in range(7):
+    t = time.process_time()
+    h = plan(0, 0, [1, {n}], [1])
+    best = min(best, time.process_time() - t)
+    L.impulse_fft_plan_destroy(h)
+report(best)
+""")
+    assert best < (3.5e-3 if n < 2000 else 6e-3)
+
+
+def test_four_step_keeps_the_tables_it_reads(hip_host):
+    # A smooth four-step pass on the mixed-radix kernel reads stage tables only: the plan holds the two
+    # levels of W_n (two times about sqrt(n) entries), the stage tables of both factors (fewer entries
+    # than points) and two workspaces.
+    n, l1, l2 = 300000, 600, 500
+    held = hip_host(PLAN + f"report(L.impulse_fft_plan_device_bytes(plan(0, 0, [1, {n}], [1])))")
+    s = 1
+    while s * s < n:
+        s *= 2
+    assert held <= 16 * (2 * n + s + (n + s - 1) // s + 1 + l1 + l2)
