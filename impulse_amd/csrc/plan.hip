@@ -219,6 +219,17 @@ struct Job {
     }
 };
 
+// rows[k L1 + k'] = nat[k + L2 k'], once per plan: the spectrum of a long Bluestein length is reordered
+// where it is instead of on the host between two copies
+static __global__ void k_spectrum_rows(const double2 *__restrict__ nat, double2 *__restrict__ rows, int L1, int L2)
+{
+    const long long n = (long long)L1 * L2;
+    for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x) {
+        const long long k = e / L1, kp = e - k * L1;
+        rows[e] = nat[k + L2 * kp];
+    }
+}
+
 constexpr size_t kNoAllocScratchBytes = 64ull << 20;   // scratch of execution without allocation
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
@@ -1077,21 +1088,29 @@ struct Builder {
         return pow2_supported((int)L1) && L1 >= 64 && n2 * 16 <= 0x7fffffffLL;
     }
 
-    // the kernel spectrum in row order of the four-step split n2 = L1 L2:
-    // entry k L1 + k' holds spectrum bin k + L2 k' (k < L2, k' < L1)
+    // the kernel spectrum in row order of the four-step split n2 = L1 L2: entry k L1 + k' holds spectrum
+    // bin k + L2 k' (k < L2, k' < L1).  It replaces the natural-order table, which nothing else reads.
     const double2 *spectrum_rows(const double2 *spec, long long L1, long long L2)
     {
-        const long long n2 = L1 * L2;
-        std::vector<double2> nat((size_t)n2), rows((size_t)n2);
-        if (hipMemcpy(nat.data(), spec, (size_t)n2 * sizeof(double2), hipMemcpyDeviceToHost) != hipSuccess) {
-            (void)hipGetLastError();
-            err = {E_HIP, "hipMemcpy of the Bluestein spectrum failed"};
+        auto b = std::make_shared<DevBuf>();
+        if (b->alloc((size_t)(L1 * L2) * sizeof(double2)) != OK) {
+            err = {E_NOMEM, "device allocation for a twiddle table failed"};
             return nullptr;
         }
-        for (long long k = 0; k < L2; ++k)
-            for (long long kp = 0; kp < L1; ++kp) rows[(size_t)(k * L1 + kp)] = nat[(size_t)(k + L2 * kp)];
-        auto b = upload(rows);
-        return b ? (const double2 *)b->p : nullptr;
+        const unsigned grid = (unsigned)std::min<long long>((L1 * L2 + 255) / 256, 1 << 16);
+        hipLaunchKernelGGL(k_spectrum_rows, dim3(grid), dim3(256), 0, nullptr, spec, (double2 *)b->p, (int)L1, (int)L2);
+        if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
+            (void)hipGetLastError();
+            err = {E_HIP, "reordering the Bluestein spectrum failed"};
+            return nullptr;
+        }
+        for (auto &t : plan.tables)
+            if (t->p == spec) {
+                t = b;
+                return (const double2 *)b->p;
+            }
+        plan.tables.push_back(b);
+        return (const double2 *)b->p;
     }
 
     bool add_conv_rows(FftParams P, BufRef src, BufRef dst)

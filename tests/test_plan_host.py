@@ -48,3 +48,10 @@ def test_four_step_keeps_the_tables_it_reads(hip_host):
     while s * s < n:
         s *= 2
     assert held <= 16 * (2 * n + s + (n + s - 1) // s + 1 + l1 + l2)
+
+
+def test_long_bluestein_keeps_one_spectrum(hip_host):
+    # The three-pass Bluestein reads its kernel's spectrum in row order: that table alone is kept.
+    n, n2 = 100003, 262144
+    held = hip_host(PLAN + f"report(L.impulse_fft_plan_device_bytes(plan(0, 0, [1, {n}], [1])))")
+    assert held <= 16 * (2 * n2 + n + 2048)   # workspace, spectrum, chirp, the tables of 512-point passes
