@@ -48,18 +48,13 @@
 
 #include "butterflies.h"
 #include "engine.h"
+#include "line_reach.h"
 #include "mix_fft.h"
 
 namespace ifft {
 
 constexpr int kMaxDims = kMaxBatchDims + 1;
-
-// element offsets of the lines along one axis: the other dimensions, last fastest
-struct LineMap {
-    int nd;
-    long long cnt[kMaxDims];
-    long long st[kMaxDims];
-};
+static_assert(kMaxDims == kLineDims, "a LineMap holds every dimension");
 
 struct R2rParams {
     const double *src;
@@ -331,7 +326,9 @@ __global__ void k_r2r_post(const R2rParams P)
 struct R2rMix {
     const double *src;
     double *dst;
-    long long src_lo, src_span, dst_lo, dst_span;   // byte windows of the arrays around src / dst
+    // byte windows around src / dst: the arrays, or (rel) what a workgroup's lines may reach around its first line
+    long long src_lo, src_span, dst_lo, dst_span;
+    int src_rel, dst_rel;
     LineMap in, out;
     long long sa_in, sa_out;   // element stride along the axis
     long long lines;
@@ -343,11 +340,11 @@ struct R2rMix {
 };
 
 template <int TYPE, class ROW>
-__device__ __forceinline__ void r2r_mix_load(const R2rMix &P, const ROW &row, int base, int i)
+__device__ __forceinline__ void r2r_mix_load(const R2rMix &P, long long win, const ROW &row, int base, int i)
 {
     const int M = P.S.N, N = 2 * M, NT = P.S.NT;
     const int step = (int)P.sa_in * 8;
-    const __amdgpu_buffer_rsrc_t r = make_rsrc((const char *)P.src + P.src_lo, P.src_span);
+    const __amdgpu_buffer_rsrc_t r = make_rsrc((const char *)P.src + win, P.src_span);
     auto pair = [&](int j) -> double2 {   // x[2j], x[2j + 1]
         const int o = base + 2 * j * step;
         return P.in_pairs ? bload2(r, o) : make_double2(bload1(r, o), bload1(r, o + step));
@@ -437,12 +434,12 @@ __device__ __forceinline__ void r2r_mix_load(const R2rMix &P, const ROW &row, in
 }
 
 template <int TYPE, class ROW>
-__device__ __forceinline__ void r2r_mix_store(const R2rMix &P, const ROW &row, int base, int i)
+__device__ __forceinline__ void r2r_mix_store(const R2rMix &P, long long win, const ROW &row, int base, int i)
 {
     const int M = P.S.N, N = 2 * M, NT = P.S.NT;
     const int step = (int)P.sa_out * 8;
     const double f = P.fct;
-    const __amdgpu_buffer_rsrc_t r = make_rsrc((char *)P.dst + P.dst_lo, P.dst_span);
+    const __amdgpu_buffer_rsrc_t r = make_rsrc((char *)P.dst + win, P.dst_span);
     auto put = [&](int n, double v) { bstore1(r, base + n * step, v); };
     auto put_pair = [&](int j, double a, double b) {   // y[2j], y[2j + 1]
         const int o = base + 2 * j * step;
@@ -526,18 +523,20 @@ __global__ void __launch_bounds__(kMixMaxThreads) __attribute__((amdgpu_waves_pe
     __shared__ int off[2][kMaxTB];
     const int tid = (int)threadIdx.x, tb = P.tb, NT = P.S.NT;
     const long long l0 = (long long)xcd_block(blockIdx.x, gridDim.x) * tb;
+    const long long wi = P.src_lo + (P.src_rel ? line_off(P.in, l0) * 8 : 0);
+    const long long wo = P.dst_lo + (P.dst_rel ? line_off(P.out, l0) * 8 : 0);
     if (tid < tb && l0 + tid < P.lines) {
-        off[0][tid] = (int)(line_off(P.in, l0 + tid) * 8 - P.src_lo);
-        off[1][tid] = (int)(line_off(P.out, l0 + tid) * 8 - P.dst_lo);
+        off[0][tid] = (int)(line_off(P.in, l0 + tid) * 8 - wi);
+        off[1][tid] = (int)(line_off(P.out, l0 + tid) * 8 - wo);
     }
     const int t = P.col ? tid % tb : tid / NT, i = P.col ? tid / tb : tid % NT;
     const bool valid = l0 + t < P.lines;
     const ROW row{zl + t * P.ld};
     __syncthreads();
-    if (valid) r2r_mix_load<TYPE>(P, row, off[0][t], i);
+    if (valid) r2r_mix_load<TYPE>(P, wi, row, off[0][t], i);
     __syncthreads();
     if (P.S.nst) mix_fft<true, true, TYPE == 3 ? 1 : -1>(P.S, row, i, true, row, i, true, 1.0, row, row);
-    if (valid) r2r_mix_store<TYPE>(P, row, off[1][t], i);
+    if (valid) r2r_mix_store<TYPE>(P, wo, row, off[1][t], i);
 }
 
 template <int TYPE, int WPE>
@@ -571,6 +570,12 @@ static bool smooth13_r2r(long long n)
 
 constexpr int kR2rMixMax = 4096;   // longest N/2 of the one-kernel path
 
+// byte window of an array around the pointer, or (rel) around the first line of a workgroup
+struct R2rWindow {
+    long long lo, span;
+    int rel;
+};
+
 struct R2r {
     int cosine = 1, type = 2, ortho = 0;
     struct Axis {
@@ -580,6 +585,7 @@ struct R2r {
         int fused;                        // one kernel (no sub-plan)
         MixShape S;                       // ... its stages, lines per workgroup and LDS row length
         int tb, ld, pad;
+        R2rWindow win, wout;              // ... and the arrays around its launches
         std::vector<int> rad;
         std::shared_ptr<DevBuf> tab;      // half lines: e1 | e2 (L + 1 each) | stage twiddles (fused)
         LineMap in_first, in_next, out;
@@ -634,9 +640,27 @@ static int half_tables(R2r::Axis &A, int type, Error &err)
     return OK;
 }
 
+// The window of an array [lo, hi) for workgroups of tb lines, whose offsets in it have to fit 31 bits: the
+// array itself, or what one workgroup reaches (arrays over 2 GiB).  false: neither fits, and the axis takes
+// three passes through a workspace as large as the array.  One kernel against those on one MI355X, DCT-II:
+// 33,000 rows of 8,192 (2.2 GB) 1.33 and 3.80 ms, 300,000 of 1,024 1.16 and 4.08, the middle axis of
+// 5 x 1,024 x 60,000 1.86 and 4.16.
+static bool r2r_window(R2rWindow &w, long long lo, long long hi, const LineMap &m, long long sa, long long N, long long tb)
+{
+    w = R2rWindow{lo, hi - lo, 0};
+    if (w.span <= 0x7fffffff) return true;
+    long long a, b;
+    line_reach(m, tb, a, b);
+    const long long end = (N - 1) * sa;
+    a += std::min(end, 0LL);
+    b += std::max(end, 0LL);
+    w = R2rWindow{a * 8, (b - a + 1) * 8, 1};
+    return w.span <= 0x7fffffff;
+}
+
 // The stages, lines per workgroup and LDS rows of the one-kernel path (M = N/2 points): as the
 // engine's mixed-radix passes, one line where it fills a wavefront along rows.
-static bool mix_axis(R2r::Axis &A)
+static bool mix_axis(const Plan &P, R2r::Axis &A, bool first)
 {
     if (!A.half || A.L > kR2rMixMax || !smooth13_r2r(A.L)) return false;
     int nt = 1;
@@ -675,6 +699,15 @@ static bool mix_axis(R2r::Axis &A)
     tb = std::max<long long>(1, std::min(tb, std::max<long long>(A.col ? 2 : 1, A.lines / 512)));
     if (A.col)
         while (tb & (tb - 1)) tb &= tb - 1;
+    const long long in_lo = first ? P.in_lo : P.out_lo, in_hi = first ? P.in_hi : P.out_hi;
+    const LineMap &im = first ? A.in_first : A.in_next;
+    const long long sa_in = first ? A.sa_in_first : A.sa_in_next;
+    while (!r2r_window(A.win, in_lo, in_hi, im, sa_in, A.N, tb) ||
+           !r2r_window(A.wout, P.out_lo, P.out_hi, A.out, A.sa_out, A.N, tb)) {
+        if (tb == 1) return false;
+        tb /= 2;
+    }
+    if ((A.lines + tb - 1) / tb > 0x7fffffff) return false;
     A.tb = (int)tb;
     A.ld = (int)len;
     if (A.col && tb > 1) {   // lanes across lines meet distinct bank groups
@@ -751,8 +784,7 @@ int r2r_plan_create(std::unique_ptr<Plan> &out, int kind, int type, int ortho, i
         A.sa_in_next = A.sa_out = P.sout[A.axis] / 8;
         // threads walk along lines when the axis is the input's unit-stride dimension, else across lines
         A.col = A.lines > 1 && std::llabs(a == 0 ? A.sa_in_first : A.sa_in_next) != 1;
-        // one kernel where N/2 splits into its radices and all offsets fit 31 bits
-        A.fused = P.in_hi - P.in_lo <= 0x7fffffff && P.out_hi - P.out_lo <= 0x7fffffff && mix_axis(A);
+        A.fused = mix_axis(P, A, a == 0);
         if (A.half && (rc = half_tables(A, type, err)) != OK) return rc;
         if (A.fused) {
             R->ax.push_back(std::move(A));
@@ -818,10 +850,12 @@ int r2r_execute(Plan &P, const void *in, void *out, double fct, hipStream_t s, E
             R2rMix F{};
             F.src = Q.src;
             F.dst = Q.dst;
-            F.src_lo = a == 0 ? P.in_lo : P.out_lo;
-            F.src_span = a == 0 ? P.in_hi - P.in_lo : P.out_hi - P.out_lo;
-            F.dst_lo = P.out_lo;
-            F.dst_span = P.out_hi - P.out_lo;
+            F.src_lo = A.win.lo;
+            F.src_span = A.win.span;
+            F.src_rel = A.win.rel;
+            F.dst_lo = A.wout.lo;
+            F.dst_span = A.wout.span;
+            F.dst_rel = A.wout.rel;
             F.in = Q.in;
             F.out = Q.out;
             F.sa_in = Q.sa_in;
