@@ -909,6 +909,7 @@ template <int N>
 static hipError_t launch_small(const FftParams &P, int map, int io, unsigned grid, unsigned block, size_t lds,
                                hipStream_t s)
 {
+    if (io == IO_R2C_ROWPAIR || (io == (IO_CONV | IO_W4) && map != MAP_ROW)) return hipErrorInvalidValue;
     if (map == MAP_ROW) {
         switch (io) {
             case IO_PLAIN: return launch_one_small<N, MAP_ROW, IO_PLAIN>(P, grid, block, lds, s);
@@ -1050,13 +1051,16 @@ int pow2_tb_pick(const FftParams &P, int map)
     return (P.ntf + tb - 1) / tb < fill ? pow2_tb_small(P.N, map) : tb;
 }
 
-// the instances pow2_tb_small is built for (launch_small)
+// The instances pow2_tb_small is built for (launch_small): one of each Bluestein mode, named with IO_W4.
+// The row pairs and the spectrum product are not in the per-point path, so they never turn into it.
 static int small_io(int map, int io)
 {
+    if (io == IO_CONV || io == IO_BLUE_IN || io == IO_BLUE_OUT) io |= IO_W4;
     switch (io) {
+        case IO_R2C_ROWPAIR:
         case IO_PLAIN: return io;
-        case IO_R2C_HALF:
-        case IO_CONV | IO_W4: return map == MAP_ROW ? io : IO_GENERIC;
+        case IO_CONV | IO_W4: return io;
+        case IO_R2C_HALF: return map == MAP_ROW ? io : IO_GENERIC;
         case IO_TWIDDLE:
         case IO_TWIDDLE | IO_C2R:
         case IO_BLUE_IN | IO_W4:

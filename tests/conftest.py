@@ -62,4 +62,5 @@ def hip_host(tmp_path_factory):
         assert last, r.stdout
         return json.loads(last[-1][len("REPORT "):])
 
+    run.so = so
     return run

@@ -14,7 +14,12 @@
 #include <vector>
 
 namespace {
-std::map<const void *, std::string> names;   // kernels by host stub
+// kernels by host stub; the library registers them from its constructors, maybe before this file's run
+std::map<const void *, std::string> &names()
+{
+    static auto *m = new std::map<const void *, std::string>();
+    return *m;
+}
 std::map<void *, size_t> blocks;
 size_t used = 0, limit = (size_t)-1, peak = 0;
 int per_cu = 2;
@@ -51,7 +56,7 @@ void **__hipRegisterFatBinary(const void *)
 void __hipUnregisterFatBinary(void **) {}
 void __hipRegisterFunction(void **, const void *stub, char *, const char *name, unsigned, void *, void *, dim3 *, dim3 *, int *)
 {
-    names[stub] = name;
+    names()[stub] = name;
 }
 void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
 hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, hipStream_t s)
@@ -144,7 +149,7 @@ hipError_t hipLaunchKernel(const void *stub, dim3 g, dim3 b, void **, size_t lds
 {
     char t[96];
     std::snprintf(t, sizeof(t), " %u %u %u %zu\n", g.x, g.y, b.x * b.y * b.z, lds);
-    launches += names[stub] + t;
+    launches += names()[stub] + t;
     return hipSuccess;
 }
 }

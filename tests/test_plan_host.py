@@ -1,6 +1,10 @@
 """Planning on the host (no GPU): the stand-in HIP runtime of tests/cpp/hip_stand_in.cpp."""
+import os
+import subprocess
+
 import pytest
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PLAN = """
 import time
 def strides(shape, e):
@@ -55,3 +59,23 @@ def test_long_bluestein_keeps_one_spectrum(hip_host):
     n, n2 = 100003, 262144
     held = hip_host(PLAN + f"report(L.impulse_fft_plan_device_bytes(plan(0, 0, [1, {n}], [1])))")
     assert held <= 16 * (2 * n2 + n + 2048)   # workspace, spectrum, chirp, the tables of 512-point passes
+
+
+def test_small_workgroups_keep_their_mode(hip_host, tmp_path):
+    """The spectrum product and the row pairs are not in the per-point path of the power-of-two kernel: its
+    small workgroups run them on an instance of their own, or refuse, on any grid."""
+    exe = str(tmp_path / "pow2_small")
+    lib = os.path.join(ROOT, "impulse_amd")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I", os.path.join(lib, "csrc"), os.path.join(ROOT, "tests", "cpp", "pow2_small_main.cpp"),
+                    "-o", exe, hip_host.so, "-L", lib, "-l:libimpulse_fft.so", f"-Wl,-rpath,{lib}",
+                    f"-Wl,-rpath,{os.path.dirname(hip_host.so)}", "-Wl,--allow-shlib-undefined"], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    lines = [l.split() for l in r.stdout.splitlines()]
+    assert len(lines) == 12
+    for conv, mode, grid, err, name, *_ in lines:
+        if conv == "1" and mode == "0":
+            assert err == "0" and "k_fft_pow2ILi512ELi0ELi12ELi2E" in name, (grid, name)   # spectrum product, four-wave name
+        else:
+            assert err != "0" and name == "-", (conv, mode, grid, name)
