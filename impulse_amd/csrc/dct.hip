@@ -658,6 +658,21 @@ static bool r2r_window(R2rWindow &w, long long lo, long long hi, const LineMap &
     return w.span <= 0x7fffffff;
 }
 
+// Threads of a line, where that is more than its butterflies take (16 points a thread): few lines are bound by
+// one thread's chain of loads, LDS accesses and butterflies, and many short ones by its unshared
+// loads.  Half the points each while the lines then take at most 131,072 threads, else two to eight
+// threads along rows and two across them.  MI355X, DCT-II rows: 2,000 x 90 11.4 -> 6.3 us, 100 x 6,250
+// 16.3 -> 12.2, 200,000 x 30 68 -> 25 (eight threads 35), 200,000 x 16 27 -> 19; columns 128 x 2,000
+// 19 -> 8.0, 30 x 200,000 24.4 -> 23.3 (four threads 25.2).
+static long long line_threads(const R2r::Axis &A)
+{
+    long long half = 1, share = 1;
+    while (2 * half < A.L) half *= 2;
+    while (2 * share * A.lines <= 131072) share *= 2;
+    const long long least = A.col ? (A.L < 10 ? 1 : 2) : A.L < 5 ? 1 : A.L < 8 ? 2 : A.L < 40 ? 4 : 8;
+    return std::max(least, std::min(half, share));
+}
+
 // The stages, lines per workgroup and LDS rows of the one-kernel path (M = N/2 points): as the
 // engine's mixed-radix passes, one line where it fills a wavefront along rows.
 static bool mix_axis(const Plan &P, R2r::Axis &A, bool first)
@@ -676,6 +691,7 @@ static bool mix_axis(const Plan &P, R2r::Axis &A, bool first)
             if (m > 1) A.rad.insert(A.rad.begin(), (int)m);
             nt = (int)std::max<long long>(1, A.L / 8);
         }
+        nt = std::max(nt, (int)std::min<long long>(line_threads(A), kMixMaxThreads));
         A.S.NT = nt;
         A.S.nst = (int)A.rad.size();
         for (size_t k = 0; k < A.rad.size(); ++k) A.S.codes |= (unsigned)(A.rad[k] - 1) << (4 * k);
@@ -696,7 +712,10 @@ static bool mix_axis(const Plan &P, R2r::Axis &A, bool first)
         tb = nt >= 64 ? 1 : std::min<long long>(128 / nt, 80 * 1024 / row);
     }
     tb = std::min<long long>(std::min<long long>(tb, kMaxTB), fit);
-    tb = std::max<long long>(1, std::min(tb, std::max<long long>(A.col ? 2 : 1, A.lines / 512)));
+    // small grids are spread over the chip, by whole wavefronts
+    const long long wave = std::min<long long>((63 + nt) / nt, tb);
+    tb = std::min(tb, std::max({wave, A.col ? 2LL : 1LL, A.lines / 512}));
+    tb = std::max<long long>(1, std::min(tb, A.lines));
     if (A.col)
         while (tb & (tb - 1)) tb &= tb - 1;
     const long long in_lo = first ? P.in_lo : P.out_lo, in_hi = first ? P.in_hi : P.out_hi;

@@ -47,3 +47,40 @@ report(got)
         assert min(got) > 1
     else:
         assert got == [launches] * 3
+
+
+@pytest.mark.parametrize("shape,axis", [((2000, 30), 1), ((300, 16), 1), ((2000, 10), 1), ((200000, 30), 1), ((20000, 16), 1),
+                                        ((2000, 90), 1), ((128, 2000), 0), ((30, 2000), 0), ((64, 300), 0)])
+def test_short_lines_fill_wavefronts(hip_host, shape, axis):
+    """Many short lines: no workgroup under a wavefront, and several threads a line along rows."""
+    got = hip_host(f"""
+shape, got = {list(shape)}, []
+st = _lib.strides([8 * shape[1], 8])
+for t in (2, 3, 4):
+    h = ctypes.c_void_p()
+    rc = L.impulse_fft_r2r_plan_create(ctypes.byref(h), 5, t, 0, 0, 2, _lib.sizes(shape), st, st, 1, _lib.sizes([{axis}]))
+    assert rc == 0, L.impulse_fft_last_error()
+    launches()
+    assert L.impulse_fft_execute(h, 1 << 30, 1 << 32, 1.0, None) == 0
+    got += launches()
+report(got)
+""")
+    assert len(got) == 3 and all("k_r2r_mix" in l[0] for l in got)
+    lines = shape[1 - axis]
+    for _, grid, _, block, _ in got:
+        assert int(block) >= 64
+        if axis == 1:
+            assert int(block) * int(grid) >= 2 * lines
+
+
+@pytest.mark.parametrize("n,threads", [(16, 4), (90, 32), (2048, 512), (6250, 512)])
+def test_single_line_uses_more_threads(hip_host, n, threads):
+    """One line alone is bound by a thread's chain: a thread for every two points, up to 512."""
+    got = hip_host(f"""
+h, st = ctypes.c_void_p(), _lib.strides([8 * {n}, 8])
+assert L.impulse_fft_r2r_plan_create(ctypes.byref(h), 5, 2, 0, 0, 2, _lib.sizes([1, {n}]), st, st, 1, _lib.sizes([1])) == 0
+launches()
+assert L.impulse_fft_execute(h, 1 << 30, 1 << 32, 1.0, None) == 0
+report(launches())
+""")
+    assert len(got) == 1 and int(got[0][3]) == threads
