@@ -106,27 +106,33 @@ __global__ void __launch_bounds__(256) k_upfirdn_tile(const double *__restrict__
 // the caches: `up` neighbouring taps per step) for R outputs, so an FMA takes one LDS read, of the
 // signal, instead of two, and the taps take no LDS and no copy into it.  The sum of an output runs in
 // ufd_output's order.  The first workgroups take the outputs whose taps meet either end of the signal,
-// and those past the last whole tile, T each by ufd_output itself: [0, lead) and [tail, nout).  2^22
-// samples on one MI355X: 160/147 with 1,601 taps 28.7 -> 23.0 us, with 6,401 taps 98 -> 46 us; 4/1 with 81
-// taps 72 -> 41 us; 320/441 with 17,641 taps 210 -> 61 us.  Bound now by the LDS reads of the signal (one
-// an FMA) and, at few taps, by HBM (3 TB/s).
+// and those past the last whole tile, T each by ufd_output itself: [0, lead) and [tail, nout).  Against the
+// tile or the direct kernel on one MI355X: 160/147, 2^22 outputs, 1,601 taps 24.0 -> 18.2 us; 2^22 samples: 160/147
+// with 6,401 taps 91 -> 42, 4/1 with 81 taps 89 -> 59, 320/441 with 17,641 taps 198 -> 56.  Bound now by the LDS reads of the signal (one
+// an FMA) and, at few taps, by HBM (3 TB/s).  All signals' end workgroups come first in the grid, since
+// they run longest: at its end they would run alone (20 x 450,000 samples, 2/3, 41 taps: 51 us so, 43 on the
+// tile kernel).
 template <int R>
 __global__ void __launch_bounds__(512) k_upfirdn_phase(const double *__restrict__ t, const double *__restrict__ h,
                                                        double *__restrict__ y, long long nt, int nh, int up, int down,
-                                                       long long nout, long long lead, long long tail)
+                                                       long long nout, long long lead, long long tail, unsigned nedge,
+                                                       unsigned ntile, unsigned batch)
 {
     extern __shared__ double ts[];
     const int T = (int)blockDim.x, i = (int)threadIdx.x;
-    const double *tb = t + (long long)blockIdx.y * nt;
-    double *yb = y + (long long)blockIdx.y * nout;
-    const long long nlead = (lead + T - 1) / T, nedge = nlead + (nout - tail + T - 1) / T;
-    if (blockIdx.x < nedge) {
-        const bool front = blockIdx.x < nlead;
-        const long long j = (front ? 0 : tail - nlead * T) + (long long)blockIdx.x * T + i;
+    const bool edge = blockIdx.x < nedge * batch;
+    const unsigned per = edge ? nedge : ntile, at = edge ? blockIdx.x : blockIdx.x - nedge * batch;
+    const unsigned sig = at / per, blk = at - sig * per;
+    const double *tb = t + (long long)sig * nt;
+    double *yb = y + (long long)sig * nout;
+    if (edge) {
+        const long long nlead = (lead + T - 1) / T;
+        const bool front = blk < nlead;
+        const long long j = (front ? 0 : tail - nlead * T) + (long long)blk * T + i;
         if (j < (front ? lead : nout)) yb[j] = ufd_output(tb, 0, h, j, nt, nh, up, down);
         return;
     }
-    const long long J0 = lead + ((long long)blockIdx.x - nedge) * (T * R);
+    const long long J0 = lead + (long long)blk * (T * R);
     const long long first = J0 * down - (nh - 1), q1 = (J0 + (long long)T * R - 1) * down / up;
     const long long q0 = first / up;
     const int nseg = (int)(q1 - q0 + 1);
@@ -238,7 +244,8 @@ struct Upfirdn {
     int up = 1, down = 1, algo = 1;
     DevBuf h;                                  // taps (direct)
     int seg_cap = 0;                           // signal points per tile in LDS (0: untiled direct kernel)
-    long long phase_lead = 0, phase_tail = 0, phase_grid = 0;
+    long long phase_lead = 0, phase_tail = 0;
+    unsigned phase_edges = 0, phase_tiles = 0;     // its workgroups per signal: ends, whole tiles
     int phase_t = 0, phase_r = 0, phase_seg = 0;   // k_upfirdn_phase: threads, outputs per thread, LDS points (0: not taken)
     long long P = 0, B = 0, nblk = 0, nspec = 0;
     std::unique_ptr<Plan> r2c, c2r;
@@ -274,10 +281,18 @@ static void fft_shape(Upfirdn &U)
 }
 
 // Threads (the multiple of `up` up to 512 that fills its wavefronts best, near 256 on a tie), outputs per
-// thread and LDS segment of the phase kernel.  Eight outputs a thread where that leaves 1,024 whole tiles,
-// four where that leaves 512; smaller problems are bound by one workgroup's latency and stay with the
-// tile kernel (65,536 samples, 147/160, 41 taps a phase: 11.7 us there, 20 us here), as do rates above
-// 512 and segments over the LDS budget.
+// thread and LDS segment of the phase kernel.  Where the tile kernel takes the filter too, four outputs a
+// thread: the segment of eight leaves a CU fewer workgroups (2^22 outputs: 2/3, 41 taps 33.8 us with eight,
+// 26.8 with four; 160/147, 1,601 taps 20.7 and 18.2).  Filters past its LDS take eight from 1,024 whole tiles on,
+// which read the taps half as often (320/441, 38,401 taps, 2^24 outputs 521 us, 628 with four).  The tile kernel keeps
+//  * fewer than 512 whole tiles, which are bound by one workgroup's latency (65,536 samples, 147/160, 41 taps
+//    a phase: 11.7 us there, 20 us here), and rates above 512;
+//  * segments over 20 KiB in many outputs with 15 to 99 taps a phase (1/4, 31 taps: 2^24 outputs 298 us there,
+//    325 here, 2^22 74 and 79, 2^20 18.5 and 17.1; 1/3, 46 taps: 2^24 183 and 202, 2^22 46.5 and 44.5), over 36
+//    KiB with more (1/5, 121 taps: 498 and 539);
+//  * short signals: an output of the ends costs as much as six of a tile, so those may be one in 64 (2,000
+//    x 1,000 samples, 2/1, 31 taps, two fifths at the ends: 24 us there, 37 here; 200 x 20,000, 1/1, one in
+//    twelve: 33 and 38).
 static void phase_shape(Upfirdn &U)
 {
     int best = 0;
@@ -290,23 +305,29 @@ static void phase_shape(Upfirdn &U)
         }
     }
     if (!best) return;
+    const bool tile = U.seg_cap > 0;
+    const long long taps = (U.nh + U.up - 1) / U.up;   // of a phase
     for (int R : {8, 4}) {
         const long long per = (long long)best * R;
         const long long span = ((per - 1) * U.down) / U.up + (U.nh - 1) / U.up + 3;
+        const bool many = U.nout * U.batch > (span * 8 <= 28 * 1024 ? 5LL << 20 : 5LL << 19);
+        const long long lds = R == 8 ? (tile ? 0 : kUfdLdsBytes / 2)
+                              : !tile || !many || taps <= 14 ? kUfdLdsBytes : taps < 100 ? 20 * 1024 : 36 * 1024;
         // whole tiles from the first output with all its taps (a multiple of T) to the last one
         const long long lead = ((U.nh - 1 + U.down - 1) / U.down + best - 1) / best * best;
         const long long good = std::min(U.nout, ((U.nt - 1) * U.up + U.up - 1) / U.down + 1);   // outputs with qhi <= nt - 1
         const long long tiles = good > lead ? (good - lead) / per : 0;
         const long long edges = (lead + best - 1) / best + (U.nout - (lead + tiles * per) + best - 1) / best;
-        if (span * 8 > (R == 8 ? kUfdLdsBytes / 2 : kUfdLdsBytes) || tiles * U.batch < (R == 8 ? 1024 : 512) ||
-            tiles + edges >= (1LL << 31))
+        if (span * 8 > lds || tiles * U.batch < (R == 8 ? 1024 : 512) ||
+            (tile && (U.nout - tiles * per) * 64 > U.nout) || (tiles + edges) * U.batch >= (1LL << 31))
             continue;
         U.phase_t = best;
         U.phase_r = R;
         U.phase_seg = (int)span;
         U.phase_lead = lead;
         U.phase_tail = lead + tiles * per;
-        U.phase_grid = tiles + edges;
+        U.phase_edges = (unsigned)edges;
+        U.phase_tiles = (unsigned)tiles;
         return;
     }
 }
@@ -411,14 +432,14 @@ int upfirdn_execute(Upfirdn &U, const double *t, double *y, hipStream_t s, Error
     const long long total = U.batch * U.nout;
     if (U.algo == 1) {
         if (U.phase_t > 0) {
-            const dim3 grid((unsigned)U.phase_grid, (unsigned)U.batch), block((unsigned)U.phase_t);
+            const dim3 grid((U.phase_edges + U.phase_tiles) * (unsigned)U.batch), block((unsigned)U.phase_t);
             const size_t lds = (size_t)U.phase_seg * 8;
             if (U.phase_r == 8)
                 hipLaunchKernelGGL(k_upfirdn_phase<8>, grid, block, lds, s, t, (const double *)U.h.p, y, U.nt, (int)U.nh, U.up,
-                                   U.down, U.nout, U.phase_lead, U.phase_tail);
+                                   U.down, U.nout, U.phase_lead, U.phase_tail, U.phase_edges, U.phase_tiles, (unsigned)U.batch);
             else
                 hipLaunchKernelGGL(k_upfirdn_phase<4>, grid, block, lds, s, t, (const double *)U.h.p, y, U.nt, (int)U.nh, U.up,
-                                   U.down, U.nout, U.phase_lead, U.phase_tail);
+                                   U.down, U.nout, U.phase_lead, U.phase_tail, U.phase_edges, U.phase_tiles, (unsigned)U.batch);
         } else if (U.seg_cap > 0) {
             const long long tiles = (U.nout + 256 * kUfdTileR - 1) / (256 * kUfdTileR);
             const size_t lds = (size_t)(U.nh + U.seg_cap) * 8;
