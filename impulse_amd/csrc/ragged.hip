@@ -657,6 +657,7 @@ struct Ragged {
     int precision = 0;   // 0: FP64 stages; 1: radix-16 stages as exact bf16-slice MFMA products
     DevBuf bx;           // their B operand table (precision 1)
     // derived for the configuration: the tasks of the phases back to back
+    int start = -1;   // the starting budget in use; -1: configured by the caller
     std::vector<RaggedTask> tasks;
     int phase_off[kPhases] = {0, 0, 0, 0}, phase_cnt[kPhases] = {0, 0, 0, 0}, phase_grid[kPhases] = {0, 0, 0, 0};
     int queue_off[kPhases][8] = {}, queue_cnt[kPhases][8] = {};   // per phase: the XCD queues within it
@@ -907,26 +908,48 @@ static int resident_grid(const Ragged &R, int threads, int waves, size_t lds)
     return ncu * per;
 }
 
-// Whether the batch is better off with the largest budget from the start: Bluestein units that the small
-// one splits over four phases but this one keeps in LDS, no unit that it splits itself, and at most three
-// units a CU, so that the phases' latency weighs more than the overlap of small workgroups.  Times with
-// 1,024 and with 256 threads (MI355X): 100 signals of 64 to 4,096 points 73 and 99 us, 251 of 471 to 5,082
-// 83 and 106, 600 of 500 to 4,096 94 and 115; 4,000 of 64 to 4,096 305 and 169.
-static bool single_phase_pays(const Ragged &R)
+// The configurations a batch may start with, by LDS budget.
+struct RaggedBudget {
+    int threads, points, waves;
+};
+constexpr RaggedBudget kBudgets[3] = {{256, 2048, 3}, {512, 4096, 4}, {1024, 8192, 0}};
+
+// The budget of a batch until the caller tunes or sets one.  Small workgroups, three to a CU, overlap one's
+// loads with another's stages: 256 threads and 2,048 points was the fastest of all, or within 3 % of it, on
+// batches that mix lengths up to 16,384 points and beyond (4,000 of 64 to 262,144 points 5.0 ms, 7.3 with
+// 1,024 threads; 300 of 1,000 to 200,000 0.19 and 0.31).  Transforms over 2,048 points then pass through a workspace
+// in two phases, Bluestein ones in four.  Where a larger budget holds every transform of the batch in
+// LDS, it is taken (MI355X, microseconds with 256 / 512 / 1,024 threads)
+//  * for Bluestein transforms over 2,048 points among at most three units a CU, which the four phases'
+//    latency bounds, the largest: 100 signals of 64 to 4,096 points 99 / - / 73, 600 of 500 to 4,096 115 / - / 94;
+//  * for fewer units than a quarter of the CUs, that of 4,096 points: 30 x 8,192 41 / 34 / 38;
+//  * else by the points per budget and length, at the measured time of each: 1,000 x 8,192 139 / 83 / 118,
+//    1,000 x 16,384 240 / 457 / 183, 2,000 x 4,100 496 / 803 / 414, 4,000 of 64 to 4,096 169 / - / 305.
+// The matrix-core precision spends as long on a point whatever the budget, so only the first holds for it.
+static int starting_budget(const Ragged &R, int precision)
 {
     int ncu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, R.device) != hipSuccess || ncu <= 0) {
         (void)hipGetLastError();
         ncu = 256;
     }
-    if (R.units.size() > 3 * (size_t)ncu) return false;
+    static const double ps[3][3] = {{17, 35, 65}, {34, 21, 35}, {31, 55, 24}};   // a point, by length and budget
+    double cost[3] = {0.0, 0.0, 0.0};
+    long long longest = 0;
     bool split = false;
     for (const auto &u : R.units) {
         const long long n = (long long)R.n[(size_t)u.first], L = transform_len(n, u.second >= 0);
-        if (L > 8192) return false;
+        longest = std::max(longest, L);
+        if (L > 8192) return 0;
         split |= L > 2048 && !rg_smooth13(n % 2 == 0 ? n / 2 : n);
+        for (int b = 0; b < 3; ++b) cost[b] += (double)L * ps[L <= 2048 ? 0 : L <= 4096 ? 1 : 2][b];
     }
-    return split;
+    if (longest <= 2048) return 0;
+    if (split && R.units.size() <= 3 * (size_t)ncu) return 2;
+    if (precision) return 0;
+    const int larger = longest <= 4096 ? 1 : 2;
+    if (4 * R.units.size() < (size_t)ncu) return larger == 1 ? 1 : 0;
+    return cost[larger] < cost[0] ? larger : 0;
 }
 
 static int build_tasks(Ragged &R, int threads, int lds_max, int waves, Error &err)
@@ -1129,6 +1152,14 @@ static int build_spectra(Ragged &R, Error &err)
     return OK;
 }
 
+static int start_with(Ragged &R, int budget, Error &err)
+{
+    const RaggedBudget &b = kBudgets[budget];
+    const int rc = build_tasks(R, b.threads, b.points, b.waves, err);
+    R.start = rc == OK ? budget : -1;
+    return rc;
+}
+
 int ragged_create(Ragged **out, size_t count, const size_t *lengths, const size_t *in_off, const size_t *out_off,
                   int forward, Error &err)
 {
@@ -1180,17 +1211,12 @@ int ragged_create(Ragged **out, size_t count, const size_t *lengths, const size_
             }
     rc = build_spectra(*R, err);
     if (rc != OK) return rc;
-    // The configuration until the caller tunes or sets one: 256 threads, 2,048 points and three waves
-    // per SIMD was the fastest of all, or within 3 % of it, on every batch measured (100 to 4,000
-    // signals of 64 to 262,144 points; 4,000: 5.06 ms against 7.27 ms with 1,024 threads and 8,192
-    // points, 300 of 1,000 to 200,000 points: 0.189 against 0.314 ms): three workgroups a CU overlap
-    // one's loads with another's stages.  Lengths it cannot split go to the larger budgets, and so
-    // do batches whose workspace does not fit: transforms a budget holds in LDS need none.
-    rc = E_UNSUPPORTED;
-    const int budget[3][3] = {{256, 2048, 3}, {512, 4096, 4}, {1024, 8192, 0}};
-    if (single_phase_pays(*R)) rc = build_tasks(*R, budget[2][0], budget[2][1], budget[2][2], err);
+    // Lengths the starting budget cannot split go to the other budgets, and so do batches whose
+    // workspace does not fit: transforms a budget holds in LDS need none.
+    const int start = starting_budget(*R, 0);
+    rc = start_with(*R, start, err);
     for (int k = 0; k < 3 && (rc == E_UNSUPPORTED || rc == E_NOMEM); ++k)
-        rc = build_tasks(*R, budget[k][0], budget[k][1], budget[k][2], err);
+        if (k != start) rc = start_with(*R, k, err);
     if (rc != OK) return rc;
     *out = R.release();
     return OK;
@@ -1211,6 +1237,7 @@ int ragged_configure(Ragged &R, int threads, int lds_max, int order, int waves, 
     }
     if (threads == 1024) waves = 0;   // 1024 threads always leave 128 registers
     R.rorder = order;
+    R.start = -1;
     if (threads == R.threads && lds_max == R.lds_max && waves == R.waves && !R.tasks.empty()) {
         R.drop_graph();
         return OK;
@@ -1233,6 +1260,15 @@ int ragged_set_precision(Ragged &R, int precision, Error &err)
             (void)hipGetLastError();
             err = {E_HIP, std::string("ragged table: ") + hipGetErrorString(e)};
             return E_HIP;
+        }
+    }
+    // a batch that nobody configured starts anew with the precision's budget, or keeps its own
+    const int had = R.start, want = starting_budget(R, precision);
+    if (had >= 0 && want != had) {
+        Error e2{0, ""};
+        if (start_with(R, want, e2) != OK) {
+            const int rc = start_with(R, had, err);
+            if (rc != OK) return rc;
         }
     }
     R.precision = precision;

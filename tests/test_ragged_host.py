@@ -25,11 +25,11 @@ report(resource.getrusage(resource.RUSAGE_SELF).ru_maxrss)
 
 
 def test_budget_follows_device_memory(hip_host):
-    # The starting budget keeps a workspace for these transforms of 8,192 points, the largest one holds
+    # The starting budget keeps a workspace for the transforms of 8,192 points, the largest one holds
     # them in LDS: where the workspace does not fit, the batch is created without it.
     roomy, tight = hip_host(CREATE + """
-n = [16384] * 1000
-ins, outs = [16384 * i for i in range(1000)], [8193 * i for i in range(1000)]
+n = [16384] * 1000 + [4096] * 4000
+ins, outs = [16384 * i for i in range(5000)], [8193 * i for i in range(5000)]
 got = []
 for limit in (1 << 40, 64 << 20):
     S.standin_limit(limit)
@@ -85,3 +85,48 @@ L.impulse_fft_ragged_info(h, None, ctypes.byref(b), None, None, None, None, None
 report([rc, b.value, L.impulse_fft_ragged_execute(h, 1 << 40, 1 << 41, 1.0, None)])
 """)
     assert (rc, budget, run) == (0, 8192, 0)
+
+
+@pytest.mark.parametrize("lengths,points", [
+    ("[2048] * 1000", 2048), ("[4096] * 10000", 2048),                       # held by the smallest budget
+    ("[8192] * 1", 4096), ("[8192] * 1000", 4096), ("[4095] * 2000", 4096), ("[2047] * 2000", 4096),
+    ("[16384] * 30", 2048), ("[16384] * 64", 8192), ("[16384] * 1000", 8192), ("[4100] * 2000", 8192),
+    ("[16384] * 1000 + [16386] * 10", 2048),                                 # 8,193 = 3 * 2731: Bluestein beyond 8,192 points
+    ("[16384] * 100 + [4096] * 2000", 2048),                                 # mostly short ones
+    ("[97] * 5 + [8198]", 2048), ("[97] * 5 + [2206]", 8192), ("[96] * 768 + [2206]", 2048),
+])
+def test_starting_budget(hip_host, lengths, points):
+    """The larger budgets where they hold all of a batch in LDS and are faster on it (256 CUs)."""
+    got = hip_host(CREATE + f"""
+n = {lengths}
+ins, outs = [0] * len(n), [16384 * i for i in range(len(n))]
+rc, h = create(n, ins, outs)
+assert rc == 0, L.impulse_fft_last_error()
+b = ctypes.c_int()
+L.impulse_fft_ragged_info(h, None, ctypes.byref(b), None, None, None, None, None)
+report(b.value)
+""")
+    assert got == points
+
+
+def test_starting_budget_follows_precision(hip_host):
+    """A batch starts with the budget of its precision until a configuration is set."""
+    got = hip_host(CREATE + """
+n = [16384] * 1000
+rc, h = create(n, [0] * 1000, [8193 * i for i in range(1000)])
+assert rc == 0
+def budget():
+    b = ctypes.c_int()
+    L.impulse_fft_ragged_info(h, None, ctypes.byref(b), None, None, None, None, None)
+    return b.value
+got = [budget()]
+for precision in (1, 0, 1):
+    assert L.impulse_fft_ragged_set_precision(h, precision) == 0
+    got.append(budget())
+assert L.impulse_fft_ragged_configure(h, 512, 4096, 0, 4) == 0
+for precision in (0, 1):
+    assert L.impulse_fft_ragged_set_precision(h, precision) == 0
+    got.append(budget())
+report(got)
+""")
+    assert got == [8192, 2048, 8192, 2048, 4096, 4096]
