@@ -695,11 +695,11 @@ struct Builder {
         for (long long n = std::max<long long>(need, kMixMinLen); n <= kMaxLdsLen && seen < 16; ++n) {
             if (best && n > need + need / 16) break;
             if (!smooth13(n)) continue;
-            ++seen;
             std::vector<int> rad;
             int nt;
             double cost;
             if (!mix_factor((int)n, kMixMaxThreads, rad, nt, &cost)) continue;
+            ++seen;   // lengths that take more than its threads do not count
             if (!best || cost < least) {
                 best = n;
                 least = cost;

@@ -79,3 +79,26 @@ def test_small_workgroups_keep_their_mode(hip_host, tmp_path):
             assert err == "0" and "k_fft_pow2ILi512ELi0ELi12ELi2E" in name, (grid, name)   # spectrum product, four-wave name
         else:
             assert err != "0" and name == "-", (conv, mode, grid, name)
+
+
+def test_bluestein_lengths_find_their_kernel(hip_host):
+    """Every non-smooth length whose padded transform fits one pass runs on the mixed-radix Bluestein kernel,
+    also where many smooth lengths just above it need more threads than that kernel has."""
+    got = hip_host(PLAN + """
+got = {}
+for n in list(range(17, 4096, 97)) + [3841, 3850, 3851, 3889, 3899, 3900, 3907, 4093, 4096]:
+    h = plan(0, 0, [2, n], [1])
+    L.impulse_fft_execute(h, 1 << 30, 1 << 31, 1.0, None)
+    launches()
+    L.impulse_fft_execute(h, 1 << 30, 1 << 31, 1.0, None)
+    got[n] = [l[0] for l in launches()]
+    L.impulse_fft_plan_destroy(h)
+report(got)
+""")
+    for n, names in got.items():
+        m = int(n)
+        for p in (2, 3, 5, 7, 11, 13):
+            while m % p == 0:
+                m //= p
+        if m > 1:
+            assert len(names) == 1 and "k_fft_mix_blue" in names[0], (n, names)
