@@ -15,13 +15,16 @@ def test_sparse_offsets(hip_host, gap):
     # Two short signals far apart in their buffers: the host memory of a batch follows the samples
     # it holds, not the distance between them.
     kib = hip_host(CREATE + f"""
-import resource
+def peak():   # address space of this process, KiB
+    return next(int(l.split()[1]) for l in open("/proc/self/status") if l.startswith("VmPeak"))
+rc, h = create([1000, 4099], [0, 8192], [0, 8192])   # the same batch close together
+before = peak()
 rc, h = create([1000, 4099], [0, {gap}], [0, {gap}])
 assert rc == 0, L.impulse_fft_last_error()
 assert L.impulse_fft_ragged_configure(h, 512, 4096, 0, 0) == 0
-report(resource.getrusage(resource.RUSAGE_SELF).ru_maxrss)
+report(peak() - before)
 """)
-    assert kib < 256 << 10
+    assert kib < 64 << 10
 
 
 def test_budget_follows_device_memory(hip_host):
