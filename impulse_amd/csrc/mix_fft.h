@@ -2,7 +2,7 @@
 // first stage's inputs and the last stage's outputs going straight between
 // registers and the caller's loads and stores.
 //
-// A length N = R0 R1 ... (two or three stages mostly, any radices 2..16) is factored on the
+// A length N = R0 R1 ... (two to four stages mostly, six at most, radices 2..16) is factored on the
 // host (mix_factor).  Stage s of radix R, with p the product of the earlier
 // radices, takes butterflies b in [0, N/R), k = b mod p:
 //   inputs  x[b + q N/R] W_{pR}^{q k},  outputs y[(b - k) R + k + q p],  q < R,
