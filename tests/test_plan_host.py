@@ -29,17 +29,19 @@ def plan(kind, dtype, shape, axes):
 @pytest.mark.parametrize("n", [1999, 3851])
 def test_bluestein_length_is_searched_once(hip_host, n):
     # The candidate lengths of a Bluestein axis are factored once, in microseconds each: such a plan
-    # takes little more than its tables (5,000 and 8,192 entries, milliseconds), not several searches.
-    best = hip_host(PLAN + f"""
-best = 1.0
-for _ in range(7):
-    t = time.process_time()
-    h = plan(0, 0, [1, {n}], [1])
-    best = min(best, time.process_time() - t)
-    L.impulse_fft_plan_destroy(h)
+    # takes little more than its tables, not several searches.  It computes about four tables of its
+    # padded length (4,000 and 8,192 points); the plan of 8,192 points, with one such table, is the measure.
+    mine, measure = hip_host(PLAN + f"""
+best = [1.0, 1.0]
+for _ in range(9):
+    for k, m in enumerate(({n}, 8192)):
+        t = time.process_time()
+        h = plan(0, 0, [1, m], [1])
+        best[k] = min(best[k], time.process_time() - t)
+        L.impulse_fft_plan_destroy(h)
 report(best)
 """)
-    assert best < (3.5e-3 if n < 2000 else 6e-3)
+    assert mine < (4.5 if n < 2000 else 8) * measure
 
 
 def test_four_step_keeps_the_tables_it_reads(hip_host):
