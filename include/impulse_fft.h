@@ -322,7 +322,10 @@ int impulse_fft_ragged_tune(impulse_fft_ragged batch, const float *in, void *out
  * of two as radix-8 rather than radix-16 stages),
  * waves_per_simd 0 (registers as the workgroup size allows), 4 (at most 128
  * registers per lane: more resident workgroups, some spills) or, with 256
- * threads, 3 (at most 168). */
+ * threads, 3 (at most 168).  Where the workspace of a configuration does not
+ * fit the device memory the call returns IMPULSE_FFT_ERR_NOMEM and leaves the
+ * batch without a configuration: executes return
+ * IMPULSE_FFT_ERR_INVALID_ARG until one that fits is set (or tuned). */
 int impulse_fft_ragged_configure(impulse_fft_ragged batch, int threads, int lds_points, int radix_order,
                                  int waves_per_simd);
 /* Arithmetic of the LDS stages (no PocketFFT counterpart):
@@ -334,7 +337,9 @@ int impulse_fft_ragged_configure(impulse_fft_ragged batch, int threads, int lds_
  *       FP64 (error ~1e-12 relative) -- with powers of two planned as radix-16
  *       stages whatever the radix order; twiddles, the Bluestein chirp and its
  *       spectrum, and the other radices stay FP64.
- * Applies from the next execute (the graph is re-captured). */
+ * Applies from the next execute (the graph is re-captured).  A batch that was
+ * neither configured nor tuned also changes to the configuration it would
+ * start with in that precision. */
 typedef enum impulse_fft_ragged_precision {
     IMPULSE_FFT_RAGGED_FP64 = 0,
     IMPULSE_FFT_RAGGED_MFMA_BF16X = 1
